@@ -249,6 +249,12 @@ int pscf_batch_eri_s8(int dtype, const void* d_mols, int nmol, const int* const*
 int pscf_batch_eri_s8_div(int dtype, const void* d_mols, int nmol, const int* const* h_work, const int* h_nwork,
                           const int* d_atm, const int* d_bas, const double* d_env, const int* d_shell_ao,
                           const int* d_shl_sorted, void* d_out, void* stream);
+/* The same ERIs of every molecule (div as in pscf_batch_eri_s8_div) without
+ * work lists: each angular class enumerates the molecules' own shell-pair
+ * tiles.  d_order (optional) lists the molecules largest first. */
+int pscf_batch_eri_s8_all(int dtype, const void* d_mols, const int* d_order, int nmol, const int* d_atm,
+                          const int* d_bas, const double* d_env, const int* d_shell_ao, const int* d_shl_sorted,
+                          void* d_out, int div, void* stream);
 /* Work list (owner, first index) pairs [total][2] covering range(count_i) of
  * each owner i in steps of `size`, from d_first = the exclusive prefix sums
  * of ceil(count_i / size) (n + 1 entries, d_first[n] = total): the chunk

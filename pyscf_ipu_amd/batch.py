@@ -215,10 +215,10 @@ class BatchRKS:
         self.kp = int(bas[:, 2].max()) if len(bas) else 1
         self.sizes = {"eri": int(n_s8.sum()), "mat": int((nao * nao).sum()), "vec": int(nao.sum()),
                       "ao": int(ao_sz.sum()), "state": int(st.sum()), "grid": int(ngrid.sum())}
-        # work lists of the grid expansion (per atom) and of the six ERI classes
-        # (per molecule): chunk counts here, the (owner, first) lists built on
-        # the device at set-up (pscf_batch_chunks)
+        # work list of the grid expansion (per atom): chunk counts here, the
+        # (owner, first) list built on the device at set-up (pscf_batch_chunks)
         self.grid_counts = apts
+        # shell quartets per molecule of each ERI class
         self.eri_counts = []
         for X, Y in CLASSES:
             nx, ny = class_pairs(X, ns, npp), class_pairs(Y, ns, npp)
@@ -309,14 +309,11 @@ class BatchRKS:
             self.Dt.copy_(dm0)
         # ERIs
         self.eri = device.empty(S["eri"], T)
-        works = [self._work_list(c) for c in self.eri_counts]
-        arr = (ctypes.c_void_p * 6)(*[w.data_ptr() for w in works])
-        cnt = (ctypes.c_int * 6)(*[w.shape[0] for w in works])
         tm("eri_s8")
         # stored over their multiplicity as they are written, the form the J/K
         # contraction takes
-        _lib.call("pscf_batch_eri_s8_div", self.code, P(self.d_desc), self.M, arr, cnt, P(self.d_atm),
-                  P(self.d_bas), P(self.d_env), P(self.d_shell_ao), P(self.d_shl), P(self.eri), st)
+        _lib.call("pscf_batch_eri_s8_all", self.code, P(self.d_desc), P(self.d_order), self.M, P(self.d_atm),
+                  P(self.d_bas), P(self.d_env), P(self.d_shell_ao), P(self.d_shl), P(self.eri), 1, st)
         tm("end")
         # iteration buffers.  dJK is FP64; in FP32 mode it is built
         # incrementally, dJK += JK(D_new - D_old) with the change in FP32, so the
@@ -340,7 +337,7 @@ class BatchRKS:
         # the last ENERGY_HIST iteration energies of each molecule (ring, slot = iteration % ENERGY_HIST)
         self.E_hist = device.zeros((self.M, ENERGY_HIST), f64)
         self.state = device.zeros(S["state"], f64)
-        self._keep = [gw, ae, ap0, am, toff, tn, tg] + works
+        self._keep = [gw, ae, ap0, am, toff, tn, tg]
         torch.cuda.synchronize()
 
     # ---------------------------------------------------------------- iterations ---

@@ -3,19 +3,19 @@
 // The reference's ERI generator is libcint's Rys-quadrature scheme
 // (pyscf_ipu/electron_repulsion/int2e_sph.cpp: CINTg0_2e :1785-1900, 2D
 // recurrence CINTg0_2e_2d :1475-1600, primitive loop CINT2e_loop_nopt
-// :2452-2723, one shell quartet per IPU tile).  Here the same quadrature runs
-// one contracted shell quartet per GPU lane, with every wavefront of a launch
-// in a single angular class (ss|ss), (ps|ss), (ps|ps), (pp|ss), (pp|ps) or
-// (pp|pp), so the per-class code is fully unrolled and branch-free:
+// :2452-2723, one shell quartet per IPU tile).  The packed s8 arrays come from
+// the shell-pair engine of eri_pairs.h.  The same quadrature as libcint's, one
+// contracted shell quartet per lane, serves explicit quartet lists
+// (pscf_eri_quartets), batches given by quartet work lists
+// (pscf_batch_eri_s8, pscf_batch_eri_s8_div) and the gradient:
 //   * Boys F_m(T) from a Taylor table staged in LDS (F_0..F_14 on a 0.1 grid
 //     up to T = 39.9, asymptote above),
 //   * Rys roots/weights from the Boys moments in closed form (1-3 roots), FP64,
 //   * 2D recurrence G(n, m) per root and axis, horizontal transfer to
 //     (i j | k l), accumulation of sum_r w_r Ix Iy Iz over primitive quartets.
-// Launches for the packed s8 array enumerate (bra pair, ket pair) directly from
-// a class-sorted shell-pair list, so no quartet list is materialised.
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "batch.h"
@@ -26,6 +26,29 @@ namespace pscf {
 
 // --------------------------------------------------------------- Boys table ---
 __device__ double g_boys[BOYS_NT * BOYS_NM];
+// Prefix sum of shell widths (2l+1) into LDS, by the first wave.
+__device__ inline void stage_ao_loc(int* ao_loc, const int* __restrict__ bas, int nbas) {
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  for (int i0 = 0; i0 < nbas && threadIdx.x < 64; i0 += 64) {
+    const int w = i0 + lane < nbas ? 2 * bas[(i0 + lane) * BAS_SLOTS + 1] + 1 : 0;
+    int inc = w;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(inc, d);
+      if (lane >= d) inc += v;
+    }
+    if (i0 + lane < nbas) ao_loc[i0 + lane] = base + inc - w;
+    base += __shfl(inc, 63);
+  }
+  if (threadIdx.x == 0) ao_loc[nbas] = base;
+}
+
+}  // namespace pscf
+
+#include "eri_pairs.h"
+
+namespace pscf {
 static std::mutex g_boys_mu;
 static bool g_boys_ready[64];
 
@@ -71,6 +94,15 @@ static int ensure_boys_table() {
     for (int m = 0; m < BOYS_NM; m++) tab[i * BOYS_NM + m] = (double)f[m];
   }
   PSCF_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_boys), tab.data(), sizeof(double) * tab.size(), 0, hipMemcpyHostToDevice));
+  std::vector<float> tabf((BOYSF_LMAX + 1) * BOYSF_NT * 4);
+  for (int i = 0; i < BOYSF_NT; i++) {
+    boys_row_host((long double)i / 16.0L, f);
+    for (int l = 0; l <= BOYSF_LMAX; l++) {
+      float* row = &tabf[(l * BOYSF_NT + i) * 4];
+      for (int k = 0; k < 4; k++) row[k] = (float)(f[l + k] / (k == 3 ? 6 : (k == 2 ? 2 : 1)));
+    }
+  }
+  PSCF_HIP(hipMemcpyToSymbol(HIP_SYMBOL(g_boysf), tabf.data(), sizeof(float) * tabf.size(), 0, hipMemcpyHostToDevice));
   if (dev < 64) g_boys_ready[dev] = true;
   return PSCF_OK;
 }
@@ -99,18 +131,6 @@ __device__ inline ShellD load_shell(const int* __restrict__ atm, const int* __re
   return s;
 }
 
-// Prefix sum of shell widths (2l+1) into LDS.
-__device__ inline void stage_ao_loc(int* ao_loc, const int* __restrict__ bas, int nbas) {
-  if (threadIdx.x == 0) {
-    int acc = 0;
-    for (int i = 0; i < nbas; i++) {
-      ao_loc[i] = acc;
-      acc += 2 * bas[i * BAS_SLOTS + 1] + 1;
-    }
-    ao_loc[nbas] = acc;
-  }
-}
-
 template <int L>
 struct NComp {
   static constexpr int v = L ? 3 : 1;
@@ -129,11 +149,9 @@ __device__ constexpr int cexp(int f, int d) {
 // unroll and the ket-pair data (exponent sum, its reciprocal, the Gaussian
 // product prefactor with its exp) is computed once per contracted quartet
 // instead of once per bra primitive pair; NPC = 0 reads the counts at run time.
-// SCREEN (FP32, quartets of four 3-primitive shells): bra primitive pairs with
-// a negligible Gaussian-product prefactor skip their ket loop (bound below).
-template <typename T, typename BT, int NTERMS, int LI, int LJ, int LK, int LL, int NPC, bool SCREEN>
+template <typename T, typename BT, int NTERMS, int LI, int LJ, int LK, int LL, int NPC>
 __device__ inline void shell_quartet_np(const ShellD& A, const ShellD& B, const ShellD& C, const ShellD& D,
-                                        const BT* __restrict__ tab, T* acc, bool screen) {
+                                        const BT* __restrict__ tab, T* acc) {
   constexpr int NR = (LI + LJ + LK + LL) / 2 + 1;
   constexpr int NMAX = LI + LJ, MMAX = LK + LL;
   constexpr int NI = NComp<LI>::v, NJ = NComp<LJ>::v, NK = NComp<LK>::v, NL = NComp<LL>::v;
@@ -178,16 +196,6 @@ __device__ inline void shell_quartet_np(const ShellD& A, const ShellD& B, const 
       const T aj = (T)B.e[pb];
       const T aij = ai + aj, r_aij = drcp<T>(aij);
       const T kab = dexp<T>(-ai * aj * r_aij * rab2) * ca * (T)B.c[pb];
-      // SCREEN: a bra primitive pair whose Gaussian-product prefactor is below
-      // the bound skips its ket loop.  What it would add to an ERI is at most
-      // 34.99 r_aij |kab| (akl^-3/2 <= 5.1) (sum of |kcd| over the 3 x 3 ket
-      // primitive pairs, <= 9 x 15^2 for STO-3G shells) angc (<= 0.06) times
-      // the 1D-integral products (< 1e5 for molecules under 20 bohr): below
-      // 1e-10, far under the FP32 rounding of the ERIs themselves (~1e-7 of the
-      // largest).  The lanes of a wave mostly share their bra pair, so whole
-      // waves skip together.
-      if constexpr (SCREEN && sizeof(T) == 4)
-        if (screen && fabsf(kab) * r_aij < 4e-20f) continue;
       T PA[3], P[3];
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
@@ -305,17 +313,15 @@ __device__ inline void shell_quartet_np(const ShellD& A, const ShellD& B, const 
 // (ps|ss), the most numerous) four shells with 3 primitives (every STO-3G
 // shell) take the unrolled, ket-hoisted form; the multi-root classes and FP64
 // keep rolled loops (unrolled, they need more registers than a lane has).
-// SCREEN (the batched STO-3G form) enables the primitive-pair screening of
-// shell_quartet_np on quartets of four 3-primitive shells.
-template <typename T, typename BT, int NTERMS, int LI, int LJ, int LK, int LL, bool SCREEN = false>
+template <typename T, typename BT, int NTERMS, int LI, int LJ, int LK, int LL>
 __device__ inline void shell_quartet(const ShellD& A, const ShellD& B, const ShellD& C, const ShellD& D,
                                      const BT* __restrict__ tab, T* acc) {
   constexpr bool ONE_ROOT = LI + LJ + LK + LL <= 1 && sizeof(T) == 4;  // FP32 (FP64 would need 2x the registers)
   const bool np3 = A.np == 3 && B.np == 3 && C.np == 3 && D.np == 3;
   if (ONE_ROOT && np3)
-    shell_quartet_np<T, BT, NTERMS, LI, LJ, LK, LL, ONE_ROOT ? 3 : 0, SCREEN>(A, B, C, D, tab, acc, true);
+    shell_quartet_np<T, BT, NTERMS, LI, LJ, LK, LL, ONE_ROOT ? 3 : 0>(A, B, C, D, tab, acc);
   else
-    shell_quartet_np<T, BT, NTERMS, LI, LJ, LK, LL, 0, SCREEN>(A, B, C, D, tab, acc, np3);
+    shell_quartet_np<T, BT, NTERMS, LI, LJ, LK, LL, 0>(A, B, C, D, tab, acc);
 }
 
 template <typename BT>
@@ -346,98 +352,6 @@ template <>
 struct BoysType<float, 1> {
   using type = float;
 };
-
-// Quartet q of class (X, Y) of a molecule's s8 array: pair a of class X and
-// pair b of class Y (a >= b within one class), pairs listed from x0 / y0.
-template <typename T, int X, int Y>
-__device__ inline void s8_quartet(const int* __restrict__ atm, const int* __restrict__ bas,
-                                  const double* __restrict__ env, const int* __restrict__ ao_loc,
-                                  const int* __restrict__ pairs, int x0, int nx, int y0, int ny, int64_t q,
-                                  const double* tab64, const float* tab32, T* __restrict__ out) {
-  constexpr int LI = PairL<X>::a, LJ = PairL<X>::b, LK = PairL<Y>::a, LL = PairL<Y>::b;
-  constexpr int NR = (LI + LJ + LK + LL) / 2 + 1;
-  using BT = typename BoysType<T, NR>::type;
-  const BT* tab;
-  if constexpr (sizeof(BT) == 8) tab = tab64; else tab = tab32;
-  const bool tri_launch = (X == Y);
-  const int64_t total = tri_launch ? tri((int64_t)nx) : (int64_t)nx * ny;
-  if (q >= total) return;
-  int64_t a, b;
-  if (tri_launch) {
-    a = (int64_t)((sqrt(8.0 * (double)q + 1.0) - 1.0) * 0.5);
-    while (tri(a + 1) <= q) ++a;
-    while (tri(a) > q) --a;
-    b = q - tri(a);
-  } else {
-    a = q / ny;
-    b = q - a * ny;
-  }
-  const int i = pairs[2 * (x0 + a)], j = pairs[2 * (x0 + a) + 1];
-  const int k = pairs[2 * (y0 + b)], l = pairs[2 * (y0 + b) + 1];
-  const ShellD A = load_shell(atm, bas, env, ao_loc, i), B = load_shell(atm, bas, env, ao_loc, j);
-  const ShellD C = load_shell(atm, bas, env, ao_loc, k), D = load_shell(atm, bas, env, ao_loc, l);
-  constexpr int NI = NComp<LI>::v, NJ = NComp<LJ>::v, NK = NComp<LK>::v, NL = NComp<LL>::v;
-  T acc[NI * NJ * NK * NL];
-  shell_quartet<T, BT, BoysTerms<BT>::v, LI, LJ, LK, LL>(A, B, C, D, tab, acc);
-  const bool diag_bra = (i == j), diag_ket = (k == l), same_pair = tri_launch && (a == b);
-#pragma unroll
-  for (int fi = 0; fi < NI; ++fi)
-#pragma unroll
-    for (int fj = 0; fj < NJ; ++fj)
-#pragma unroll
-      for (int fk = 0; fk < NK; ++fk)
-#pragma unroll
-        for (int fl = 0; fl < NL; ++fl) {
-          const int64_t p = A.ao0 + fi, qq = B.ao0 + fj, r = C.ao0 + fk, s = D.ao0 + fl;
-          if (diag_bra && qq > p) continue;
-          if (diag_ket && s > r) continue;
-          const int64_t pq = p >= qq ? tri(p) + qq : tri(qq) + p;
-          const int64_t rs = r >= s ? tri(r) + s : tri(s) + r;
-          if (same_pair && rs > pq) continue;
-          const int64_t idx = pq >= rs ? tri(pq) + rs : tri(rs) + pq;
-          out[idx] = acc[((fi * NJ + fj) * NK + fk) * NL + fl];
-        }
-}
-
-// The six shell-pair classes of one molecule in one launch, so they run side
-// by side rather than one after another: blocks [b0[c], b0[c + 1]) take class
-// S8_ORDER[c], the heaviest first.  off / cnt: each pair class's first pair
-// and count in `pairs` (s-s, p-s, p-p).
-constexpr int S8_CLASSES = 6;
-struct S8Launch {
-  int off[3], cnt[3];
-  int b0[S8_CLASSES + 1];
-};
-
-template <typename T>
-__global__ void __launch_bounds__(256) eri_s8_kernel(const int* __restrict__ atm, const int* __restrict__ bas,
-                                                     const double* __restrict__ env, int nbas,
-                                                     const int* __restrict__ pairs, S8Launch L,
-                                                     T* __restrict__ out) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  double* tab64 = reinterpret_cast<double*>(smem);
-  float* tab32 = reinterpret_cast<float*>(smem + sizeof(double) * BOYS_NT * BOYS_NM);
-  int* ao_loc = reinterpret_cast<int*>(smem + (sizeof(double) + sizeof(float)) * BOYS_NT * BOYS_NM);
-  for (int i = threadIdx.x; i < BOYS_NT * BOYS_NM; i += blockDim.x) {
-    tab64[i] = g_boys[i];
-    if constexpr (sizeof(T) == 4) tab32[i] = (float)g_boys[i];
-  }
-  stage_ao_loc(ao_loc, bas, nbas);
-  __syncthreads();
-  const int b = blockIdx.x;
-  const int c = b < L.b0[1] ? 0 : b < L.b0[2] ? 1 : b < L.b0[3] ? 2 : b < L.b0[4] ? 3 : b < L.b0[5] ? 4 : 5;
-  const int64_t q = (int64_t)(b - L.b0[c]) * blockDim.x + threadIdx.x;
-  const int* o = L.off;
-  const int* n = L.cnt;
-  switch (c) {  // S8_ORDER: (2,2), (2,1), (2,0), (1,1), (1,0), (0,0)
-    case 0: s8_quartet<T, 2, 2>(atm, bas, env, ao_loc, pairs, o[2], n[2], o[2], n[2], q, tab64, tab32, out); break;
-    case 1: s8_quartet<T, 2, 1>(atm, bas, env, ao_loc, pairs, o[2], n[2], o[1], n[1], q, tab64, tab32, out); break;
-    case 2: s8_quartet<T, 2, 0>(atm, bas, env, ao_loc, pairs, o[2], n[2], o[0], n[0], q, tab64, tab32, out); break;
-    case 3: s8_quartet<T, 1, 1>(atm, bas, env, ao_loc, pairs, o[1], n[1], o[1], n[1], q, tab64, tab32, out); break;
-    case 4: s8_quartet<T, 1, 0>(atm, bas, env, ao_loc, pairs, o[1], n[1], o[0], n[0], q, tab64, tab32, out); break;
-    default: s8_quartet<T, 0, 0>(atm, bas, env, ao_loc, pairs, o[0], n[0], o[0], n[0], q, tab64, tab32, out); break;
-  }
-}
 
 // Quartets of an explicit list; each lane canonicalises its quartet to a class
 // with l_i >= l_j, l_k >= l_l, (l_i + l_j) >= (l_k + l_l) and writes the block
@@ -691,95 +605,6 @@ __global__ void __launch_bounds__(256) int1e_kernel(const int* __restrict__ atm,
 }
 
 // ------------------------------------------------------------ batched form ---
-// Shell pair a of class X from a molecule's class-sorted shell list
-// (s shells then p shells): ss = tri over s, ps = (p, s) rectangle, pp = tri over p.
-template <int X>
-__device__ inline void pair_shells(int64_t a, int ns, int np, const int* __restrict__ sl, int& i, int& j) {
-  if (X == 1) {
-    i = sl[ns + (int)(a / ns)];
-    j = sl[(int)(a % ns)];
-  } else {
-    int64_t t = (int64_t)((sqrt(8.0 * (double)a + 1.0) - 1.0) * 0.5);
-    while (tri(t + 1) <= a) ++t;
-    while (tri(t) > a) --t;
-    const int base = X == 0 ? 0 : ns;
-    i = sl[base + (int)t];
-    j = sl[base + (int)(a - tri(t))];
-  }
-}
-
-__host__ __device__ inline int64_t class_pairs(int X, int64_t ns, int64_t np) {
-  return X == 0 ? tri(ns) : (X == 1 ? ns * np : tri(np));
-}
-
-// One chunk of <= 256 quartets of class (X, Y) of one molecule per workgroup.
-template <typename T, int X, int Y>
-__global__ void __launch_bounds__(256) eri_s8_batch_kernel(const BatchMol* __restrict__ mols,
-                                                           const int* __restrict__ work,
-                                                           const int* __restrict__ atm, const int* __restrict__ bas,
-                                                           const double* __restrict__ env,
-                                                           const int* __restrict__ shell_ao,
-                                                           const int* __restrict__ shl_sorted, T* __restrict__ out,
-                                                           int div) {
-  constexpr int LI = PairL<X>::a, LJ = PairL<X>::b, LK = PairL<Y>::a, LL = PairL<Y>::b;
-  constexpr int NR = (LI + LJ + LK + LL) / 2 + 1;
-  using BT = typename BoysType<T, NR>::type;
-  extern __shared__ __align__(16) unsigned char smem[];
-  BT* tab = reinterpret_cast<BT*>(smem);
-  for (int i = threadIdx.x; i < BOYS_NT * BOYS_NM; i += blockDim.x) tab[i] = (BT)g_boys[i];
-  __syncthreads();
-  const int m = work[2 * blockIdx.x];
-  const int64_t q = (int64_t)work[2 * blockIdx.x + 1] + threadIdx.x;
-  const BatchMol M = mols[m];
-  const int ns = (int)M.ns, np = (int)M.np;
-  const int64_t nx = class_pairs(X, ns, np), ny = class_pairs(Y, ns, np);
-  const bool tri_launch = (X == Y);
-  const int64_t total = tri_launch ? tri(nx) : nx * ny;
-  if (q >= total) return;
-  int64_t a, b;
-  if (tri_launch) {
-    a = (int64_t)((sqrt(8.0 * (double)q + 1.0) - 1.0) * 0.5);
-    while (tri(a + 1) <= q) ++a;
-    while (tri(a) > q) --a;
-    b = q - tri(a);
-  } else {
-    a = q / ny;
-    b = q - a * ny;
-  }
-  const int* sl = shl_sorted + M.shl0;
-  int i, j, k, l;
-  pair_shells<X>(a, ns, np, sl, i, j);
-  pair_shells<Y>(b, ns, np, sl, k, l);
-  // shell_ao holds each shell's first AO within its molecule
-  const ShellD A = load_shell(atm, bas, env, shell_ao, i), B = load_shell(atm, bas, env, shell_ao, j);
-  const ShellD C = load_shell(atm, bas, env, shell_ao, k), D = load_shell(atm, bas, env, shell_ao, l);
-  constexpr int NI = NComp<LI>::v, NJ = NComp<LJ>::v, NK = NComp<LK>::v, NL = NComp<LL>::v;
-  T acc[NI * NJ * NK * NL];
-  shell_quartet<T, BT, BoysTerms<BT>::v, LI, LJ, LK, LL, true>(A, B, C, D, tab, acc);
-  const bool diag_bra = (i == j), diag_ket = (k == l), same_pair = tri_launch && (a == b);
-  T* dst = out + M.eri0;
-#pragma unroll
-  for (int fi = 0; fi < NI; ++fi)
-#pragma unroll
-    for (int fj = 0; fj < NJ; ++fj)
-#pragma unroll
-      for (int fk = 0; fk < NK; ++fk)
-#pragma unroll
-        for (int fl = 0; fl < NL; ++fl) {
-          const int64_t p = A.ao0 + fi, qq = B.ao0 + fj, r = C.ao0 + fk, s = D.ao0 + fl;
-          if (diag_bra && qq > p) continue;
-          if (diag_ket && s > r) continue;
-          const int64_t pq = p >= qq ? tri(p) + qq : tri(qq) + p;
-          const int64_t rs = r >= s ? tri(r) + s : tri(s) + r;
-          if (same_pair && rs > pq) continue;
-          const int64_t idx = pq >= rs ? tri(pq) + rs : tri(rs) + pq;
-          T v = acc[((fi * NJ + fj) * NK + fk) * NL + fl];
-          // div: over the element's multiplicity 2^([p==q] + [r==s] + [pq==rs])
-          if (div) v *= T(1.0 / (double)(1 << ((p == qq) + (r == s) + (pq == rs))));
-          dst[idx] = v;
-        }
-}
-
 // One workgroup per molecule, one wave per shell pair: S and H_core = T + V.
 __global__ void __launch_bounds__(256) int1e_batch_kernel(const BatchMol* __restrict__ mols,
                                                           const int* __restrict__ atm, const int* __restrict__ bas,
@@ -1053,26 +878,42 @@ __global__ void __launch_bounds__(256) eri_grad_kernel(const int* __restrict__ a
     if (g_lds[i] != 0.0) atomicAdd(grad + i, g_lds[i]);
 }
 
+// Tile shapes (bra x ket shell pairs), large to small.
+static const int EP_SHAPES[][2] = {{32, 64}, {16, 64}, {16, 32}, {8, 32}, {8, 16}, {4, 16}};
+// relative cost of a shell quartet of each class (instructions per primitive quartet)
+static const double EP_COST[EP_CLASSES] = {15, 4, 1.6, 2, 1.3, 1};
+
 template <typename T>
 static int eri_s8_all(const int* atm, const int* bas, const double* env, int nbas, const int* pairs, const int* cnt,
                       T* out, hipStream_t st) {
-  static const int order[S8_CLASSES][2] = {{2, 2}, {2, 1}, {2, 0}, {1, 1}, {1, 0}, {0, 0}};
-  S8Launch L;
-  L.off[0] = 0;
-  L.off[1] = cnt[0];
-  L.off[2] = cnt[0] + cnt[1];
-  for (int x = 0; x < 3; ++x) L.cnt[x] = cnt[x];
+  EpLaunch E;
+  E.off[0] = 0;
+  E.off[1] = cnt[0];
+  E.off[2] = cnt[0] + cnt[1];
+  double total = 0;
+  for (int x = 0; x < 3; ++x) E.cnt[x] = cnt[x];
+  for (int c = 0; c < EP_CLASSES; ++c) total += EP_COST[c] * s8_class_quartets(EP_X[c], EP_Y[c], cnt);
+  // the largest tile that still gives about three workgroups per CU: a tile
+  // stages its primitives once, but one molecule has to spread over the chip
   int64_t blocks = 0;
-  for (int c = 0; c < S8_CLASSES; ++c) {
-    L.b0[c] = (int)blocks;
-    blocks += (s8_class_quartets(order[c][0], order[c][1], cnt) + 255) / 256;
+  for (int c = 0; c < EP_CLASSES; ++c) {
+    int k = 0;
+    const int last = (int)(sizeof(EP_SHAPES) / sizeof(EP_SHAPES[0])) - 1;
+    while (k < last && EP_COST[c] * EP_SHAPES[k][0] * EP_SHAPES[k][1] > total / 768) ++k;
+    E.na[c] = EP_SHAPES[k][0];
+    E.nb[c] = EP_SHAPES[k][1];
+    E.b0[c] = (int)blocks;
+    const int64_t nx = cnt[EP_X[c]], ny = cnt[EP_Y[c]];
+    blocks += c == 0 ? EpRun<T, 0, true>::tiles(nx, ny, E.na[c], E.nb[c])
+                     : (EP_X[c] == EP_Y[c] ? ep_tiles<1, 1>(nx, ny, E.na[c], E.nb[c])
+                                           : ep_tiles<0, 1>(nx, ny, E.na[c], E.nb[c]));
     PSCF_REQUIRE(blocks < (1ll << 31), "pscf_eri_s8: too many quartets");
   }
-  L.b0[S8_CLASSES] = (int)blocks;
+  E.b0[EP_CLASSES] = (int)blocks;
+  const size_t shm = ep_lds_max<T>() + sizeof(int) * (nbas + 1);
   if (blocks == 0) return PSCF_OK;
-  const size_t shm = (sizeof(double) + sizeof(float)) * BOYS_NT * BOYS_NM + sizeof(int) * (nbas + 1);
-  PSCF_SET_LDS(eri_s8_kernel<T>, shm);
-  eri_s8_kernel<T><<<(unsigned)blocks, 256, shm, st>>>(atm, bas, env, nbas, pairs, L, out);
+  PSCF_SET_LDS((eri_s8_kernel<T>), shm);
+  eri_s8_kernel<T><<<(unsigned)blocks, EP_THREADS, shm, st>>>(atm, bas, env, nbas, pairs, E, out);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
 }
@@ -1371,15 +1212,16 @@ extern "C" int pscf_int1e(const int* d_atm, int natm, const int* d_bas, int nbas
   return PSCF_OK;
 }
 
-template <typename T, int X, int Y>
-static int launch_batch_s8(const BatchMol* mols, const int* work, int nwork, const int* atm, const int* bas,
-                           const double* env, const int* shell_ao, const int* shl, T* out, int div, hipStream_t st) {
-  if (nwork == 0) return PSCF_OK;
-  constexpr int LI = PairL<X>::a, LJ = PairL<X>::b, LK = PairL<Y>::a, LL = PairL<Y>::b;
-  constexpr int NR = (LI + LJ + LK + LL) / 2 + 1;
-  using BT = typename BoysType<T, NR>::type;
-  const size_t shm = sizeof(BT) * BOYS_NT * BOYS_NM;
-  eri_s8_batch_kernel<T, X, Y><<<nwork, 256, shm, st>>>(mols, work, atm, bas, env, shell_ao, shl, out, div);
+// The lists come lightest class first: list l holds class EP_CLASSES - 1 - l.
+template <typename T, int C>
+static int launch_list(const BatchMol* mols, const int* const* work, const int* nwork, const int* atm, const int* bas,
+                       const double* env, const int* shell_ao, const int* shl, T* out, int div, hipStream_t st) {
+  const int n = nwork[EP_CLASSES - 1 - C];
+  if (n == 0) return PSCF_OK;
+  const size_t shm = ep_lds<T, C>();
+  PSCF_SET_LDS((eri_s8_list_kernel<T, C>), shm);
+  eri_s8_list_kernel<T, C><<<(n + EP_GROUP - 1) / EP_GROUP, EP_THREADS, shm, st>>>(
+      mols, work[EP_CLASSES - 1 - C], n, atm, bas, env, shell_ao, shl, out, div);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
 }
@@ -1387,14 +1229,13 @@ static int launch_batch_s8(const BatchMol* mols, const int* work, int nwork, con
 template <typename T>
 static int batch_s8_all(const BatchMol* mols, const int* const* work, const int* nwork, const int* atm, const int* bas,
                         const double* env, const int* shell_ao, const int* shl, T* out, int div, hipStream_t st) {
-  int rc;
-  if ((rc = launch_batch_s8<T, 0, 0>(mols, work[0], nwork[0], atm, bas, env, shell_ao, shl, out, div, st))) return rc;
-  if ((rc = launch_batch_s8<T, 1, 0>(mols, work[1], nwork[1], atm, bas, env, shell_ao, shl, out, div, st))) return rc;
-  if ((rc = launch_batch_s8<T, 1, 1>(mols, work[2], nwork[2], atm, bas, env, shell_ao, shl, out, div, st))) return rc;
-  if ((rc = launch_batch_s8<T, 2, 0>(mols, work[3], nwork[3], atm, bas, env, shell_ao, shl, out, div, st))) return rc;
-  if ((rc = launch_batch_s8<T, 2, 1>(mols, work[4], nwork[4], atm, bas, env, shell_ao, shl, out, div, st))) return rc;
-  if ((rc = launch_batch_s8<T, 2, 2>(mols, work[5], nwork[5], atm, bas, env, shell_ao, shl, out, div, st))) return rc;
-  return PSCF_OK;
+  int rc = launch_list<T, 0>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_list<T, 1>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_list<T, 2>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_list<T, 3>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_list<T, 4>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_list<T, 5>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
+  return rc;
 }
 
 static int batch_eri_s8_any(int dtype, const void* d_mols, int nmol, const int* const* h_work, const int* h_nwork,
@@ -1413,6 +1254,52 @@ static int batch_eri_s8_any(int dtype, const void* d_mols, int nmol, const int* 
                                 d_shl_sorted, (double*)d_out, div, st);
   return batch_s8_all<float>((const BatchMol*)d_mols, h_work, h_nwork, d_atm, d_bas, d_env, d_shell_ao, d_shl_sorted,
                              (float*)d_out, div, st);
+}
+
+// Tiles: the heavy classes have few pairs per molecule, so theirs are small; a
+// small batch takes smaller tiles still, to spread over the chip.
+template <typename T, int C>
+static int launch_mols(const BatchMol* mols, const int* order, int nmol, const int* atm, const int* bas,
+                       const double* env, const int* shell_ao, const int* shl, T* out, int div, hipStream_t st) {
+  static const int big[EP_CLASSES][2] = {{4, 64}, {8, 64}, {16, 64}, {16, 64}, {32, 64}, {32, 64}};
+  static const int small[EP_CLASSES][2] = {{4, 16}, {4, 16}, {16, 32}, {8, 32}, {16, 32}, {16, 32}};
+  const int* tile = nmol >= 32 ? big[C] : small[C];
+  const int per = (nmol >= 8192 ? 4 : (nmol <= 256 ? 128 : 32768 / nmol)) - 1;
+  PSCF_REQUIRE((int64_t)nmol * per < (1ll << 31), "pscf_batch_eri_s8_all: too many molecules");
+  const size_t shm = ep_lds<T, C>();
+  PSCF_SET_LDS((eri_s8_mols_kernel<T, C>), shm);
+  eri_s8_mols_kernel<T, C><<<(unsigned)nmol * per, EP_THREADS, shm, st>>>(mols, order, per, atm, bas, env, shell_ao,
+                                                                          shl, tile[0], tile[1], out, div);
+  PSCF_HIP(hipGetLastError());
+  return PSCF_OK;
+}
+
+template <typename T>
+static int mols_all(const BatchMol* mols, const int* order, int nmol, const int* atm, const int* bas, const double* env,
+                    const int* shell_ao, const int* shl, T* out, int div, hipStream_t st) {
+  int rc = launch_mols<T, 0>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_mols<T, 1>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_mols<T, 2>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_mols<T, 3>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_mols<T, 4>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_mols<T, 5>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
+  return rc;
+}
+
+extern "C" int pscf_batch_eri_s8_all(int dtype, const void* d_mols, const int* d_order, int nmol, const int* d_atm,
+                                     const int* d_bas, const double* d_env, const int* d_shell_ao,
+                                     const int* d_shl_sorted, void* d_out, int div, void* stream) {
+  PSCF_REQUIRE(dtype == PSCF_F64 || dtype == PSCF_F32, "pscf_batch_eri_s8_all: bad dtype");
+  PSCF_REQUIRE(nmol > 0 && d_mols && d_atm && d_bas && d_env && d_shell_ao && d_shl_sorted && d_out,
+               "pscf_batch_eri_s8_all: bad arguments");
+  int rc = ensure_boys_table();
+  if (rc) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == PSCF_F64)
+    return mols_all<double>((const BatchMol*)d_mols, d_order, nmol, d_atm, d_bas, d_env, d_shell_ao, d_shl_sorted,
+                            (double*)d_out, div, st);
+  return mols_all<float>((const BatchMol*)d_mols, d_order, nmol, d_atm, d_bas, d_env, d_shell_ao, d_shl_sorted,
+                         (float*)d_out, div, st);
 }
 
 extern "C" int pscf_batch_eri_s8(int dtype, const void* d_mols, int nmol, const int* const* h_work,
