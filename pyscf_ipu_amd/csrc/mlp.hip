@@ -11,6 +11,7 @@
 
 #include "batch.h"
 #include "common.h"
+#include "wave.h"
 
 namespace pscf {
 
@@ -40,12 +41,202 @@ enum Epilogue : int {
   EPI_BIAS = 1,       // out = acc + b (FP32)
   EPI_DSILU = 2,      // dZ = acc * dsilu(Zprev) -> FP32 out and BF16 out2
   EPI_ATOMIC = 3,     // out += acc (FP32 atomics; split-K)
+  EPI_DSILU_SUM = 4,  // out2 = dZ = acc * dsilu(Zprev) (BF16), out[n] += sum_m dZ[m][n] (FP32 atomics)
 };
 
 constexpr int GBM = 64, GBN = 64, GBK = 16;
 
+// What to do with one accumulated element (row, col).
+template <int EPI>
+__device__ __forceinline__ float gemm_store(float v, int row, int col, int64_t o, const float* __restrict__ bias,
+                                            const float* __restrict__ aux, float* __restrict__ out,
+                                            bf16_t* __restrict__ out2) {
+  if (EPI == EPI_BIAS_SILU) {
+    const float z = v + bias[col];
+    out[o] = z;
+    out2[o] = f2bf(silu(z));
+  } else if (EPI == EPI_BIAS) {
+    out[o] = v + bias[col];
+  } else if (EPI == EPI_DSILU || EPI == EPI_DSILU_SUM) {
+    v *= dsilu(aux[o]);
+    if (EPI == EPI_DSILU) out[o] = v;
+    out2[o] = f2bf(v);
+  } else {
+    atomicAdd(out + o, v);
+  }
+  return v;
+}
+
+// ------------------------------------------------------------ tiled GEMM ----
+// The same product for operands with 16-byte aligned rows (every layer of the
+// network): 16-byte global loads one K step ahead of the MFMAs, both operands
+// staged as [row][k] (a k-major operand is transposed on the way, four k rows
+// at a time), fragments read as one ds_read_b64.  Row stride 36 elements: the
+// fragment reads and the transposing writes fall on all banks.  Each output
+// accumulates k in steps of 16 in order, as in gemm_bf16_kernel: same bits.
+// 16384 rows: a hidden layer 28 -> 17 us (its 34 MB take 7 at HBM rate; 128 x
+// 128 tiles, one workgroup per CU: 25), backward data with its column sums 68
+// -> 18 us, a weight gradient 64 -> 16 us; a training step 653 -> 182 us.
+// Row stride of the staged operands: the fragment reads (16 rows, 8 bytes) and
+// the transposing writes fall on all banks.
+constexpr int tile_stride(int TK) { return TK == 32 ? 36 : TK + 16; }
+
+// Stages rows [r0, r0 + R) x k [k0, k0 + TK) of a [row][k] operand (T: stored [k][row]).
+template <int R, int TK, bool T>
+struct TileLoad {
+  static constexpr int KP = TK / 8, NT = (R * KP + 255) / 256;  // 16-byte pieces per row, per thread
+  static constexpr int KQ = TK / 4, TASKS = KQ * R / 8;         // T: blocks of four k rows x eight rows
+  static_assert(!T || TASKS <= 256, "one transposing block per thread");
+  uint4 v[T ? 4 : NT];
+  __device__ inline void load(const bf16_t* __restrict__ P, int ld, int r0, int rows, int k0, int kend) {
+    const int tid = threadIdx.x;
+    if constexpr (!T) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        const int e = tid + 256 * i, r = e / KP, k = k0 + (e % KP) * 8;
+        uint4 x = {0, 0, 0, 0};
+        if (r < R && r0 + r < rows && k < kend) {
+          x = *reinterpret_cast<const uint4*>(P + (int64_t)(r0 + r) * ld + k);
+          if (k + 8 > kend) {  // the tail of the last piece is not part of K
+            unsigned* w = reinterpret_cast<unsigned*>(&x);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              if (k + 2 * q >= kend) w[q] = 0;
+              else if (k + 2 * q + 1 >= kend) w[q] &= 0xffffu;
+            }
+          }
+        }
+        v[i] = x;
+      }
+    } else {
+      const int kq = tid % KQ, r = tid / KQ * 8;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = k0 + kq * 4 + q;
+        v[q] = tid < TASKS && k < kend && r0 + r < rows
+                   ? *reinterpret_cast<const uint4*>(P + (int64_t)k * ld + r0 + r)
+                   : uint4{0, 0, 0, 0};
+      }
+    }
+  }
+  __device__ inline void store(bf16_t* __restrict__ S) {
+    constexpr int TS = tile_stride(TK);
+    const int tid = threadIdx.x;
+    if constexpr (!T) {
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        const int e = tid + 256 * i, r = e / KP;
+        if (r < R) {
+          uint2* d = reinterpret_cast<uint2*>(S + r * TS + (e % KP) * 8);
+          d[0] = uint2{v[i].x, v[i].y};
+          d[1] = uint2{v[i].z, v[i].w};
+        }
+      }
+    } else if (tid < TASKS) {
+      const int kq = tid % KQ, r = tid / KQ * 8;
+      const unsigned* w0 = reinterpret_cast<const unsigned*>(&v[0]);
+      const unsigned* w1 = reinterpret_cast<const unsigned*>(&v[1]);
+      const unsigned* w2 = reinterpret_cast<const unsigned*>(&v[2]);
+      const unsigned* w3 = reinterpret_cast<const unsigned*>(&v[3]);
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {  // rows r + 2p and r + 2p + 1
+        *reinterpret_cast<uint2*>(S + (r + 2 * p) * TS + kq * 4) =
+            uint2{(w0[p] & 0xffffu) | (w1[p] << 16), (w2[p] & 0xffffu) | (w3[p] << 16)};
+        *reinterpret_cast<uint2*>(S + (r + 2 * p + 1) * TS + kq * 4) =
+            uint2{(w0[p] >> 16) | (w1[p] & 0xffff0000u), (w2[p] >> 16) | (w3[p] & 0xffff0000u)};
+      }
+    }
+  }
+};
+
+// Workgroup tile BM x BN, K in steps of TK, 4 waves of (BM / WM) x
+// (BN / (4 / WM)).  TA, TB as in gemm_bf16_kernel; blockIdx.z splits the K
+// steps (EPI_ATOMIC only).  A workgroup walks the row tiles blockIdx.y,
+// blockIdx.y + gridDim.y, ...
+template <int BM, int BN, int TK, int WM, bool TA, bool TB, int EPI>
+__global__ void __launch_bounds__(256) gemm_tile_kernel(int M, int N, int K, const bf16_t* __restrict__ A, int lda,
+                                                        const bf16_t* __restrict__ B, int ldb,
+                                                        const float* __restrict__ bias, const float* __restrict__ aux,
+                                                        float* __restrict__ out, bf16_t* __restrict__ out2, int ldc) {
+  constexpr int WN = 4 / WM, FM = BM / WM / 16, FN = BN / WN / 16, TS = tile_stride(TK);
+  __shared__ __align__(16) bf16_t As[BM * TS];
+  __shared__ __align__(16) bf16_t Bs[BN * TS];
+  __shared__ float csum[EPI == EPI_DSILU_SUM ? WM * BN : 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
+  const int n0 = blockIdx.x * BN;
+  const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
+  const int steps = (K + TK - 1) / TK, per = (steps + gridDim.z - 1) / gridDim.z;
+  const int s0 = blockIdx.z * per, s1 = min(steps, s0 + per);
+  if (s0 >= s1) return;
+  float sum[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) sum[j] = 0.f;
+  for (int m0 = blockIdx.y * BM; m0 < M; m0 += gridDim.y * BM) {
+    f32x4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    TileLoad<BM, TK, TA> la;
+    TileLoad<BN, TK, !TB> lb;
+    la.load(A, lda, m0, M, s0 * TK, K);
+    lb.load(B, ldb, n0, N, s0 * TK, K);
+    for (int s = s0; s < s1; ++s) {
+      __syncthreads();  // the last step's fragments are read
+      la.store(As);
+      lb.store(Bs);
+      __syncthreads();
+      if (s + 1 < s1) {
+        la.load(A, lda, m0, M, (s + 1) * TK, K);
+        lb.load(B, ldb, n0, N, (s + 1) * TK, K);
+      }
+#pragma unroll
+      for (int kk = 0; kk < TK; kk += 16) {
+        bf16x4 a[FM], b[FN];
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+          a[i] = *reinterpret_cast<const bf16x4*>(As + (wm + i * 16 + li) * TS + kk + 4 * lg);
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          b[j] = *reinterpret_cast<const bf16x4*>(Bs + (wn + j * 16 + li) * TS + kk + 4 * lg);
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[i], b[j], acc[i][j], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int col = n0 + wn + j * 16 + li;
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int row = m0 + wm + i * 16 + 4 * lg + q;
+          if (row < M && col < N)
+            sum[j] += gemm_store<EPI>(acc[i][j][q], row, col, (int64_t)row * ldc + col, bias, aux, out, out2);
+        }
+    }
+  }
+  if constexpr (EPI == EPI_DSILU_SUM) {  // one atomic per column and workgroup
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const float t = xor32_sum(xor16_sum(sum[j]));
+      if (lg == 0) csum[(wave / WN) * BN + wn + j * 16 + li] = t;
+    }
+    __syncthreads();
+    for (int c = threadIdx.x; c < BN; c += 256) {
+      float t = 0.f;
+#pragma unroll
+      for (int w = 0; w < WM; ++w) t += csum[w * BN + c];
+      if (n0 + c < N) atomicAdd(out + n0 + c, t);
+    }
+  }
+}
+
 // C[M][N] = op(A)[M][K] * op(B)[K][N], BF16 operands, FP32 accumulation on
-// v_mfma_f32_16x16x16bf16_1k.  A(m,k) = TA ? A[k*lda+m] : A[m*lda+k];
+// v_mfma_f32_16x16x16bf16_1k, for any alignment.  A(m,k) = TA ? A[k*lda+m] : A[m*lda+k];
 // B(k,n) = TB ? B[n*ldb+k] : B[k*ldb+n].  Workgroup: 64x64 tile, 4 waves of
 // 32x32 (2x2 MFMA blocks).  blockIdx.z splits K into gridDim.z ranges (only
 // with EPI_ATOMIC).  Out-of-range rows/cols/ks are zero-filled.
@@ -106,55 +297,65 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(int M, int N, int K, con
         const int row = m0 + wm + i * 16 + 4 * (lane >> 4) + q;
         const int col = n0 + wn + j * 16 + (lane & 15);
         if (row >= M || col >= N) continue;
-        const float v = acc[i][j][q];
-        const int64_t o = (int64_t)row * ldc + col;
-        if (EPI == EPI_BIAS_SILU) {
-          const float z = v + bias[col];
-          out[o] = z;
-          out2[o] = f2bf(silu(z));
-        } else if (EPI == EPI_BIAS) {
-          out[o] = v + bias[col];
-        } else if (EPI == EPI_DSILU) {
-          const float dz = v * dsilu(aux[o]);
-          out[o] = dz;
-          out2[o] = f2bf(dz);
-        } else {
-          atomicAdd(out + o, v);
-        }
+        gemm_store<EPI>(acc[i][j][q], row, col, (int64_t)row * ldc + col, bias, aux, out, out2);
       }
 }
 
 // g = 2 (pred - Y) mask / nvalid on the padded output (ld = 32); BF16 and
-// FP32 copies of g; loss accumulated into *loss (FP64).
-__global__ void mse_grad_kernel(int B, const float* __restrict__ pred, const float* __restrict__ Y,
-                                const float* __restrict__ mask, float inv_n, float* __restrict__ g32,
-                                bf16_t* __restrict__ g16, double* __restrict__ loss) {
+// FP32 copies of g; loss accumulated into *loss (FP64).  At most 512
+// workgroups: the loss is one address, and with an atomic per 256 elements
+// that was the time (27 -> 9 us for 16384 rows).  A thread keeps its column, so
+// db (optional) gets the column sums of g, the output layer's bias gradient.
+__global__ void __launch_bounds__(256) mse_grad_kernel(int64_t n, const float* __restrict__ pred,
+                                                       const float* __restrict__ Y, const float* __restrict__ mask,
+                                                       float inv_n, float* __restrict__ g32, bf16_t* __restrict__ g16,
+                                                       double* __restrict__ loss, float* __restrict__ db) {
   __shared__ double red[4];
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  __shared__ float cred[8][32];
   double l = 0.0;
-  if (i < (int64_t)B * 32) {
+  float cs = 0.f;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const float d = (pred[i] - Y[i]) * mask[i];
-    l = (double)d * d * inv_n;
+    l += (double)d * d * inv_n;
     const float g = 2.0f * d * inv_n;
     g32[i] = g;
     g16[i] = f2bf(g);
+    cs += g;
   }
-  for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = l;
+  l = wave_sum_last(l);
+  if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = l;
+  cred[threadIdx.x >> 5][threadIdx.x & 31] = cs;
   __syncthreads();
   if (threadIdx.x == 0) atomicAdd(loss, red[0] + red[1] + red[2] + red[3]);
+  if (db && threadIdx.x < 32) {
+    float t = 0.f;
+    for (int k = 0; k < 8; ++k) t += cred[k][threadIdx.x];
+    atomicAdd(db + threadIdx.x, t);
+  }
 }
 
-// db[n] = sum_m dZ[m][n]  (one workgroup per column, fixed-order tree)
-__global__ void colsum_kernel(int M, int N, const float* __restrict__ dz, int ld, float* __restrict__ db) {
-  __shared__ float red[4];
-  const int n = blockIdx.x;
+// db[n] = sum_m dZ[m][n], db zeroed first: workgroups of 256 rows x 32 columns
+// (rows in 128-byte pieces) add their sums.
+constexpr int CS_ROWS = 256;
+__global__ void colsum_zero_kernel(int N, float* __restrict__ db) {
+  const int n = blockIdx.x * blockDim.x + threadIdx.x;
+  if (n < N) db[n] = 0.f;
+}
+__global__ void __launch_bounds__(256) colsum_kernel(int M, int N, const float* __restrict__ dz, int ld,
+                                                     float* __restrict__ db) {
+  __shared__ float red[8][32];
+  const int c = threadIdx.x & 31, r = threadIdx.x >> 5, n = blockIdx.x * 32 + c;
+  const int m1 = min(M, (int)(blockIdx.y + 1) * CS_ROWS);
   float s = 0.f;
-  for (int m = threadIdx.x; m < M; m += blockDim.x) s += dz[(int64_t)m * ld + n];
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  if (n < N)
+    for (int m = blockIdx.y * CS_ROWS + r; m < m1; m += 8) s += dz[(int64_t)m * ld + n];
+  red[r][c] = s;
   __syncthreads();
-  if (threadIdx.x == 0) db[n] = red[0] + red[1] + red[2] + red[3];
+  if (threadIdx.x < 32 && n < N) {
+    float t = 0.f;
+    for (int k = 0; k < 8; ++k) t += red[k][c];
+    atomicAdd(db + n, t);
+  }
 }
 
 // Adam on FP32 master weights; BF16 working copy refreshed.
@@ -256,12 +457,47 @@ __global__ void f32_to_bf16_kernel(int64_t n, const float* __restrict__ x, bf16_
   if (i < n) y[i] = f2bf(x[i]);
 }
 
+template <int BM, int BN, int TK, int WM, bool TA, bool TB, int EPI>
+static void launch_tile(int M, int N, int K, const void* A, int lda, const void* B, int ldb, const float* bias,
+                        const float* aux, float* out, void* out2, int ldc, int rows, int ksplit, hipStream_t st) {
+  dim3 grid((N + BN - 1) / BN, rows, ksplit);
+  gemm_tile_kernel<BM, BN, TK, WM, TA, TB, EPI><<<grid, 256, 0, st>>>(M, N, K, (const bf16_t*)A, lda, (const bf16_t*)B,
+                                                                      ldb, bias, aux, out, (bf16_t*)out2, ldc);
+}
+
+// Tiled form where every row starts 16-byte aligned and the rows reach to a
+// multiple of 8 elements (the pieces it loads): 64 x 64 tiles, 64 x 32 for the
+// narrow layer.
 template <bool TA, bool TB, int EPI>
 static int launch_gemm(int M, int N, int K, const void* A, int lda, const void* B, int ldb, const float* bias,
                        const float* aux, float* out, void* out2, int ldc, int ksplit, hipStream_t st) {
-  dim3 grid((N + GBN - 1) / GBN, (M + GBM - 1) / GBM, ksplit);
-  gemm_bf16_kernel<TA, TB, EPI><<<grid, 256, 0, st>>>(M, N, K, (const bf16_t*)A, lda, (const bf16_t*)B, ldb, bias,
-                                                      aux, out, (bf16_t*)out2, ldc);
+  const bool aligned = (((uintptr_t)A | (uintptr_t)B) & 15) == 0 && lda % 8 == 0 && ldb % 8 == 0 &&
+                       ((TA ? M : K) + 7) / 8 * 8 <= lda && ((TB ? K : N) + 7) / 8 * 8 <= ldb;
+  // the grid's y extent is limited to 65535; column sums: few workgroups per
+  // column, each of which adds to the same addresses
+  const int mt = (M + 63) / 64, rows = EPI == EPI_DSILU_SUM ? (mt < 256 ? mt : 256) : (mt < 65535 ? mt : 65535);
+  if (aligned) {
+    if constexpr (EPI == EPI_ATOMIC) {
+      // steps of 128 k: the loop is bound by the latency of its loads.  K
+      // ranges for two workgroups per CU: every range adds all outputs
+      const int tiles = mt * ((N + 63) / 64), want = (512 + tiles - 1) / tiles;
+      const int ks = ksplit < want ? ksplit : want;
+      if (N <= 32)
+        launch_tile<64, 32, 128, 4, TA, TB, EPI>(M, N, K, A, lda, B, ldb, bias, aux, out, out2, ldc, rows, ks, st);
+      else
+        launch_tile<64, 64, 128, 2, TA, TB, EPI>(M, N, K, A, lda, B, ldb, bias, aux, out, out2, ldc, rows, ks, st);
+    } else if (N <= 32) {
+      launch_tile<64, 32, 32, 4, TA, TB, EPI>(M, N, K, A, lda, B, ldb, bias, aux, out, out2, ldc, rows, 1, st);
+    } else {
+      launch_tile<64, 64, 32, 2, TA, TB, EPI>(M, N, K, A, lda, B, ldb, bias, aux, out, out2, ldc, rows, 1, st);
+    }
+  } else if constexpr (EPI == EPI_DSILU_SUM) {
+    PSCF_REQUIRE(false, "pscf_mlp_gemm: op 4 needs 16-byte aligned rows");
+  } else {
+    dim3 grid((N + GBN - 1) / GBN, (M + GBM - 1) / GBM, ksplit);
+    gemm_bf16_kernel<TA, TB, EPI><<<grid, 256, 0, st>>>(M, N, K, (const bf16_t*)A, lda, (const bf16_t*)B, ldb, bias,
+                                                        aux, out, (bf16_t*)out2, ldc);
+  }
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
 }
@@ -274,6 +510,7 @@ using namespace pscf;
 //     1 = forward output (X W + b; out FP32)
 //     2 = backward data (dY W^T, times dsilu(aux = Z of the layer below); out FP32, out2 BF16)
 //     3 = weight gradient (X^T dY accumulated into out with atomics; ksplit > 1 allowed)
+//     4 = as 2, but no FP32 copy: out2 BF16, and out[n] += the column sums (the bias gradient)
 extern "C" int pscf_mlp_gemm(int op, int M, int N, int K, const void* d_A, int lda, const void* d_B, int ldb,
                              const float* d_bias, const float* d_aux, float* d_out, void* d_out2, int ldc, int ksplit,
                              void* stream) {
@@ -294,6 +531,10 @@ extern "C" int pscf_mlp_gemm(int op, int M, int N, int K, const void* d_A, int l
       PSCF_REQUIRE(d_aux && d_out2, "pscf_mlp_gemm: backward needs Z and BF16 output");
       return launch_gemm<false, true, EPI_DSILU>(M, N, K, d_A, lda, d_B, ldb, nullptr, d_aux, d_out, d_out2, ldc, 1,
                                                  st);
+    case 4:
+      PSCF_REQUIRE(d_aux && d_out2, "pscf_mlp_gemm: backward needs Z and BF16 output");
+      return launch_gemm<false, true, EPI_DSILU_SUM>(M, N, K, d_A, lda, d_B, ldb, nullptr, d_aux, d_out, d_out2, ldc,
+                                                     1, st);
     case 3:
       return launch_gemm<true, false, EPI_ATOMIC>(M, N, K, d_A, lda, d_B, ldb, nullptr, nullptr, d_out, nullptr, ldc,
                                                   ksplit, st);
@@ -304,20 +545,28 @@ extern "C" int pscf_mlp_gemm(int op, int M, int N, int K, const void* d_A, int l
   return PSCF_EINVAL;
 }
 
-extern "C" int pscf_mlp_mse_grad(int B, const float* d_pred, const float* d_Y, const float* d_mask, float inv_n,
-                                 float* d_g32, void* d_g16, double* d_loss, void* stream) {
+extern "C" int pscf_mlp_mse_grad_bias(int B, const float* d_pred, const float* d_Y, const float* d_mask, float inv_n,
+                                      float* d_g32, void* d_g16, double* d_loss, float* d_db, void* stream) {
   PSCF_REQUIRE(B >= 0 && d_pred && d_Y && d_mask && d_g32 && d_g16 && d_loss, "pscf_mlp_mse_grad: bad arguments");
   if (B == 0) return PSCF_OK;
-  const int64_t n = (int64_t)B * 32;
-  mse_grad_kernel<<<(unsigned)((n + 255) / 256), 256, 0, (hipStream_t)stream>>>(B, d_pred, d_Y, d_mask, inv_n, d_g32,
-                                                                              (bf16_t*)d_g16, d_loss);
+  const int64_t n = (int64_t)B * 32, blocks = (n + 255) / 256;
+  mse_grad_kernel<<<(unsigned)(blocks < 512 ? blocks : 512), 256, 0, (hipStream_t)stream>>>(
+      n, d_pred, d_Y, d_mask, inv_n, d_g32, (bf16_t*)d_g16, d_loss, d_db);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
 }
 
+extern "C" int pscf_mlp_mse_grad(int B, const float* d_pred, const float* d_Y, const float* d_mask, float inv_n,
+                                 float* d_g32, void* d_g16, double* d_loss, void* stream) {
+  return pscf_mlp_mse_grad_bias(B, d_pred, d_Y, d_mask, inv_n, d_g32, d_g16, d_loss, nullptr, stream);
+}
+
 extern "C" int pscf_mlp_colsum(int M, int N, const float* d_dz, int ld, float* d_db, void* stream) {
   PSCF_REQUIRE(M >= 0 && N > 0 && d_dz && d_db, "pscf_mlp_colsum: bad arguments");
-  colsum_kernel<<<N, 256, 0, (hipStream_t)stream>>>(M, N, d_dz, ld, d_db);
+  colsum_zero_kernel<<<(N + 255) / 256, 256, 0, (hipStream_t)stream>>>(N, d_db);
+  if (M > 0)
+    colsum_kernel<<<dim3((N + 31) / 32, (M + CS_ROWS - 1) / CS_ROWS), 256, 0, (hipStream_t)stream>>>(M, N, d_dz, ld,
+                                                                                                      d_db);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
 }
