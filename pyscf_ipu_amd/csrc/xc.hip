@@ -172,7 +172,6 @@ struct XMTraits;
 template <>
 struct XMTraits<float> {
   typedef float v4 __attribute__((ext_vector_type(4)));
-  static constexpr int TILE = 64;
   static __device__ inline v4 mfma(float a, float b, v4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
   // row of accumulator register j in lane group lg = lane / 16: row(lg, 0) + j * RSTEP
   static __device__ inline int row(int lg, int j) { return 4 * lg + j; }
@@ -181,7 +180,6 @@ struct XMTraits<float> {
 template <>
 struct XMTraits<double> {
   typedef double v4 __attribute__((ext_vector_type(4)));
-  static constexpr int TILE = 32;
   static __device__ inline v4 mfma(double a, double b, v4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
@@ -205,57 +203,8 @@ struct XTile {
   static constexpr size_t lds_elems = (size_t)4 * XT * XS + (size_t)XT * XD + (size_t)NP * XD + 256 + 4 * XT;
 };
 
-// FP32 with 32-point tiles and nao <= 64 keeps GEMM 1's D operand in registers
-// (NJ * NP / 4 values per lane: D does not change between tiles) instead of
-// LDS, which lowers the LDS of a workgroup from 67 KB to 46 KB at NP = 64, so
-// three workgroups share a CU instead of two.  FP64 and wider shapes would need
-// more registers than they have spare and keep D in LDS.
-template <typename T, int XT, int NP>
-struct XDReg {
-  static constexpr bool on = sizeof(T) == 4 && XT == 32 && NP <= 64;
-  static constexpr size_t lds_elems = XTile<XT, NP>::lds_elems - (on ? (size_t)NP * XTile<XT, NP>::XD : 0);
-};
-
 template <typename T, int XT, int NP>
 using XVacc = typename XMTraits<T>::v4[XTile<XT, NP>::NBW];
-
-// Staging of a tile's AO values and gradients into Phi[c][p][mu] (row stride
-// XS), mu < N; padding columns are left as they are.
-// Stored form: read from ao[c * sc + mu * smu + p * sp] in HBM.  Each wave
-// moves one (c, mu) row of XT points per 64 / XT rows and instruction (lanes
-// walk points, coalesced), eight rows' loads in flight before their LDS
-// stores; c = row / N comes from three compares, not a division.
-template <typename T, int XT, int NP>
-struct XcStageStored {
-  const T* ao;
-  int sc, smu, sp, g, N;
-  __device__ inline void load(int) {}
-  __device__ inline void operator()(T* Phi, int p0, int /*p0_next*/) {
-    constexpr int XS = XTile<XT, NP>::XS;
-    constexpr int RPW = 64 / XT;  // rows per wave instruction
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int p = lane % XT, sub = lane / XT, nrow = 4 * N, rstride = 4 * RPW;
-    const int pt = p0 + p;
-    const bool in = pt < g;
-    const int ptoff = pt * sp;
-    for (int base = wave * RPW + sub; base < nrow; base += 8 * rstride) {
-      T v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int row = base + u * rstride;
-        const int c = (row >= N) + (row >= 2 * N) + (row >= 3 * N), mu = row - c * N;
-        v[u] = (row < nrow && in) ? ao[c * sc + mu * smu + ptoff] : T(0);
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int row = base + u * rstride;
-        const int c = (row >= N) + (row >= 2 * N) + (row >= 3 * N), mu = row - c * N;
-        if (row < nrow) Phi[(c * XT + p) * XS + mu] = v[u];
-      }
-    }
-  }
-};
 
 // One molecule's shells in LDS for the direct form, as records: an s shell,
 // a p shell, or an s shell and the p shell after it on the same atom with the
@@ -364,14 +313,74 @@ __device__ inline XcShells<T> xc_build_shells(unsigned char* base, int nsh_max, 
   return t;
 }
 
+template <typename T>
+__device__ inline T xc_exp2n(T x) {
+  if constexpr (sizeof(T) == 4)
+    return __builtin_amdgcn_exp2f(x);
+  else
+    return exp2(x);
+}
+
+// AO values and gradients of shell record r at the point (x, y, z), into
+// Phi[c][p][mu] with XT points per component and row stride XS (the values
+// pscf_batch_ao stores; zeros if not `in`).  Differences to the centres are
+// formed in FP64 and rounded to T; the exponentials are 2^(-a r^2) with
+// a = e log2(e) (one v_exp_f32 in FP32).
+template <typename T, int XT, int XS>
+__device__ inline void xc_eval_record(const XcShells<T>& sh, int r, double x, double y, double z, bool in, T* Phi,
+                                      int p) {
+  const int info = sh.info[r];
+  const int mu = info & 255, kind = (info >> 8) & 15, np = info >> 12;
+  const double* h = sh.hdr + 4 * r;
+  const T dx = (T)(x - h[0]), dy = (T)(y - h[1]), dz = (T)(z - h[2]);
+  const T r2 = dx * dx + dy * dy + dz * dz;
+  // the first three primitive slots are evaluated unconditionally (kp >=
+  // 3, unused slots hold zero coefficients), so their loads issue with the
+  // header's and no lane branches on the primitive count
+  XcPrim<T> q3[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) q3[k] = sh.prim[r * sh.kp + k];
+  T rs = T(0), ds = T(0), rp = T(0), dp = T(0);
+  auto add = [&](const XcPrim<T>& q) {
+    const T ex = xc_exp2n(-q.a * r2);
+    const T te = q.e * ex;
+    rs += q.cs * ex;
+    ds += q.cs * te;
+    rp += q.cp * ex;
+    dp += q.cp * te;
+  };
+  if (in && (double)r2 <= h[3]) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) add(q3[k]);
+    for (int k = 3; k < np; ++k) add(sh.prim[r * sh.kp + k]);
+  }
+  ds *= T(-2);
+  dp *= T(-2);
+  T* qs = Phi + p * XS + mu;
+  if (kind != 1) {
+    qs[0] = rs;
+    qs[XT * XS] = ds * dx;
+    qs[2 * XT * XS] = ds * dy;
+    qs[3 * XT * XS] = ds * dz;
+  }
+  if (kind != 0) {
+    T* qp = qs + (kind == 2 ? 1 : 0);
+    const T d[3] = {dx, dy, dz};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      qp[a] = d[a] * rp;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) qp[(1 + c) * XT * XS + a] = (a == c ? rp : T(0)) + d[a] * d[c] * dp;
+    }
+  }
+}
+
 // Direct form: the AO values and gradients of the tile's points evaluated
-// from the shell records (the values pscf_batch_ao stores).  Thread t takes
+// from the shell records.  Thread t takes
 // point t % XT of the tile (XC_THREADS is a multiple of XT, so a thread keeps
 // its point) and records t / XT, t / XT + XC_THREADS / XT, ...; the point's
 // coordinates for the next tile are loaded at the end of each stage, so their
-// latency hides behind the tile's GEMMs.  Differences to the centres are
-// formed in FP64 and rounded to T; the exponentials are 2^(-a r^2) with
-// a = e log2(e) (one v_exp_f32 in FP32).
+// latency hides behind the tile's GEMMs.
 template <typename T, int XT, int NP>
 struct XcStageDirect {
   XcShells<T> sh;
@@ -385,64 +394,13 @@ struct XcStageDirect {
     py = in ? coords[3 * pt + 1] : 0.0;
     pz = in ? coords[3 * pt + 2] : 0.0;
   }
-  __device__ static inline T exp2n(T x) {
-    if constexpr (sizeof(T) == 4)
-      return __builtin_amdgcn_exp2f(x);
-    else
-      return exp2(x);
-  }
   __device__ inline void operator()(T* Phi, int p0, int p0_next) {
-    constexpr int XS = XTile<XT, NP>::XS;
     const int tid = threadIdx.x, p = tid % XT;
     const bool in = p0 + p < g;
     const double x = px, y = py, z = pz;
     load(p0_next);
-    for (int r = tid / XT; r < sh.nrec; r += XC_THREADS / XT) {
-      const int info = sh.info[r];
-      const int mu = info & 255, kind = (info >> 8) & 15, np = info >> 12;
-      const double* h = sh.hdr + 4 * r;
-      const T dx = (T)(x - h[0]), dy = (T)(y - h[1]), dz = (T)(z - h[2]);
-      const T r2 = dx * dx + dy * dy + dz * dz;
-      // the first three primitive slots are evaluated unconditionally (kp >=
-      // 3, unused slots hold zero coefficients), so their loads issue with the
-      // header's and no lane branches on the primitive count
-      XcPrim<T> q3[3];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) q3[k] = sh.prim[r * sh.kp + k];
-      T rs = T(0), ds = T(0), rp = T(0), dp = T(0);
-      auto add = [&](const XcPrim<T>& q) {
-        const T ex = exp2n(-q.a * r2);
-        const T te = q.e * ex;
-        rs += q.cs * ex;
-        ds += q.cs * te;
-        rp += q.cp * ex;
-        dp += q.cp * te;
-      };
-      if (in && (double)r2 <= h[3]) {
-#pragma unroll
-        for (int k = 0; k < 3; ++k) add(q3[k]);
-        for (int k = 3; k < np; ++k) add(sh.prim[r * sh.kp + k]);
-      }
-      ds *= T(-2);
-      dp *= T(-2);
-      T* qs = Phi + p * XS + mu;
-      if (kind != 1) {
-        qs[0] = rs;
-        qs[XT * XS] = ds * dx;
-        qs[2 * XT * XS] = ds * dy;
-        qs[3 * XT * XS] = ds * dz;
-      }
-      if (kind != 0) {
-        T* qp = qs + (kind == 2 ? 1 : 0);
-        const T d[3] = {dx, dy, dz};
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          qp[a] = d[a] * rp;
-#pragma unroll
-          for (int c = 0; c < 3; ++c) qp[(1 + c) * XT * XS + a] = (a == c ? rp : T(0)) + d[a] * d[c] * dp;
-        }
-      }
-    }
+    for (int r = tid / XT; r < sh.nrec; r += XC_THREADS / XT)
+      xc_eval_record<T, XT, XTile<XT, NP>::XS>(sh, r, x, y, z, in, Phi, p);
   }
 };
 
@@ -454,36 +412,19 @@ __device__ inline void xc_tiles(const XCArgs<T>& a, unsigned char* smem, int til
   constexpr int PB = L::PB, NSLOT = L::NSLOT, NB = L::NB, XS = L::XS, XD = L::XD, NVB = L::NVB, NBW = L::NBW;
   constexpr int RS = XMTraits<T>::RSTEP;
   const int N = a.N;
-  constexpr bool DREG = XDReg<T, XT, NP>::on;
-  constexpr int NK = NP / 4;
   T* Phi = reinterpret_cast<T*>(smem);        // [4][XT][XS]
   T* Y = Phi + 4 * XT * XS;                   // [XT][XD]
-  T* Dm = Y + XT * XD;                        // [NP][XD] (not when DREG)
-  T* rpart = Dm + (DREG ? 0 : NP * XD);       // [NSLOT][4][XT]
+  T* Dm = Y + XT * XD;                        // [NP][XD]
+  T* rpart = Dm + NP * XD;       // [NSLOT][4][XT]
   T* coef = rpart + 256;                      // [4][XT]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lg = lane >> 4;
   const int pb = wave % PB, slot = wave / PB;
-  // GEMM 1's B operand of this lane: D[k0 + lg][column block of jb, li]
-  T dreg[DREG ? L::NJ * NK : 1];
   __syncthreads();
-  if (DREG) {
-#pragma unroll
-    for (int jb = 0; jb < L::NJ; ++jb) {
-      const int cbk = slot + jb * NSLOT < NB ? slot + jb * NSLOT : NB - 1;  // as in GEMM 1
-      const int col = cbk * 16 + li;
-#pragma unroll
-      for (int kk = 0; kk < NK; ++kk) {
-        const int row = kk * 4 + lg;
-        dreg[DREG ? jb * NK + kk : 0] = (row < N && col < N) ? a.dm[row * N + col] : T(0);
-      }
-    }
-  } else {
-    for (int x = tid; x < NP * NP; x += blockDim.x) {
-      const int i = x / NP, j = x - i * NP;
-      Dm[i * XD + j] = (i < N && j < N) ? a.dm[i * N + j] : T(0);
-    }
+  for (int x = tid; x < NP * NP; x += blockDim.x) {
+    const int i = x / NP, j = x - i * NP;
+    Dm[i * XD + j] = (i < N && j < N) ? a.dm[i * N + j] : T(0);
   }
   // padding columns nu in [N, NP) of Phi stay zero for every tile
   for (int x = tid; x < 4 * XT * (NP - N); x += blockDim.x) {
@@ -529,7 +470,7 @@ __device__ inline void xc_tiles(const XCArgs<T>& a, unsigned char* smem, int til
         v4 acc = {T(0), T(0), T(0), T(0)};
 #pragma unroll
         for (int k0 = 0; k0 < NP; k0 += 4)
-          acc = XMTraits<T>::mfma(Phi[a1 + k0], DREG ? dreg[DREG ? jb * NK + k0 / 4 : 0] : Dm[b1 + k0 * XD + cb], acc);
+          acc = XMTraits<T>::mfma(Phi[a1 + k0], Dm[b1 + k0 * XD + cb], acc);
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[j] *= scale;
 #pragma unroll
@@ -642,39 +583,53 @@ __device__ inline double xc_block_energy(double e_loc, double* red) {
   return s;
 }
 
+}  // namespace pscf
+
+#include "xc_wave.h"
+
+namespace pscf {
+
+// Resident workgroups the register budget is set for: two per CU while a
+// wave's D, V and AO values fit 256 registers.
 template <typename T, int NP>
-__global__ void __launch_bounds__(XC_THREADS) xc_fused_kernel(XCArgs<T> a) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int XT = XMTraits<T>::TILE;
+constexpr int xw_min_blocks() {
+  return sizeof(T) == 4 ? (NP <= 64 ? 2 : 1) : (NP <= 16 ? 2 : 1);
+}
+
+// One molecule, stored AO block: tiles blockIdx.x, blockIdx.x + gridDim.x, ...;
+// FP64 adds the workgroup's V + V^T and energy into the zeroed outputs (exact
+// atomics), FP32 leaves V and the energy in part_v and part_e.
+template <typename T, int NP>
+__global__ void __launch_bounds__(XC_THREADS, (xw_min_blocks<T, NP>())) xc_wave_kernel(XCArgs<T> a) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  T* smem = reinterpret_cast<T*>(smem_raw);
+  typedef XW<T, NP, true> L;
+  T dreg[L::ND];
+  typename L::v4 vacc[L::NB * L::NB];
+  XwAO<T, NP> ao;
   double e_loc = 0.0;
-  XVacc<T, XT, NP> vacc;
-  // AO strides as 32-bit element offsets (the host checks that the AO block
-  // is below 2^31 elements)
-  XcStageStored<T, XT, NP> stage{a.ao, (int)a.sc, (int)a.smu, (int)a.sp, a.g, a.N};
-  xc_tiles<T, XT, NP>(a, smem, blockIdx.x, gridDim.x, (a.g + XT - 1) / XT, stage, vacc, e_loc);
-  double* red = reinterpret_cast<double*>(smem);
-  if constexpr (sizeof(T) == 8) {
-    if (a.vout != nullptr) {
-      // this workgroup's V + V^T and energy into the outputs (exact atomics)
-      __syncthreads();
-      const double e = xc_block_energy(e_loc, red);
-      if (threadIdx.x == 0) atomicAdd(a.eout, quant40(e));
-      __syncthreads();
-      T* Vl = reinterpret_cast<T*>(smem);
-      xm_store_v<T, XT, NP>(vacc, a.N, Vl, a.N);
-      __syncthreads();
-      const int NN = a.N * a.N;
-      for (int x = threadIdx.x; x < NN; x += blockDim.x) {
-        const int i = x / a.N, j = x - i * a.N;
-        atomicAdd(a.vout + x, quant40(Vl[x] + Vl[j * a.N + i]));
-      }
-      return;
-    }
-  }
-  xm_store_v<T, XT, NP>(vacc, a.N, a.part_v + (int64_t)blockIdx.x * a.N * a.N, a.N);
+  XwStored<T, NP> stage{a.ao, (int)a.sc, (int)a.smu, (int)a.sp, a.g, a.N};
+  stage.init();
+  const int ntiles = (a.g + 63) / 64, p0 = blockIdx.x * 64 + (int)(threadIdx.x >> 6) * 16;
+  stage.template load<0, 1>(p0, ao.f0);
+  stage.template load<1, 4>(p0, ao.fg);
+  xw_load_d<T, NP, true>(a.dm, a.N, dreg);
+  xw_begin<T, NP, true>(smem, a.dm, a.N, vacc);
+  xw_tiles_stored<T, NP>(a, smem, blockIdx.x, gridDim.x, ntiles, -1, stage, ao, dreg, vacc, e_loc);
+  double* red = reinterpret_cast<double*>(smem + L::MAIN);
   __syncthreads();
   const double e = xc_block_energy(e_loc, red);
-  if (threadIdx.x == 0) a.part_e[blockIdx.x] = e;
+  const int N = a.N;
+  if (a.vout != nullptr) {
+    if (threadIdx.x == 0) atomicAdd(a.eout, quant40(e));
+    xw_flush<T, NP, true>(smem, N, vacc, [&](int i, int j, T v, T vt) {
+      atomicAdd((double*)a.vout + i * N + j, quant40((double)v + vt));
+    });
+  } else {
+    if (threadIdx.x == 0) a.part_e[blockIdx.x] = e;
+    T* dst = a.part_v + (int64_t)blockIdx.x * N * N;
+    xw_flush<T, NP, true>(smem, N, vacc, [&](int i, int j, T v, T) { dst[i * N + j] = v; });
+  }
 }
 
 // Batched: workgroup (blockIdx.x, blockIdx.y) takes molecule order[blockIdx.x]
@@ -714,23 +669,12 @@ __device__ inline bool xc_mol_outside(const BatchMol& Mo, int max_nao, int nsh_m
          (nsh_max > 0 && Mo.nbas > nsh_max);
 }
 
-// FP32 with 32-point tiles: three workgroups per CU up to nao 64 (their LDS
-// fits), two above; the register cap this sets costs a few spilled values
-// outside the GEMM loops and runs faster than fewer resident workgroups.
 template <typename T, int XT, int NP>
-constexpr int xc_batch_min_blocks() {
-  return (sizeof(T) == 4 && XT == 32) ? (NP <= 64 ? 3 : 2) : 1;
-}
-
-template <typename T, int XT, int NP, bool DIRECT>
-__global__ void __launch_bounds__(XC_THREADS, (xc_batch_min_blocks<T, XT, NP>())) xc_batch_kernel(const BatchMol* __restrict__ mols,
-                                                              const int* __restrict__ order, int max_nao,
-                                                              const double* __restrict__ ctl, const T* __restrict__ ao,
-                                                              XcDirect da, const T* __restrict__ dm,
-                                                              const T* __restrict__ w, T eps, T* __restrict__ vxc,
-                                                              double* __restrict__ exc, T* __restrict__ part_v,
-                                                              double* __restrict__ part_e, int64_t part_v_elems,
-                                                              int64_t part_e_elems) {
+__global__ void __launch_bounds__(XC_THREADS) xc_batch_kernel(
+    const BatchMol* __restrict__ mols, const int* __restrict__ order, int max_nao, const double* __restrict__ ctl,
+    const T* __restrict__ /*ao*/, XcDirect da, const T* __restrict__ dm, const T* __restrict__ w, T eps,
+    T* __restrict__ vxc, double* __restrict__ exc, T* __restrict__ part_v, double* __restrict__ part_e,
+    int64_t part_v_elems, int64_t part_e_elems) {
   static_assert(XC_CHUNK_PTS % XT == 0, "a chunk is a whole number of tiles");
   extern __shared__ __align__(16) unsigned char smem[];
   const int m = order[blockIdx.x];
@@ -740,7 +684,7 @@ __global__ void __launch_bounds__(XC_THREADS, (xc_batch_min_blocks<T, XT, NP>())
   const int part = blockIdx.y, nparts = gridDim.y;
   // LDS and tiles were sized for max_nao (and nsh_max shells), offsets are
   // 32-bit: flag a molecule outside those bounds
-  if (xc_mol_outside(Mo, max_nao, DIRECT ? da.nsh_max : 0)) {
+  if (xc_mol_outside(Mo, max_nao, da.nsh_max)) {
     if (part == 0) {
       for (int x = threadIdx.x; x < N * N; x += blockDim.x) vxc[Mo.mat0 + x] = T(NAN);
       if (threadIdx.x == 0) exc[m] = NAN;
@@ -748,14 +692,8 @@ __global__ void __launch_bounds__(XC_THREADS, (xc_batch_min_blocks<T, XT, NP>())
     return;
   }
   XCArgs<T> a;
-  a.vout = nullptr;
-  a.eout = nullptr;
   a.N = N;
   a.g = (int)Mo.ngrid;
-  a.ao = DIRECT ? nullptr : ao + Mo.ao0;
-  a.sc = (int64_t)a.N * a.g;
-  a.smu = a.g;
-  a.sp = 1;
   a.dm = dm + Mo.mat0;
   a.w = w + Mo.grid0;
   a.eps = eps;
@@ -796,22 +734,105 @@ __global__ void __launch_bounds__(XC_THREADS, (xc_batch_min_blocks<T, XT, NP>())
       if (threadIdx.x == 0) part_e[slot] = e;
     }
   };
+  XcStageDirect<T, XT, NP> stage;
+  stage.sh = xc_build_shells<T>(smem + da.tab_off, da.nsh_max, da.kp, (int)Mo.bas0, (int)Mo.nbas, da.atm, da.bas,
+                                da.env);
+  stage.coords = da.coords + 3 * Mo.grid0;
+  stage.g = a.g;
+  run(stage);
+}
+
+// xc_batch_kernel with wave-private tiles: the same chunks and outputs; a
+// chunk's slot holds the lower triangle of its V + V^T, packed.
+template <typename T, int NP, bool DIRECT>
+__global__ void __launch_bounds__(XC_THREADS, (xw_min_blocks<T, NP>())) xc_wave_batch_kernel(
+    const BatchMol* __restrict__ mols, const int* __restrict__ order, int max_nao, const double* __restrict__ ctl,
+    const T* __restrict__ ao, XcDirect da, const T* __restrict__ dm, const T* __restrict__ w, T eps,
+    T* __restrict__ vxc, double* __restrict__ exc, T* __restrict__ part_v, double* __restrict__ part_e,
+    int64_t part_v_elems, int64_t part_e_elems) {
+  typedef XW<T, NP, !DIRECT> L;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  T* smem = reinterpret_cast<T*>(smem_raw);
+  const int m = order[blockIdx.x];
+  if (ctl != nullptr && ctl[m * CTL + 1] == 0.0) return;
+  const BatchMol Mo = mols[m];
+  const int N = (int)Mo.nao, part = blockIdx.y, nparts = gridDim.y;
+  if (xc_mol_outside(Mo, max_nao, DIRECT ? da.nsh_max : 0)) {
+    if (part == 0) {
+      for (int x = threadIdx.x; x < N * N; x += blockDim.x) vxc[Mo.mat0 + x] = T(NAN);
+      if (threadIdx.x == 0) exc[m] = NAN;
+    }
+    return;
+  }
+  XCArgs<T> a;
+  a.N = N;
+  a.g = (int)Mo.ngrid;
+  a.w = w + Mo.grid0;
+  a.eps = eps;
+  const int ntiles = N > 0 ? (a.g + 63) / 64 : 0, nchunk = (a.g + XC_CHUNK_PTS - 1) / XC_CHUNK_PTS;
+  if (nchunk <= 1 ? part != 0
+                  : part >= nchunk || !xc_parts_fit(nchunk, gridDim.x, max_nao, part_v_elems, part_e_elems))
+    return;  // buffers that do not fit are marked by the reduction
+  constexpr int TPC = XC_CHUNK_PTS / 64;  // tiles per chunk
+  const int wp = (int)(threadIdx.x >> 6) * 16, nrun = nchunk > 1 ? nchunk : 1;
+  const T* D = dm + Mo.mat0;
+  double* red = reinterpret_cast<double*>(smem + L::MAIN);
+  T dreg[L::ND];
+  typename L::v4 vacc[L::NB * L::NB];
+  xw_load_d<T, NP, !DIRECT>(D, N, dreg);
+  auto flush = [&](int c, double e_loc) {
+    __syncthreads();
+    const double e = xc_block_energy(e_loc, red);
+    if (nchunk > 1) {
+      const int64_t slot = (int64_t)c * gridDim.x + blockIdx.x;
+      if (threadIdx.x == 0) part_e[slot] = e;
+      T* dst = part_v + slot * max_nao * max_nao;
+      xw_flush<T, NP, !DIRECT>(smem, N, vacc, [&](int i, int j, T v, T vt) {
+        if (j <= i) dst[i * (i + 1) / 2 + j] = v + vt;
+      });
+    } else {
+      if (threadIdx.x == 0) exc[m] = e;
+      T* dst = vxc + Mo.mat0;
+      xw_flush<T, NP, !DIRECT>(smem, N, vacc, [&](int i, int j, T v, T vt) { dst[i * N + j] = v + vt; });
+    }
+  };
   if constexpr (DIRECT) {
-    XcStageDirect<T, XT, NP> stage;
-    stage.sh = xc_build_shells<T>(smem + da.tab_off, da.nsh_max, da.kp, (int)Mo.bas0, (int)Mo.nbas, da.atm, da.bas,
+    XwDirect<T, NP> stage;
+    stage.sh = xc_build_shells<T>(smem_raw + da.tab_off, da.nsh_max, da.kp, (int)Mo.bas0, (int)Mo.nbas, da.atm, da.bas,
                                   da.env);
     stage.coords = da.coords + 3 * Mo.grid0;
     stage.g = a.g;
-    run(stage);
+    for (int c = part; c < nrun; c += nparts) {
+      double e_loc = 0.0;
+      stage.load(c * XC_CHUNK_PTS + wp);
+      xw_begin<T, NP, false>(smem, D, N, vacc);
+      xw_tiles_direct<T, NP>(a, smem, c * TPC, min(ntiles, (c + 1) * TPC), stage, dreg, vacc, e_loc);
+      flush(c, e_loc);
+    }
   } else {
-    XcStageStored<T, XT, NP> stage{a.ao, (int)a.sc, (int)a.smu, (int)a.sp, a.g, a.N};
-    run(stage);
+    XwStored<T, NP> stage{ao + Mo.ao0, N * a.g, a.g, 1, a.g, N};
+    XwAO<T, NP> f;
+    stage.init();
+    if (part * TPC < ntiles) {
+      stage.template load<0, 1>(part * XC_CHUNK_PTS + wp, f.f0);
+      stage.template load<1, 4>(part * XC_CHUNK_PTS + wp, f.fg);
+    }
+    for (int c = part; c < nrun; c += nparts) {
+      double e_loc = 0.0;
+      xw_begin<T, NP, true>(smem, D, N, vacc);
+      xw_tiles_stored<T, NP>(a, smem, c * TPC, 1, min(ntiles, (c + 1) * TPC),
+                             c + nparts < nrun ? (c + nparts) * TPC : -1, stage, f, dreg, vacc, e_loc);
+      flush(c, e_loc);
+    }
   }
 }
 
-// Sums the chunks of xc_batch_kernel in order: V_xc = sum_c (V_c + V_c^T),
-// E_xc = sum_c e_c, one workgroup per active molecule with more than one chunk.
-template <typename T>
+// Sums the chunks in order: E_xc = sum_c e_c and V_xc = sum_c (V_c + V_c^T).
+// PACKED (xc_wave_batch_kernel): the slots hold packed lower triangles of V_c +
+// V_c^T, blockIdx.y takes 256 of their elements.  Else (xc_batch_kernel) they
+// hold V_c, and one workgroup per molecule takes the sum and its transpose
+// through LDS.
+template <typename T, bool PACKED>
 __global__ void __launch_bounds__(256) xc_batch_reduce_kernel(const BatchMol* __restrict__ mols,
                                                               const int* __restrict__ order, int max_nao,
                                                               const double* __restrict__ ctl,
@@ -823,29 +844,52 @@ __global__ void __launch_bounds__(256) xc_batch_reduce_kernel(const BatchMol* __
   if (ctl != nullptr && ctl[m * CTL + 1] == 0.0) return;
   const BatchMol Mo = mols[m];
   const int N = (int)Mo.nao;
-  if (xc_mol_outside(Mo, max_nao, nsh_max)) return;  // flagged by xc_batch_kernel
+  if (xc_mol_outside(Mo, max_nao, nsh_max)) return;  // flagged by the XC kernel
   const int nchunk = (int)((Mo.ngrid + XC_CHUNK_PTS - 1) / XC_CHUNK_PTS);
-  if (nchunk <= 1) return;  // written by xc_batch_kernel
+  if (nchunk <= 1) return;  // written by the XC kernel
   if (!xc_parts_fit(nchunk, gridDim.x, max_nao, part_v_elems, part_e_elems)) {
-    for (int x = threadIdx.x; x < N * N; x += blockDim.x) vxc[Mo.mat0 + x] = T(NAN);
-    if (threadIdx.x == 0) exc[m] = NAN;
+    if (blockIdx.y == 0) {
+      for (int x = threadIdx.x; x < N * N; x += blockDim.x) vxc[Mo.mat0 + x] = T(NAN);
+      if (threadIdx.x == 0) exc[m] = NAN;
+    }
     return;
   }
-  // chunk sums element by element (coalesced), in chunk order, into LDS;
-  // then V + V^T from LDS
-  extern __shared__ __align__(16) unsigned char smem_r[];
-  T* Vs = reinterpret_cast<T*>(smem_r);
-  for (int x = threadIdx.x; x < N * N; x += blockDim.x) {
+  const int64_t cs = (int64_t)gridDim.x * max_nao * max_nao;
+  const T* pv = part_v + (int64_t)blockIdx.x * max_nao * max_nao;
+  // the chunks of one element, added in order; eight loads in flight
+  auto chunk_sum = [&](int x) {
     T v = T(0);
-    for (int c = 0; c < nchunk; ++c) v += part_v[((int64_t)c * gridDim.x + blockIdx.x) * max_nao * max_nao + x];
-    Vs[x] = v;
+    for (int c = 0; c < nchunk; c += 8) {
+      T t[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) t[u] = pv[min(c + u, nchunk - 1) * cs + x];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v += c + u < nchunk ? t[u] : T(0);
+    }
+    return v;
+  };
+  if constexpr (PACKED) {
+    const int x = blockIdx.y * 256 + threadIdx.x;
+    if (x < N * (N + 1) / 2) {
+      int i = (int)((sqrtf(8.0f * x + 1.0f) - 1.0f) * 0.5f);
+      while ((i + 1) * (i + 2) / 2 <= x) ++i;
+      while (i * (i + 1) / 2 > x) --i;
+      const int j = x - i * (i + 1) / 2;
+      const T v = chunk_sum(x);
+      vxc[Mo.mat0 + i * N + j] = v;
+      vxc[Mo.mat0 + j * N + i] = v;
+    }
+  } else {
+    extern __shared__ __align__(16) unsigned char smem_r[];
+    T* Vs = reinterpret_cast<T*>(smem_r);
+    for (int x = threadIdx.x; x < N * N; x += blockDim.x) Vs[x] = chunk_sum(x);
+    __syncthreads();
+    for (int x = threadIdx.x; x < N * N; x += blockDim.x) {
+      const int i = x / N, j = x - i * N;
+      vxc[Mo.mat0 + x] = Vs[x] + Vs[j * N + i];
+    }
   }
-  __syncthreads();
-  for (int x = threadIdx.x; x < N * N; x += blockDim.x) {
-    const int i = x / N, j = x - i * N;
-    vxc[Mo.mat0 + x] = Vs[x] + Vs[j * N + i];
-  }
-  if (threadIdx.x == 0) {
+  if (threadIdx.x == 0 && blockIdx.y == 0) {
     double e = 0.0;
     for (int c = 0; c < nchunk; ++c) e += part_e[(int64_t)c * gridDim.x + blockIdx.x];
     exc[m] = e;
@@ -1130,7 +1174,7 @@ __global__ void __launch_bounds__(256) ao_batch_kernel(const BatchMol* __restric
 
 template <typename T, int XT, int NP>
 static size_t xc_lds(int N) {
-  const size_t main = sizeof(T) * XDReg<T, XT, NP>::lds_elems;
+  const size_t main = sizeof(T) * XTile<XT, NP>::lds_elems;
   const size_t tail = sizeof(T) * (size_t)N * N + 8 * sizeof(double);  // V + energy partials after the tiles
   return (main > tail ? main : tail) + 8 * sizeof(double);
 }
@@ -1156,11 +1200,11 @@ static XcWs xc_ws(size_t es, int N, int g) {
 }
 
 template <typename T, int NP>
-static int xc_fused_launch(const XCArgs<T>& a, int nb, hipStream_t st) {
-  const size_t lds = xc_lds<T, XMTraits<T>::TILE, NP>(a.N);
+static int xc_launch(const XCArgs<T>& a, int nb, hipStream_t st) {
+  const size_t lds = XW<T, NP, true>::lds_bytes;
   PSCF_REQUIRE((int)lds <= xc_max_lds(), "pscf_xc: N=%d needs %zu B LDS", a.N, lds);
-  PSCF_SET_LDS((xc_fused_kernel<T, NP>), lds);
-  xc_fused_kernel<T, NP><<<nb, XC_THREADS, lds, st>>>(a);
+  PSCF_SET_LDS((xc_wave_kernel<T, NP>), lds);
+  xc_wave_kernel<T, NP><<<nb, XC_THREADS, lds, st>>>(a);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
 }
@@ -1196,11 +1240,11 @@ static int xc_impl(const T* ao, int64_t sc, int64_t smu, int64_t sp, int g, int 
   }
   int rc;
   switch (xm_np(N)) {
-    case 16: rc = xc_fused_launch<T, 16>(a, nb, st); break;
-    case 32: rc = xc_fused_launch<T, 32>(a, nb, st); break;
-    case 48: rc = xc_fused_launch<T, 48>(a, nb, st); break;
-    case 64: rc = xc_fused_launch<T, 64>(a, nb, st); break;
-    default: rc = xc_fused_launch<T, 80>(a, nb, st); break;
+    case 16: rc = xc_launch<T, 16>(a, nb, st); break;
+    case 32: rc = xc_launch<T, 32>(a, nb, st); break;
+    case 48: rc = xc_launch<T, 48>(a, nb, st); break;
+    case 64: rc = xc_launch<T, 64>(a, nb, st); break;
+    default: rc = xc_launch<T, 80>(a, nb, st); break;
   }
   if (rc || ATOMIC) return rc;
   return reduce_parts<T, true>(a.part_v, nb, N, (T*)((char*)ws + lay.lvl_off), vxc, a.part_e, exc, st);
@@ -1555,50 +1599,62 @@ extern "C" int pscf_batch_ao(int dtype, const void* d_mols, const int* d_ptmol, 
 
 // LDS of the batched kernel: the tile pipeline (or, after the tiles, V and
 // the energy partials), then in the direct form the shell table.
-template <typename T, int XT, int NP>
-static size_t xc_batch_lds(int max_nao, const XcDirect* da) {
-  const size_t base = (xc_lds<T, XT, NP>(max_nao) + 31) & ~(size_t)31;
-  return da ? base + xc_shell_bytes(da->nsh_max, da->kp, sizeof(T)) : base;
-}
+// Workgroups per molecule at least: as molecules converge, the rest still
+// spread over the CUs (the sums do not depend on the split).  1024 9-heavy
+// molecules, all active: 6.18 ms per XC pass with one each, 5.98 with four.
+constexpr int XW_PARTS = 4;
 
-template <typename T, int XT, int NP>
+// FP64 direct launches above nao 48 keep xc_batch_kernel: four AO components
+// of 64 points and a wave's FP64 D and V do not fit a CU and its registers.
+template <typename T, int NP, bool DIRECT>
 static int batch_xc_launch(const void* d_mols, const int* d_order, int nmol, int max_nao, const double* d_ctl,
                            const void* d_ao, const XcDirect* da, const void* d_dm, const void* d_w, double eps,
                            void* d_vxc, double* d_exc, int split, void* d_part_v, double* d_part_e,
                            int64_t part_v_elems, int64_t part_e_elems, hipStream_t st) {
-  const size_t lds = xc_batch_lds<T, XT, NP>(max_nao, da);
+  constexpr bool WAVE = !(DIRECT && sizeof(T) == 8 && NP > 48);
+  XcDirect a = DIRECT ? *da : XcDirect{};
+  size_t lds;
+  if constexpr (WAVE)
+    lds = XW<T, NP, !DIRECT>::lds_bytes;
+  else
+    lds = (xc_lds<T, 32, NP>(max_nao) + 31) & ~(size_t)31;
+  a.tab_off = (int)lds;
+  if (DIRECT) lds += xc_shell_bytes(a.nsh_max, a.kp, sizeof(T));
   PSCF_REQUIRE((int)lds <= xc_max_lds(), "pscf_batch_xc: nao %d needs %zu B LDS", max_nao, lds);
-  const dim3 grid(nmol, split);
-  if (da) {
-    XcDirect a = *da;
-    a.tab_off = (int)((xc_lds<T, XT, NP>(max_nao) + 31) & ~(size_t)31);
-    PSCF_SET_LDS((xc_batch_kernel<T, XT, NP, true>), lds);
-    xc_batch_kernel<T, XT, NP, true><<<grid, XC_THREADS, lds, st>>>(
-        (const BatchMol*)d_mols, d_order, max_nao, d_ctl, nullptr, a, (const T*)d_dm, (const T*)d_w, (T)eps,
-        (T*)d_vxc, d_exc, (T*)d_part_v, d_part_e, part_v_elems, part_e_elems);
-  } else {
-    PSCF_SET_LDS((xc_batch_kernel<T, XT, NP, false>), lds);
-    xc_batch_kernel<T, XT, NP, false><<<grid, XC_THREADS, lds, st>>>(
-        (const BatchMol*)d_mols, d_order, max_nao, d_ctl, (const T*)d_ao, XcDirect{}, (const T*)d_dm,
-        (const T*)d_w, (T)eps, (T*)d_vxc, d_exc, (T*)d_part_v, d_part_e, part_v_elems, part_e_elems);
-  }
-  PSCF_HIP(hipGetLastError());
-  xc_batch_reduce_kernel<T><<<nmol, 256, sizeof(T) * (size_t)max_nao * max_nao, st>>>(
+  auto run = [&](auto kernel) -> int {
+    PSCF_SET_LDS(kernel, lds);
+    kernel<<<dim3(nmol, WAVE && split < XW_PARTS ? XW_PARTS : split), XC_THREADS, lds, st>>>((const BatchMol*)d_mols, d_order, max_nao, d_ctl,
+                                                       (const T*)d_ao, a, (const T*)d_dm, (const T*)d_w, (T)eps,
+                                                       (T*)d_vxc, d_exc, (T*)d_part_v, d_part_e, part_v_elems,
+                                                       part_e_elems);
+    PSCF_HIP(hipGetLastError());
+    return PSCF_OK;
+  };
+  int rc;
+  if constexpr (WAVE)
+    rc = run(xc_wave_batch_kernel<T, NP, DIRECT>);
+  else
+    rc = run(xc_batch_kernel<T, 32, NP>);
+  if (rc) return rc;
+  const dim3 rgrid(nmol, WAVE ? (max_nao * (max_nao + 1) / 2 + 255) / 256 : 1);
+  xc_batch_reduce_kernel<T, WAVE><<<rgrid, 256, WAVE ? 0 : sizeof(T) * (size_t)max_nao * max_nao, st>>>(
       (const BatchMol*)d_mols, d_order, max_nao, d_ctl, (const T*)d_part_v, d_part_e, part_v_elems, part_e_elems,
-      (T*)d_vxc, d_exc, da ? da->nsh_max : 0);
+      (T*)d_vxc, d_exc, DIRECT ? a.nsh_max : 0);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
 }
 
-template <typename T, int XT>
+template <typename T>
 static int batch_xc_np(int np, const void* d_mols, const int* d_order, int nmol, int max_nao, const double* d_ctl,
                        const void* d_ao, const XcDirect* da, const void* d_dm, const void* d_w, double eps,
                        void* d_vxc, double* d_exc, int split, void* d_part_v, double* d_part_e, int64_t pv,
                        int64_t pe, hipStream_t st) {
-#define PSCF_XC_NP(V)                                                                                           \
-  case V:                                                                                                       \
-    return batch_xc_launch<T, XT, V>(d_mols, d_order, nmol, max_nao, d_ctl, d_ao, da, d_dm, d_w, eps, d_vxc,  \
-                                     d_exc, split, d_part_v, d_part_e, pv, pe, st);
+#define PSCF_XC_NP(V)                                                                                              \
+  case V:                                                                                                          \
+    return da ? batch_xc_launch<T, V, true>(d_mols, d_order, nmol, max_nao, d_ctl, d_ao, da, d_dm, d_w, eps,       \
+                                            d_vxc, d_exc, split, d_part_v, d_part_e, pv, pe, st)                   \
+              : batch_xc_launch<T, V, false>(d_mols, d_order, nmol, max_nao, d_ctl, d_ao, da, d_dm, d_w, eps,      \
+                                             d_vxc, d_exc, split, d_part_v, d_part_e, pv, pe, st);
   switch (np) {
     PSCF_XC_NP(16)
     PSCF_XC_NP(32)
@@ -1624,14 +1680,11 @@ static int batch_xc_any(int dtype, const void* d_mols, const int* d_order, int n
   PSCF_REQUIRE(max_nao <= XM_MAXN, "pscf_batch_xc: nao %d too large", max_nao);
   hipStream_t st = (hipStream_t)stream;
   const int np = xm_np(max_nao);
-  if (dtype == PSCF_F64)
-    return batch_xc_np<double, 32>(np, d_mols, d_order, nmol, max_nao, d_ctl, d_ao, da, d_dm, d_w, eps, d_vxc,
-                                   d_exc, split, d_part_v, d_part_e, part_v_elems, part_e_elems, st);
-  if (tile == 64)
-    return batch_xc_np<float, 64>(np, d_mols, d_order, nmol, max_nao, d_ctl, d_ao, da, d_dm, d_w, eps, d_vxc,
-                                  d_exc, split, d_part_v, d_part_e, part_v_elems, part_e_elems, st);
-  return batch_xc_np<float, 32>(np, d_mols, d_order, nmol, max_nao, d_ctl, d_ao, da, d_dm, d_w, eps, d_vxc, d_exc,
-                                split, d_part_v, d_part_e, part_v_elems, part_e_elems, st);
+  // the tile (32 or 64 points) is a choice of older kernels: the wave-private
+  // tiles have one shape
+  return (dtype == PSCF_F64 ? batch_xc_np<double> : batch_xc_np<float>)(
+      np, d_mols, d_order, nmol, max_nao, d_ctl, d_ao, da, d_dm, d_w, eps, d_vxc, d_exc, split, d_part_v, d_part_e,
+      part_v_elems, part_e_elems, st);
 }
 
 extern "C" int pscf_batch_xc(int dtype, const void* d_mols, const int* d_order, int nmol, int max_nao,
