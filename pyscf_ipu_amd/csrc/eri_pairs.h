@@ -149,7 +149,8 @@ __device__ inline void ep_stage_table(double* tab, const double* __restrict__ g)
   for (int i = threadIdx.x; i < BOYSD_NT; i += EP_THREADS) {
     const double* s = g + 2 * i * BOYS_NM + L;  // every second node of the 0.1 grid
 #pragma unroll
-    for (int k = 0; k <= BOYSD_TERMS; ++k) tab[i * BOYSD_COLS + k] = s[k] * INV_FACT[k];
+    for (int k = 0; k <= BOYSD_TERMS; ++k)  // (order 5: a term less, still below 1e-19)
+      tab[i * BOYSD_COLS + k] = L + k < BOYS_NM ? s[L + k < BOYS_NM ? k : 0] * INV_FACT[k] : 0.0;
     if constexpr (L > 0) tab[i * BOYSD_COLS + BOYSD_TERMS + 1] = exp(-(double)i * BOYSD_H);
   }
 }
@@ -162,20 +163,20 @@ __host__ __device__ constexpr int hidx(int t, int u, int v) {
 }
 __host__ __device__ constexpr int hcount(int L) { return (L + 1) * (L + 2) * (L + 3) / 6; }
 struct HermiteTable {
-  int up[20][3];             // index raised once along each axis (orders 0-3)
-  int axis[35];              // an axis of the highest power
-  int lo1[35], lo2[35];      // lowered once and twice along it
-  int pow[35];               // the power after lowering once
+  int up[35][3];             // index raised once along each axis (orders 0-4)
+  int axis[56];              // an axis of the highest power
+  int lo1[56], lo2[56];      // lowered once and twice along it
+  int pow[56];               // the power after lowering once
 };
 constexpr HermiteTable make_hermite_table() {
   HermiteTable h{};
-  for (int s = 0; s <= 4; ++s)
+  for (int s = 0; s <= 5; ++s)
     for (int w = 0; w <= s; ++w)
       for (int v = 0; v <= w; ++v) {
         const int t[3] = {s - w, w - v, v};
         const int k = hidx(t[0], t[1], t[2]);
         for (int d = 0; d < 3; ++d)
-          if (s < 4) h.up[k][d] = hidx(t[0] + (d == 0), t[1] + (d == 1), t[2] + (d == 2));
+          if (s < 5) h.up[k][d] = hidx(t[0] + (d == 0), t[1] + (d == 1), t[2] + (d == 2));
         if (s == 0) continue;
         const int d = t[0] >= t[1] && t[0] >= t[2] ? 0 : (t[1] >= t[2] ? 1 : 2);
         h.axis[k] = d;
@@ -381,9 +382,9 @@ __device__ inline void ep_stage(const EpMol& M, int first, int s, int f, int e, 
 
 // Cuts the staged ket primitives into chunks of at most 64 lanes holding whole
 // shell pairs (a pair with more takes several chunks).  One wave calls it.
-template <typename T, int X, int Y>
-__device__ inline void ep_chunks(EpShared<T, X, Y>& sh, int lane) {
-  const EpSide<T, Y>& K = sh.ket;
+template <class Shared>
+__device__ inline void ep_chunks(Shared& sh, int lane) {
+  const auto& K = sh.ket;
   const int n = K.n, end = lane < n ? K.cs[lane + 1] : 0x7fffffff;
   int t = 0, pos = 0, c = 0, split = 0;
   while (t < n) {
