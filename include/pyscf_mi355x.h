@@ -384,8 +384,8 @@ int pscf_cast_to(int out_type, const double* d_x, void* d_y, int64_t n, void* st
  * AO-grid GEMMs X = D phi0 and V = phi0 Y^T, AO values phi [4][N][g] stored as
  * ao_type:  stage 0: rho_c = sum_nu X phi_c, B3LYP (b3lyp.py:13-39), E_xc
  * block partials (pscf_xc_large_parts(g) of them), coefficients coef [4][g];
- * stage 1: Y = sum_c coef_c phi_c (ao_type).  finish: V_xc = Vh + Vh^T and
- * E_xc from the partials. */
+ * stage 1: Y = sum_c coef_c phi_c (ao_type).  stage 2: both, reading phi once.
+ * finish: V_xc = Vh + Vh^T and E_xc from the partials. */
 int pscf_xc_large_parts(int g);
 int pscf_xc_large_stage(int stage, int ao_type, int N, int g, const double* d_X, const void* d_phi, const double* d_w,
                         double eps, double* d_coef, double* d_e_part, void* d_Y, void* stream);

@@ -4,10 +4,9 @@
 // (pyscf_ipu/electron_repulsion/int2e_sph.cpp: CINTg0_2e :1785-1900, 2D
 // recurrence CINTg0_2e_2d :1475-1600, primitive loop CINT2e_loop_nopt
 // :2452-2723, one shell quartet per IPU tile).  The packed s8 arrays come from
-// the shell-pair engine of eri_pairs.h.  The same quadrature as libcint's, one
-// contracted shell quartet per lane, serves explicit quartet lists
-// (pscf_eri_quartets), batches given by quartet work lists
-// (pscf_batch_eri_s8, pscf_batch_eri_s8_div) and the gradient:
+// the shell-pair engine of eri_pairs.h, the gradient from eri_grad.h.  The same
+// quadrature as libcint's, one contracted shell quartet per lane, serves
+// explicit quartet lists (pscf_eri_quartets):
 //   * Boys F_m(T) from a Taylor table staged in LDS (F_0..F_14 on a 0.1 grid
 //     up to T = 39.9, asymptote above),
 //   * Rys roots/weights from the Boys moments in closed form (1-3 roots), FP64,

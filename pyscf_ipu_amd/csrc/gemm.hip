@@ -50,6 +50,10 @@ struct GIn<G_F64> {
 constexpr int QM = 64, QN = 64, QK = 16;
 
 // ACC64: accumulate in FP64; otherwise FP32 with the type's own MFMA.
+// A K chunk's 8 loads per thread are issued one chunk ahead and two LDS buffers
+// take turns, so a chunk costs one barrier and its loads run behind the last
+// chunk's MFMAs (FP64, nao 161 x 90k points: X = D phi0 213 -> 155 us, and V =
+// phi0 Y^T, also split over four times as many workgroups, 467 -> 161 us).
 template <int TY, bool ACC64, bool TA, bool TB, bool ATOMIC>
 __global__ void __launch_bounds__(256) gemm_kernel(int M, int N, int K, const typename GIn<TY>::t* __restrict__ A,
                                                    int64_t lda, const typename GIn<TY>::t* __restrict__ B, int64_t ldb,
@@ -58,8 +62,8 @@ __global__ void __launch_bounds__(256) gemm_kernel(int M, int N, int K, const ty
   // staged tiles, already widened to the compute type of the MFMA inputs
   typedef typename std::conditional<ACC64, double, typename std::conditional<TY == G_F64, double, float>::type>::type
       Tst;
-  __shared__ Tst As[QM][QK + 1];
-  __shared__ Tst Bs[QK][QN + 1];
+  __shared__ Tst As[2][QM][QK + 1];
+  __shared__ Tst Bs[2][QK][QN + 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
   const int m0 = blockIdx.y * QM, n0 = blockIdx.x * QN;
@@ -74,22 +78,46 @@ __global__ void __launch_bounds__(256) gemm_kernel(int M, int N, int K, const ty
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) acc[i][j][q] = 0;
-  for (int k0 = kbeg; k0 < kend; k0 += QK) {
+  // element r of this thread in the A and B tiles; consecutive lanes walk the
+  // operand's contiguous index
+  auto a_at = [&](int r, int& m, int& k) {
+    const int e = tid + r * 256;
+    m = TA ? e % QM : e / QK;
+    k = TA ? e / QM : e % QK;
+  };
+  auto b_at = [&](int r, int& k, int& n) {
+    const int e = tid + r * 256;
+    k = TB ? e % QK : e / QN;
+    n = TB ? e / QK : e % QN;
+  };
+  Tin ra[4], rb[4];
+  auto load = [&](int k0) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int e = tid + r * 256;
-      const int am = e / QK, ak = e % QK;
-      const int gm = m0 + am, gk = k0 + ak;
-      Tst va = 0;
-      if (gm < M && gk < kend) va = (Tst)GIn<TY>::f(TA ? A[(int64_t)gk * lda + gm] : A[(int64_t)gm * lda + gk]);
-      As[am][ak] = va;
-      const int bk = e / QN, bn = e % QN;
-      const int gk2 = k0 + bk, gn = n0 + bn;
-      Tst vb = 0;
-      if (gn < N && gk2 < kend) vb = (Tst)GIn<TY>::f(TB ? B[(int64_t)gn * ldb + gk2] : B[(int64_t)gk2 * ldb + gn]);
-      Bs[bk][bn] = vb;
+      int m, k, n;
+      a_at(r, m, k);
+      const int gm = m0 + m, gk = k0 + k;
+      ra[r] = gm < M && gk < kend ? (TA ? A[(int64_t)gk * lda + gm] : A[(int64_t)gm * lda + gk]) : Tin(0);
+      b_at(r, k, n);
+      const int gn = n0 + n, gk2 = k0 + k;
+      rb[r] = gn < N && gk2 < kend ? (TB ? B[(int64_t)gn * ldb + gk2] : B[(int64_t)gk2 * ldb + gn]) : Tin(0);
     }
+  };
+  if (kbeg < kend) load(kbeg);
+  int buf = 0;
+  for (int k0 = kbeg; k0 < kend; k0 += QK, buf ^= 1) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      int m, k, n;
+      a_at(r, m, k);
+      As[buf][m][k] = (Tst)GIn<TY>::f(ra[r]);
+      b_at(r, k, n);
+      Bs[buf][k][n] = (Tst)GIn<TY>::f(rb[r]);
+    }
+    // a wave writes this buffer again two chunks on, after the next barrier,
+    // which every wave reaches only past its reads of this chunk
     __syncthreads();
+    if (k0 + QK < kend) load(k0 + QK);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -98,32 +126,31 @@ __global__ void __launch_bounds__(256) gemm_kernel(int M, int N, int K, const ty
         if constexpr (ACC64) {
 #pragma unroll
           for (int kk = 0; kk < QK; kk += 4)
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)As[rm][kk + lg], (double)Bs[kk + lg][cn],
+            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)As[buf][rm][kk + lg], (double)Bs[buf][kk + lg][cn],
                                                              acc[i][j], 0, 0, 0);
         } else if constexpr (TY == G_F32 || TY == G_F64) {
 #pragma unroll
           for (int kk = 0; kk < QK; kk += 4)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)As[rm][kk + lg], (float)Bs[kk + lg][cn], acc[i][j],
-                                                             0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32((float)As[buf][rm][kk + lg], (float)Bs[buf][kk + lg][cn],
+                                                             acc[i][j], 0, 0, 0);
         } else if constexpr (TY == G_BF16) {
           gs16x4 a, b;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            a[q] = (short)(__float_as_uint((float)As[rm][4 * lg + q]) >> 16);
-            b[q] = (short)(__float_as_uint((float)Bs[4 * lg + q][cn]) >> 16);
+            a[q] = (short)(__float_as_uint((float)As[buf][rm][4 * lg + q]) >> 16);
+            b[q] = (short)(__float_as_uint((float)Bs[buf][4 * lg + q][cn]) >> 16);
           }
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[i][j], 0, 0, 0);
         } else {
           gh16x4 a, b;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            a[q] = (_Float16)(float)As[rm][4 * lg + q];
-            b[q] = (_Float16)(float)Bs[4 * lg + q][cn];
+            a[q] = (_Float16)(float)As[buf][rm][4 * lg + q];
+            b[q] = (_Float16)(float)Bs[buf][4 * lg + q][cn];
           }
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, acc[i][j], 0, 0, 0);
         }
       }
-    __syncthreads();
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i)

@@ -125,6 +125,9 @@ __global__ void __launch_bounds__(256) jk_s1_kernel(int N, const T* __restrict__
   for (int r = tid; r < N; r += blockDim.x) out[(int64_t)p * N + r] = jacc[r] - hhalf * kacc[r];
 }
 
+// Points per energy part and per tile of xc_rho_y_large_kernel.
+constexpr int XL_PTS = 16;
+
 // Per point p: rho_c = sum_nu X[nu][p] phi_c[nu][p] (c = 0: rho, 1..3: grad/2),
 // B3LYP, E_xc partial sums per block, and the V_xc coefficients
 // coef = (v_rho w / 2, 4 v_sigma w rho_x, .., ..).  phi: [4][N][g] in type TY.
@@ -158,7 +161,10 @@ __global__ void __launch_bounds__(256) xc_rho_large_kernel(int N, int g, const d
   el = l_wave_sum(el);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = el;
   __syncthreads();
-  if (threadIdx.x == 0) e_part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+  // one energy part per XL_PTS points; this block's sum is in its first
+  const int part = blockIdx.x * (256 / XL_PTS) + (int)threadIdx.x;
+  if (threadIdx.x < 256 / XL_PTS && part < (g + XL_PTS - 1) / XL_PTS)
+    e_part[part] = threadIdx.x == 0 ? red[0] + red[1] + red[2] + red[3] : 0.0;
 }
 
 template <int TY>
@@ -177,7 +183,99 @@ __global__ void __launch_bounds__(256) xc_y_large_kernel(int N, int g, const dou
   }
 }
 
-// E_xc = sum of the block partials (Neumaier) and V_xc = Vh + Vh^T.
+// Both stages of XL_PTS points: a thread's phi values (point t % 16, rows
+// nu = t / 16 + 16 u, u < NU) stay in its registers between them, so phi is read
+// once: HBM-bound at 6 N g elements where the two kernels move 10 (nao 161 x 90k
+// points, FP64: 241 us as two, 131 now; 204 with the tile in LDS, a workgroup per
+// CU).  Waves 0-2 take a part of the functional each.
+template <int TY, int NU>
+__global__ void __launch_bounds__(256, 2) xc_rho_y_large_kernel(int N, int g, const double* __restrict__ X,
+                                                                const typename LT<TY>::t* __restrict__ phi,
+                                                                const double* __restrict__ w, double eps,
+                                                                double* __restrict__ coef,
+                                                                double* __restrict__ e_part,
+                                                                typename LT<TY>::t* __restrict__ Y) {
+  typedef typename LT<TY>::t T;
+  __shared__ double rho[4][4][XL_PTS], fn[3][3][XL_PTS], cf[4][XL_PTS];
+  const int tid = threadIdx.x, l = tid & 15, grp = tid >> 4, p = blockIdx.x * XL_PTS + l;
+  const bool in = p < g;
+  const int64_t sc = (int64_t)N * g, pc = in ? p : g - 1;  // points past the end repeat the last, unused
+  T v[NU][4];
+  double r[4] = {0.0, 0.0, 0.0, 0.0};
+  {
+    double x[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int nu = grp + 16 * u;
+      const int64_t o = (int64_t)(nu < N ? nu : N - 1) * g + pc;
+      x[u] = X[o];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[u][c] = phi[c * sc + o];
+    }
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+      if (grp + 16 * u < N)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) r[c] += x[u] * LT<TY>::from(v[u][c]);
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    r[c] += __shfl_xor(r[c], 16, 64);
+    r[c] += __shfl_xor(r[c], 32, 64);
+    if ((tid & 63) < XL_PTS) rho[tid >> 6][c][l] = r[c];
+  }
+  __syncthreads();
+  if (tid < 64) {  // sums over the four waves, in order
+    double t = 0.0;
+    for (int k = 0; k < 4; ++k) t += rho[k][grp][l];
+    rho[0][grp][l] = t;  // only this thread reads and writes rho[0][grp][l]
+  }
+  __syncthreads();
+  const int wave = tid >> 6;
+  if (wave < 3 && (tid & 63) < XL_PTS) {
+    double rr, gam, e = 0.0, vr = 0.0, vn = 0.0;
+    b3lyp_inputs<double>(rho[0][0][l], rho[0][1][l], rho[0][2][l], rho[0][3][l], eps, rr, gam);
+    if (wave == 0)
+      b3lyp_part<double, 0>(rr, gam, e, vr, vn);
+    else if (wave == 1)
+      b3lyp_part<double, 1>(rr, gam, e, vr, vn);
+    else
+      b3lyp_part<double, 2>(rr, gam, e, vr, vn);
+    fn[wave][0][l] = e;
+    fn[wave][1][l] = vr;
+    fn[wave][2][l] = vn;
+  }
+  __syncthreads();
+  if (tid < 64) {  // lanes 0-15 hold the points; the others only join the energy's sum
+    double el = 0.0;
+    if (tid < XL_PTS) {
+      const double e = fn[0][0][l] + fn[1][0][l] + fn[2][0][l], vr = fn[0][1][l] + fn[1][1][l] + fn[2][1][l],
+                   vn = fn[0][2][l] + fn[1][2][l] + fn[2][2][l], wt = in ? w[p] : 0.0, q = 4.0 * vn * wt;
+      if (in) el = rho[0][0][l] * wt * e;
+      cf[0][l] = 0.5 * vr * wt;
+#pragma unroll
+      for (int c = 1; c < 4; ++c) cf[c][l] = q * rho[0][c][l];
+      if (in)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) coef[c * (int64_t)g + p] = cf[c][l];
+    }
+    el = l_wave_sum(el);
+    if (tid == 0) e_part[blockIdx.x] = el;
+  }
+  __syncthreads();
+  if (!in) return;
+  const double c0 = cf[0][l], c1 = cf[1][l], c2 = cf[2][l], c3 = cf[3][l];
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    const int nu = grp + 16 * u;
+    if (nu < N)
+      Y[(int64_t)nu * g + p] = LT<TY>::to(c0 * LT<TY>::from(v[u][0]) + c1 * LT<TY>::from(v[u][1]) +
+                                          c2 * LT<TY>::from(v[u][2]) + c3 * LT<TY>::from(v[u][3]));
+  }
+}
+
+// E_xc = sum of the energy parts (Neumaier per thread, then a fixed tree) and
+// V_xc = Vh + Vh^T.
 __global__ void __launch_bounds__(256) xc_finish_large_kernel(int N, const double* __restrict__ Vh,
                                                               const double* __restrict__ e_part, int nparts,
                                                               double* __restrict__ vxc, double* __restrict__ exc) {
@@ -185,14 +283,20 @@ __global__ void __launch_bounds__(256) xc_finish_large_kernel(int N, const doubl
     const int i = x / N, j = x - i * N;
     vxc[x] = Vh[x] + Vh[j * N + i];
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  if (blockIdx.x == 0) {
+    __shared__ double red[256];
     double s = 0.0, c = 0.0;
-    for (int k = 0; k < nparts; ++k) {
+    for (int k = threadIdx.x; k < nparts; k += 256) {
       const double a = e_part[k], t = s + a;
       c += fabs(s) >= fabs(a) ? (s - t) + a : (a - t) + s;
       s = t;
     }
-    *exc = s + c;
+    red[threadIdx.x] = s + c;
+    for (int n = 128; n > 0; n >>= 1) {
+      __syncthreads();
+      if ((int)threadIdx.x < n) red[threadIdx.x] += red[threadIdx.x + n];
+    }
+    if (threadIdx.x == 0) *exc = red[0];
   }
 }
 
@@ -209,9 +313,21 @@ static int xc_large_launch(int stage, int N, int g, const double* X, const void*
                            double* coef, double* e_part, void* Y, hipStream_t st) {
   typedef typename LT<TY>::t T;
   const unsigned blocks = (unsigned)((g + 255) / 256);
-  if (stage == 0)
-    xc_rho_large_kernel<TY><<<blocks, 256, 0, st>>>(N, g, X, (const T*)phi, w, eps, coef, e_part);
-  else
+  if (stage == 2 && N <= 256) {  // above, a thread's values do not fit its registers
+    auto run = [&](auto kernel) {
+      kernel<<<(g + XL_PTS - 1) / XL_PTS, 256, 0, st>>>(N, g, X, (const T*)phi, w, eps, coef, e_part, (T*)Y);
+    };
+    if (N <= 128)
+      run(xc_rho_y_large_kernel<TY, 8>);
+    else if (N <= 176)
+      run(xc_rho_y_large_kernel<TY, 11>);
+    else
+      run(xc_rho_y_large_kernel<TY, 16>);
+    PSCF_HIP(hipGetLastError());
+    return PSCF_OK;
+  }
+  if (stage != 1) xc_rho_large_kernel<TY><<<blocks, 256, 0, st>>>(N, g, X, (const T*)phi, w, eps, coef, e_part);
+  if (stage != 0)
     xc_y_large_kernel<TY><<<blocks, 256, 0, st>>>(N, g, coef, (const T*)phi, (T*)Y);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
@@ -269,12 +385,12 @@ extern "C" int pscf_jk_s1(int dtype, const void* d_s1, int N, const double* d_dm
   return PSCF_OK;
 }
 
-extern "C" int pscf_xc_large_parts(int g) { return (g + 255) / 256; }
+extern "C" int pscf_xc_large_parts(int g) { return (g + XL_PTS - 1) / XL_PTS; }
 
 extern "C" int pscf_xc_large_stage(int stage, int ao_type, int N, int g, const double* d_X, const void* d_phi,
                                    const double* d_w, double eps, double* d_coef, double* d_e_part, void* d_Y,
                                    void* stream) {
-  PSCF_REQUIRE(stage == 0 || stage == 1, "pscf_xc_large_stage: bad stage");
+  PSCF_REQUIRE(stage >= 0 && stage <= 2, "pscf_xc_large_stage: bad stage");
   PSCF_REQUIRE(N > 0 && g > 0 && d_phi && d_coef, "pscf_xc_large_stage: bad arguments");
   PSCF_REQUIRE(stage == 1 || (d_X && d_w && d_e_part), "pscf_xc_large_stage: stage 0 needs X, w, e_part");
   PSCF_REQUIRE(stage == 0 || d_Y, "pscf_xc_large_stage: stage 1 needs Y");

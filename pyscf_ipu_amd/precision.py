@@ -132,13 +132,11 @@ class LargeRKS(RKS):
         # X[nu][p] = sum_mu D[nu][mu] phi0[mu][p]
         _lib.call("pscf_gemm", self.gemm_type, self.acc64, 0, 0, 0, N, G, N, P(self.Dg), N, P(self.phi), G,
                   P(self.X), G, 1, st)
-        _lib.call("pscf_xc_large_stage", 0, self.gemm_type, N, G, P(self.X), P(self.phi), P(self.weights64),
-                  EPSILON_B3LYP, P(self.coef), P(self.e_part), None, st)
-        _lib.call("pscf_xc_large_stage", 1, self.gemm_type, N, G, None, P(self.phi), None, EPSILON_B3LYP,
-                  P(self.coef), None, P(self.Y), st)
+        _lib.call("pscf_xc_large_stage", 2, self.gemm_type, N, G, P(self.X), P(self.phi), P(self.weights64),
+                  EPSILON_B3LYP, P(self.coef), P(self.e_part), P(self.Y), st)
         # Vh[mu][nu] = sum_p phi0[mu][p] Y[nu][p], K = G split over workgroups
         self.Vh.zero_()
-        ksplit = max(1, min(256, G // 2048))
+        ksplit = max(1, min(256, G // 512))
         _lib.call("pscf_gemm", self.gemm_type, self.acc64, 0, 1, 1, N, N, G, P(self.phi), G, P(self.Y), G,
                   P(self.Vh), N, ksplit, st)
         _lib.call("pscf_xc_large_finish", N, P(self.Vh), P(self.e_part), self.nparts, P(self.Vxc), P(self.exc), st)
