@@ -25,62 +25,6 @@ static int max_lds_bytes() { return device_max_lds(); }
 constexpr int JK_THREADS = 256;
 constexpr int JK_MAX_BLOCKS = 240;
 
-// ------------------------------------------------------------- sparse form ---
-template <typename T, bool LDS>
-__global__ void __launch_bounds__(JK_THREADS) jk_sparse_kernel(const T* __restrict__ eri,
-                                                               const int16_t* __restrict__ idx, int64_t nnz,
-                                                               const T* __restrict__ dm_g, int N, T kscale,
-                                                               T* __restrict__ part) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int NN = N * N;
-  const T* dm = dm_g;
-  T* acc = part;  // global-atomic mode accumulates into out directly
-  if constexpr (LDS) {
-    T* sdm = reinterpret_cast<T*>(smem);
-    acc = sdm + NN;
-    for (int x = threadIdx.x; x < NN; x += blockDim.x) {
-      sdm[x] = dm_g[x];
-      acc[x] = T(0);
-    }
-    __syncthreads();
-    dm = sdm;
-  }
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < nnz; e += stride) {
-    const uint2 packed = reinterpret_cast<const uint2*>(idx)[e];
-    const int i = (int)(packed.x & 0xffffu), j = (int)(packed.x >> 16);
-    const int k = (int)(packed.y & 0xffffu), l = (int)(packed.y >> 16);
-    // out-of-range indices are dropped, like the reference's FILL_OR_DROP gather/scatter
-    if (i >= N || j >= N || k >= N || l >= N) continue;
-    const T v = eri[e];
-    const int ij = i * N + j, ji = j * N + i, kl = k * N + l, lk = l * N + k;
-    // J: patterns 0-7 gather {ij, ji, kl, lk}, scatter {kl, lk, ij, ji}
-    const T tj1 = v * (dm[ij] + dm[ji]);
-    const T tj2 = v * (dm[kl] + dm[lk]);
-    atomicAdd(acc + kl, tj1);
-    atomicAdd(acc + lk, tj1);
-    atomicAdd(acc + ij, tj2);
-    atomicAdd(acc + ji, tj2);
-    // K: patterns 16-23 gather / 24-31 scatter, scaled by -hyb/2
-    const T vk = v * kscale;
-    const int il = i * N + l, jl = j * N + l, ik = i * N + k, jk = j * N + k;
-    const int kj = k * N + j, lj = l * N + j, ki = k * N + i, li = l * N + i;
-    atomicAdd(acc + il, vk * dm[kj]);
-    atomicAdd(acc + jl, vk * dm[ki]);
-    atomicAdd(acc + ik, vk * dm[lj]);
-    atomicAdd(acc + jk, vk * dm[li]);
-    atomicAdd(acc + kj, vk * dm[il]);
-    atomicAdd(acc + lj, vk * dm[ik]);
-    atomicAdd(acc + ki, vk * dm[jl]);
-    atomicAdd(acc + li, vk * dm[jk]);
-  }
-  if constexpr (LDS) {
-    __syncthreads();
-    T* dst = part + (int64_t)blockIdx.x * NN;
-    for (int x = threadIdx.x; x < NN; x += blockDim.x) dst[x] = acc[x];
-  }
-}
-
 // out[x] = sum_b part[b][x] (+ part[b][x^T] when SYM), fixed order.  One
 // 64-lane wave per output element: lanes stride over the partials, then a
 // fixed shuffle tree combines them.
@@ -525,11 +469,135 @@ __global__ void __launch_bounds__(256) zero_active_kernel(const BatchMol* __rest
   for (int x = threadIdx.x; x < NN; x += blockDim.x) out[Mo.mat0 + x] = TO(0);
 }
 
+// ------------------------------------------------------------- sparse form ---
+// LDS-atomic-bound: 12 scatters per ERI, and lanes that add to one address go
+// one after the other.  Lists in packed order (as prepare_sparse makes them)
+// give a wave one (i, j) and runs of equal k, so where a wave's elements are like
+// that, the six targets without l are summed across the lanes first (segmented
+// scans over the runs of k, one wave sum) and added once; any other wave adds
+// element by element.  A symmetric dm (compared element by element) needs only
+// one target of each transposed pair; M + M^T is the result.  The LDS copies
+// have an odd row stride, which spreads the
+// targets l N + x over the banks.  Sixteen waves share a workgroup's copies.
+// A 9-heavy-atom molecule's list in FP32: 127 us with four waves a workgroup and
+// every lane adding all 12 targets, 78 with the sums first, 45 with a symmetric
+// dm; the LDS is then active four fifths of the time (36 cycles an instruction).
+constexpr int JKS_THREADS = 1024;
+
+template <typename T, bool LDS>
+__global__ void __launch_bounds__(JKS_THREADS) jk_sparse_kernel(const T* __restrict__ eri,
+                                                                const int16_t* __restrict__ idx, int64_t nnz,
+                                                                const T* __restrict__ dm_g, int N, int ld, T kscale,
+                                                                T* __restrict__ part) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const T* dm = dm_g;
+  T* acc = part;  // global-atomic mode accumulates into out directly (ld = N)
+  bool sym = false;
+  if constexpr (LDS) {
+    T* sdm = reinterpret_cast<T*>(smem);
+    acc = sdm + N * ld;
+    for (int x = threadIdx.x; x < N * N; x += blockDim.x) {
+      const int r = x / N, y = r * ld + x - r * N;
+      sdm[y] = dm_g[x];
+      acc[y] = T(0);
+    }
+    __syncthreads();
+    dm = sdm;
+    bool eq = true;
+    for (int x = threadIdx.x; x < N * N; x += blockDim.x) {
+      const int r = x / N, c = x - r * N;
+      eq = eq && dm[r * ld + c] == dm[c * ld + r];
+    }
+    sym = __syncthreads_and(eq);
+  }
+  const int lane = threadIdx.x & 63;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t e0 = (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63); e0 < nnz; e0 += stride) {
+    const int64_t e = e0 + lane < nnz ? e0 + lane : nnz - 1;
+    const uint2 packed = reinterpret_cast<const uint2*>(idx)[e];
+    int i = (int)(packed.x & 0xffffu), j = (int)(packed.x >> 16);
+    int k = (int)(packed.y & 0xffffu), l = (int)(packed.y >> 16);
+    // out-of-range indices are dropped, like the reference's FILL_OR_DROP gather/scatter
+    const bool ok = e0 + lane < nnz && i < N && j < N && k < N && l < N;
+    const T v = ok ? eri[e] : T(0);
+    if (!ok) i = j = k = l = 0;
+    const int ij = i * ld + j, ji = j * ld + i, kl = k * ld + l, lk = l * ld + k;
+    const int il = i * ld + l, jl = j * ld + l, ik = i * ld + k, jk = j * ld + k;
+    const int kj = k * ld + j, lj = l * ld + j, ki = k * ld + i, li = l * ld + i;
+    // J: patterns 0-7 gather {ij, ji, kl, lk}, scatter {kl, lk, ij, ji};
+    // K: patterns 16-23 gather / 24-31 scatter, scaled by -hyb/2
+    const T tj1 = v * (dm[ij] + dm[ji]), vk = v * kscale;
+    T tj2 = ok ? v * (dm[kl] + dm[lk]) : T(0);
+    T aik = vk * dm[lj], ajk = vk * dm[li], akj = T(0), aki = T(0);
+    if (!sym) {
+      akj = vk * dm[il];
+      aki = vk * dm[jl];
+    }
+    if (ok) {
+      atomicAdd(acc + kl, tj1);
+      atomicAdd(acc + il, vk * dm[kj]);
+      atomicAdd(acc + jl, vk * dm[ki]);
+      if (!sym) {
+        atomicAdd(acc + lk, tj1);
+        atomicAdd(acc + lj, vk * dm[ik]);
+        atomicAdd(acc + li, vk * dm[jk]);
+      }
+    }
+    // one (i, j), k in order, and the elements dropped (if any) the last lanes
+    const uint64_t m = __ballot(ok);
+    const int kn = __shfl_down(k, 1, 64);
+    const bool last = lane == 63 || !(m >> (lane < 63 ? lane + 1 : 63) & 1);
+    const bool fits = !ok || (i == __builtin_amdgcn_readfirstlane(i) && j == __builtin_amdgcn_readfirstlane(j) &&
+                              (last || kn >= k));
+    if ((m & (m + 1)) == 0 && __all(fits)) {
+      const int key = ok ? k : -1;
+      const bool end = ok && (last || kn != k);
+      seg_scan2(aik, ajk, key);
+      if (end) {
+        atomicAdd(acc + ik, aik);
+        atomicAdd(acc + jk, ajk);
+      }
+      if (!sym) {
+        seg_scan2(akj, aki, key);
+        if (end) {
+          atomicAdd(acc + kj, akj);
+          atomicAdd(acc + ki, aki);
+        }
+      }
+      tj2 = wave_sum_last(tj2);
+      const int ij0 = __builtin_amdgcn_readfirstlane(ij), ji0 = __builtin_amdgcn_readfirstlane(ji);
+      if (lane == 63 && m != 0) {
+        atomicAdd(acc + ij0, tj2);
+        if (!sym) atomicAdd(acc + ji0, tj2);
+      }
+    } else if (ok) {
+      atomicAdd(acc + ij, tj2);
+      atomicAdd(acc + ik, aik);
+      atomicAdd(acc + jk, ajk);
+      if (!sym) {
+        atomicAdd(acc + ji, tj2);
+        atomicAdd(acc + kj, akj);
+        atomicAdd(acc + ki, aki);
+      }
+    }
+  }
+  if constexpr (LDS) {
+    __syncthreads();
+    T* dst = part + (int64_t)blockIdx.x * N * N;
+    for (int x = threadIdx.x; x < N * N; x += blockDim.x) {
+      const int r = x / N, c = x - r * N;
+      dst[x] = sym ? acc[r * ld + c] + acc[c * ld + r] : acc[r * ld + c];
+    }
+  }
+}
+
 template <typename T>
 static int jk_sparse_impl(const T* eri, const int16_t* idx, int64_t nnz, const T* dm, int N, double hyb, T* out,
                           void* ws, size_t ws_bytes, hipStream_t st) {
   const int NN = N * N;
-  const size_t lds = sizeof(T) * 2 * (size_t)NN;
+  // an odd row stride where it still fits
+  const int ld = (int)(sizeof(T) * 2 * (size_t)N * (N | 1)) <= max_lds_bytes() ? N | 1 : N;
+  const size_t lds = sizeof(T) * 2 * (size_t)N * ld;
   const T kscale = (T)(-hyb / 2.0);
   int64_t want = (nnz + JK_THREADS * 8 - 1) / (JK_THREADS * 8);
   int nb = (int)(want < 1 ? 1 : (want > JK_MAX_BLOCKS ? JK_MAX_BLOCKS : want));
@@ -537,14 +605,14 @@ static int jk_sparse_impl(const T* eri, const int16_t* idx, int64_t nnz, const T
     PSCF_REQUIRE(ws && ws_bytes >= sizeof(T) * (size_t)nb * NN, "pscf_jk_sparse: workspace too small");
     PSCF_SET_LDS((jk_sparse_kernel<T, true>), lds);
     if (nnz > 0)
-      jk_sparse_kernel<T, true><<<nb, JK_THREADS, lds, st>>>(eri, idx, nnz, dm, N, kscale, (T*)ws);
+      jk_sparse_kernel<T, true><<<nb, JKS_THREADS, lds, st>>>(eri, idx, nnz, dm, N, ld, kscale, (T*)ws);
     else
       fill_kernel<T><<<64, 256, 0, st>>>((T*)ws, (int64_t)NN, T(0)), nb = 1;
     PSCF_HIP(hipGetLastError());
     jk_reduce_kernel<T, false><<<(NN + 3) / 4, 256, 0, st>>>((const T*)ws, nb, N, out);
   } else {
     fill_kernel<T><<<64, 256, 0, st>>>(out, (int64_t)NN, T(0));
-    if (nnz > 0) jk_sparse_kernel<T, false><<<nb, JK_THREADS, 0, st>>>(eri, idx, nnz, dm, N, kscale, out);
+    if (nnz > 0) jk_sparse_kernel<T, false><<<nb, JKS_THREADS, 0, st>>>(eri, idx, nnz, dm, N, N, kscale, out);
   }
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
