@@ -1911,46 +1911,47 @@ __global__ void energy_kernel(int N, const double* __restrict__ D, const double*
 // ------------------------------------------------------------- batched ----
 // Overlap Cholesky S = L L^T and L^-1 per molecule (FP64, LDS).  A molecule
 // whose S is not positive definite is marked failed and inactive (ctl[2] = -1).
-__global__ void __launch_bounds__(256) chol_batch_kernel(const BatchMol* __restrict__ mols,
-                                                         const double* __restrict__ S, double* __restrict__ Linv,
-                                                         double* __restrict__ ctl) {
+// One elimination gives both: step k scales column k of L and row k of L^-1, then
+// every later row i takes -L_ik times row k, right of column k on what is left of
+// S and left of it on L^-1, which grow into each other's place (two barriers a
+// step; L's current column sits in the unused upper half of row k).  The sums
+// run in the order of a plain substitution.  Bound by the chain of N steps: nao
+// 60 in 58 us, where L^-1 by a thread per column, reading its own earlier
+// rows back from memory, took 214.
+constexpr int CHOL_THREADS = 512;
+__global__ void __launch_bounds__(CHOL_THREADS) chol_batch_kernel(const BatchMol* __restrict__ mols,
+                                                                  const double* __restrict__ S,
+                                                                  double* __restrict__ Linv,
+                                                                  double* __restrict__ ctl) {
   extern __shared__ __align__(16) unsigned char smem[];
   const BatchMol Mo = mols[blockIdx.x];
   const int N = (int)Mo.nao, NN = N * N;
-  double* A = reinterpret_cast<double*>(smem);
-  __shared__ int bad;
-  if (threadIdx.x == 0) bad = 0;
-  for (int x = threadIdx.x; x < NN; x += blockDim.x) A[x] = S[Mo.mat0 + x];
-  __syncthreads();
+  double* M = reinterpret_cast<double*>(smem);  // [N][N]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  bool bad = false;
+  for (int x = threadIdx.x; x < NN; x += blockDim.x) M[x] = S[Mo.mat0 + x];
   for (int k = 0; k < N; ++k) {
-    if (threadIdx.x == 0) {
-      const double d = A[k * N + k];
-      if (!(d > 0.0)) bad = 1;
-      A[k * N + k] = d > 0.0 ? sqrt(d) : 1.0;
+    __syncthreads();
+    const double d = M[k * N + k];
+    bad = bad || !(d > 0.0);
+    const double l = d > 0.0 ? sqrt(d) : 1.0, wkk = 1.0 / l;
+    double* row = M + k * N;  // row k of L^-1 | 1 / l | column k of L
+    for (int i = threadIdx.x; i < N; i += blockDim.x)
+      if (i != k) row[i] = (i < k ? row[i] : M[i * N + k]) / l;
+    __syncthreads();
+    if (threadIdx.x == 0) row[k] = wkk;
+    for (int j = lane; j < N; j += 64) {
+      const double f = j == k ? wkk : row[j];
+#pragma unroll 4
+      for (int i = k + 1 + wave; i < N; i += CHOL_THREADS / 64)
+        if (j <= i) M[i * N + j] = (j == k ? 0.0 : M[i * N + j]) - row[i] * f;
     }
-    __syncthreads();
-    const double lkk = A[k * N + k];
-    for (int i = k + 1 + threadIdx.x; i < N; i += blockDim.x) A[i * N + k] /= lkk;
-    __syncthreads();
-    const int rem = N - k - 1;
-    for (int t = threadIdx.x; t < rem * rem; t += blockDim.x) {
-      const int i = k + 1 + t / rem, j = k + 1 + t % rem;
-      if (j <= i) A[i * N + j] -= A[i * N + k] * A[j * N + k];
-    }
-    __syncthreads();
   }
-  // L^-1 column by column (forward substitution), one thread per column
+  __syncthreads();
   double* out = Linv + Mo.mat0;
-  for (int j = threadIdx.x; j < N; j += blockDim.x) {
-    for (int i = 0; i < N; ++i) {
-      if (i < j) {
-        out[i * N + j] = 0.0;
-        continue;
-      }
-      double acc = (i == j) ? 1.0 : 0.0;
-      for (int k = j; k < i; ++k) acc -= A[i * N + k] * out[k * N + j];
-      out[i * N + j] = acc / A[i * N + i];
-    }
+  for (int x = threadIdx.x; x < NN; x += blockDim.x) {
+    const int i = x / N, j = x - i * N;
+    out[x] = j <= i ? M[x] : 0.0;
   }
   if (threadIdx.x == 0 && bad) {
     ctl[blockIdx.x * CTL + 1] = 0.0;
@@ -2258,7 +2259,7 @@ extern "C" int pscf_batch_chol(const void* d_mols, int nmol, int max_nao, const 
   const int maxlds = device_max_lds();
   PSCF_REQUIRE((int)lds <= maxlds, "pscf_batch_chol: nao %d too large", max_nao);
   PSCF_SET_LDS(chol_batch_kernel, lds);
-  chol_batch_kernel<<<nmol, 256, lds, (hipStream_t)stream>>>((const BatchMol*)d_mols, d_S, d_Linv, d_ctl);
+  chol_batch_kernel<<<nmol, CHOL_THREADS, lds, (hipStream_t)stream>>>((const BatchMol*)d_mols, d_S, d_Linv, d_ctl);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
 }
