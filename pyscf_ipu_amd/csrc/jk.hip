@@ -15,6 +15,7 @@
 
 #include "batch.h"
 #include "common.h"
+#include "loop.h"
 #include "reduce.h"
 #include "wave.h"
 
@@ -768,7 +769,7 @@ static size_t jk_s8_lds(int N) {
 
 template <typename T>
 static int jk_s8_impl(const T* eri, int N, const T* dm, double hyb, T* out, void* ws, size_t ws_bytes,
-                      hipStream_t st) {
+                      hipStream_t st, bool zeroed = false) {
   // FP64 accumulator when it fits, else one of T (FP32 molecules up to nao 143)
   const bool acc64 = (int)jk_s8_lds<T, double>(N) <= max_lds_bytes();
   const size_t lds = acc64 ? jk_s8_lds<T, double>(N) : jk_s8_lds<T, T>(N);
@@ -779,7 +780,7 @@ static int jk_s8_impl(const T* eri, int N, const T* dm, double hyb, T* out, void
   // FP64: exact atomic sums into the zeroed output, no partials to reduce
   constexpr bool ATOMIC = sizeof(T) == 8;
   double* aout = ATOMIC ? (double*)out : nullptr;
-  if (ATOMIC) {
+  if (ATOMIC && !zeroed) {
     const int rz = zero2(aout, (int64_t)N * N, nullptr, 0, st);
     if (rz) return rz;
   }
@@ -1067,6 +1068,11 @@ extern "C" int pscf_jk_s8_large(int dtype, const void* d_eri_s8, int N, const do
   jk8l_sym_kernel<<<(unsigned)(nb < 65536 ? nb : 65536), 256, 0, st>>>(M, N, d_out);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
+}
+
+int pscf::jk_s8_f64_zeroed(const double* eri, int N, const double* dm, double hyb, double* out, void* ws,
+                           size_t ws_bytes, hipStream_t st) {
+  return jk_s8_impl<double>(eri, N, dm, hyb, out, ws, ws_bytes, st, true);
 }
 
 extern "C" size_t pscf_jk_s8_workspace_bytes(int dtype, int N) {

@@ -13,6 +13,7 @@
 // disjoint rotations per round) is the fallback and serves N > 64.
 #include "batch.h"
 #include "common.h"
+#include "loop.h"
 #include "wave.h"
 
 namespace pscf {
@@ -1832,11 +1833,18 @@ __global__ void __launch_bounds__(SCF_THREADS) scf_step_kernel(int it, int N, in
                                                                const T* __restrict__ dJK, const T* __restrict__ Vxc,
                                                                double* __restrict__ D, double* __restrict__ Hout,
                                                                double* __restrict__ mo_e, double* __restrict__ Cout,
-                                                               double* __restrict__ state, int use_diis) {
+                                                               double* __restrict__ state, int use_diis,
+                                                               double* zero_v, double* zero_e) {
   extern __shared__ __align__(16) unsigned char smem[];
   const ScfLds L = scf_lds_carve(smem, N);
   scf_step_body<T, T>(L, it, N, nocc, Hcore, S, Linv, dJK, Vxc, D, (T*)nullptr, (T*)nullptr, Hout, mo_e, Cout, state,
                       use_diis);
+  // (Vxc was read before the step's first barriers)
+  if (zero_v != nullptr) {
+    __syncthreads();
+    for (int x = threadIdx.x; x < N * N; x += SCF_THREADS) zero_v[x] = 0.0;
+    if (threadIdx.x == 0) *zero_e = 0.0;
+  }
 }
 
 // The same step for molecules whose three N x N working matrices exceed the
@@ -1883,8 +1891,10 @@ __global__ void __launch_bounds__(SCF_THREADS) scf_step_ws_kernel(int it, int N,
 template <typename T>
 __global__ void energy_kernel(int N, const double* __restrict__ D, const double* __restrict__ Hcore,
                               const T* __restrict__ dJK, const double* __restrict__ exc, double e_nuc,
-                              double* __restrict__ out) {
+                              double* __restrict__ out, const double* __restrict__ mo_e, double* __restrict__ host) {
   __shared__ double red[16];
+  if (host != nullptr)
+    for (int i = threadIdx.x; i < N; i += blockDim.x) host[5 + i] = mo_e[i];
   double s1 = 0.0, c1 = 0.0, s2 = 0.0, c2 = 0.0;  // Neumaier sums (1024 threads: a few terms each)
   for (int x = threadIdx.x; x < N * N; x += blockDim.x) {
     const double a = D[x] * Hcore[x];
@@ -1899,12 +1909,11 @@ __global__ void energy_kernel(int N, const double* __restrict__ D, const double*
   const double e_core = block_sum(s1 + c1, red);
   const double e_jk = 0.5 * block_sum(s2 + c2, red);
   if (threadIdx.x == 0) {
-    const double ex = *exc;
-    out[0] = e_core + e_jk + ex + e_nuc;
-    out[1] = e_core;
-    out[2] = e_jk;
-    out[3] = ex;
-    out[4] = e_nuc;
+    const double ex = *exc, e[5] = {e_core + e_jk + ex + e_nuc, e_core, e_jk, ex, e_nuc};
+    for (int k = 0; k < 5; ++k) {
+      out[k] = e[k];
+      if (host != nullptr) host[k] = e[k];
+    }
   }
 }
 
@@ -2195,20 +2204,28 @@ extern "C" int pscf_scf_step(int dtype, int iteration, int N, int nocc, const do
   PSCF_REQUIRE(N > 1 && nocc >= 0 && nocc <= N && iteration >= 0, "pscf_scf_step: bad sizes");
   PSCF_REQUIRE(d_Hcore && d_S && d_Linv && d_dJK && d_Vxc && d_D && d_H && d_mo_energy && d_C && d_state,
                "pscf_scf_step: null pointer");
+  return scf_step_zero(dtype, iteration, N, nocc, d_Hcore, d_S, d_Linv, d_dJK, d_Vxc, d_D, d_H, d_mo_energy, d_C,
+                       d_state, use_diis, nullptr, nullptr, (hipStream_t)stream);
+}
+
+int pscf::scf_step_zero(int dtype, int iteration, int N, int nocc, const double* d_Hcore, const double* d_S,
+                        const double* d_Linv, const void* d_dJK, const void* d_Vxc, double* d_D, double* d_H,
+                        double* d_mo_energy, double* d_C, void* d_state, int use_diis, double* zero_v, double* zero_e,
+                        hipStream_t st) {
   const size_t lds = scf_lds(N);
   const int maxlds = device_max_lds();
   PSCF_REQUIRE((int)lds <= maxlds, "pscf_scf_step: N=%d needs %zu B LDS (max %d)", N, lds, maxlds);
-  hipStream_t st = (hipStream_t)stream;
   if (dtype == PSCF_F64) {
     PSCF_SET_LDS(scf_step_kernel<double>, lds);
     scf_step_kernel<double><<<1, SCF_THREADS, lds, st>>>(iteration, N, nocc, d_Hcore, d_S, d_Linv,
                                                          (const double*)d_dJK, (const double*)d_Vxc, d_D, d_H,
-                                                         d_mo_energy, d_C, (double*)d_state, use_diis);
+                                                         d_mo_energy, d_C, (double*)d_state, use_diis, zero_v,
+                                                         zero_e);
   } else {
     PSCF_SET_LDS(scf_step_kernel<float>, lds);
     scf_step_kernel<float><<<1, SCF_THREADS, lds, st>>>(iteration, N, nocc, d_Hcore, d_S, d_Linv, (const float*)d_dJK,
                                                         (const float*)d_Vxc, d_D, d_H, d_mo_energy, d_C,
-                                                        (double*)d_state, use_diis);
+                                                        (double*)d_state, use_diis, zero_v, zero_e);
   }
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
@@ -2243,11 +2260,16 @@ extern "C" int pscf_energy(int dtype, int N, const double* d_D, const double* d_
                            const double* d_exc, double e_nuc, double* d_out, void* stream) {
   PSCF_REQUIRE(dtype == PSCF_F64 || dtype == PSCF_F32, "pscf_energy: bad dtype");
   PSCF_REQUIRE(N > 0 && d_D && d_Hcore && d_dJK && d_exc && d_out, "pscf_energy: bad arguments");
-  hipStream_t st = (hipStream_t)stream;
+  return energy_to_host(dtype, N, d_D, d_Hcore, d_dJK, d_exc, e_nuc, d_out, nullptr, nullptr, (hipStream_t)stream);
+}
+
+int pscf::energy_to_host(int dtype, int N, const double* d_D, const double* d_Hcore, const void* d_dJK,
+                         const double* d_exc, double e_nuc, double* d_out, const double* mo_e, double* host,
+                         hipStream_t st) {
   if (dtype == PSCF_F64)
-    energy_kernel<double><<<1, 1024, 0, st>>>(N, d_D, d_Hcore, (const double*)d_dJK, d_exc, e_nuc, d_out);
+    energy_kernel<double><<<1, 1024, 0, st>>>(N, d_D, d_Hcore, (const double*)d_dJK, d_exc, e_nuc, d_out, mo_e, host);
   else
-    energy_kernel<float><<<1, 1024, 0, st>>>(N, d_D, d_Hcore, (const float*)d_dJK, d_exc, e_nuc, d_out);
+    energy_kernel<float><<<1, 1024, 0, st>>>(N, d_D, d_Hcore, (const float*)d_dJK, d_exc, e_nuc, d_out, mo_e, host);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
 }

@@ -15,6 +15,7 @@
 #include "b3lyp.h"
 #include "batch.h"
 #include "common.h"
+#include "loop.h"
 #include "reduce.h"
 #include "wave.h"
 
@@ -148,6 +149,8 @@ struct XCArgs {
   double* part_e;   // [blocks]
   T* vout;          // FP64: V_xc (zeroed) and E_xc take each workgroup's part by
   double* eout;     //   exact atomics instead of the partials (nullptr: partials)
+  double* zero;     // set to 0 on the side: a later kernel's output
+  int64_t nzero;
 };
 
 // LDS layout: D[N][N] | phi0[N][TILE+1] | XY[N][TILE+1] | coef[4][TILE] | red[8]
@@ -608,6 +611,8 @@ __global__ void __launch_bounds__(XC_THREADS, (xw_min_blocks<T, NP>())) xc_wave_
   typename L::v4 vacc[L::NB * L::NB];
   XwAO<T, NP> ao;
   double e_loc = 0.0;
+  for (int64_t x = (int64_t)blockIdx.x * XC_THREADS + threadIdx.x; x < a.nzero; x += (int64_t)gridDim.x * XC_THREADS)
+    a.zero[x] = 0.0;
   XwStored<T, NP> stage{a.ao, (int)a.sc, (int)a.smu, (int)a.sp, a.g, a.N};
   stage.init();
   const int ntiles = (a.g + 63) / 64, p0 = blockIdx.x * 64 + (int)(threadIdx.x >> 6) * 16;
@@ -1211,7 +1216,8 @@ static int xc_launch(const XCArgs<T>& a, int nb, hipStream_t st) {
 
 template <typename T>
 static int xc_impl(const T* ao, int64_t sc, int64_t smu, int64_t sp, int g, int N, const T* dm, const T* w,
-                   double eps, double* exc, T* vxc, void* ws, size_t ws_bytes, hipStream_t st) {
+                   double eps, double* exc, T* vxc, void* ws, size_t ws_bytes, bool zeroed, double* zero,
+                   int64_t nzero, hipStream_t st) {
   PSCF_REQUIRE(N <= XM_MAXN, "pscf_xc: N=%d too large (max %d)", N, XM_MAXN);
   PSCF_REQUIRE(3 * sc + (int64_t)(N - 1) * smu + (int64_t)(g - 1) * sp < ((int64_t)1 << 31),
                "pscf_xc: AO block of %lld elements needs 32-bit offsets", (long long)(4 * sc));
@@ -1234,7 +1240,9 @@ static int xc_impl(const T* ao, int64_t sc, int64_t smu, int64_t sp, int g, int 
   constexpr bool ATOMIC = sizeof(T) == 8;
   a.vout = ATOMIC ? vxc : nullptr;
   a.eout = ATOMIC ? exc : nullptr;
-  if (ATOMIC) {
+  a.zero = zero;
+  a.nzero = nzero;
+  if (ATOMIC && !zeroed) {
     const int rz = zero2((double*)vxc, (int64_t)N * N, exc, 1, st);
     if (rz) return rz;
   }
@@ -1553,9 +1561,16 @@ extern "C" int pscf_xc(int dtype, const void* d_ao, int64_t ao_sc, int64_t ao_sm
   hipStream_t st = (hipStream_t)stream;
   if (dtype == PSCF_F64)
     return xc_impl<double>((const double*)d_ao, ao_sc, ao_smu, ao_sp, g, N, (const double*)d_dm,
-                           (const double*)d_weights, eps, d_exc, (double*)d_vxc, d_ws, ws_bytes, st);
+                           (const double*)d_weights, eps, d_exc, (double*)d_vxc, d_ws, ws_bytes, false, nullptr, 0,
+                           st);
   return xc_impl<float>((const float*)d_ao, ao_sc, ao_smu, ao_sp, g, N, (const float*)d_dm, (const float*)d_weights,
-                        eps, d_exc, (float*)d_vxc, d_ws, ws_bytes, st);
+                        eps, d_exc, (float*)d_vxc, d_ws, ws_bytes, false, nullptr, 0, st);
+}
+
+int pscf::xc_f64(const double* ao, int64_t sc, int64_t smu, int64_t sp, int g, int N, const double* dm,
+                 const double* w, double eps, double* exc, double* vxc, void* ws, size_t ws_bytes, bool zeroed,
+                 double* zero, int64_t nzero, hipStream_t st) {
+  return xc_impl<double>(ao, sc, smu, sp, g, N, dm, w, eps, exc, vxc, ws, ws_bytes, zeroed, zero, nzero, st);
 }
 
 extern "C" int pscf_batch_grid(const int* d_work, int nwork, const int* d_atom_elem, const int64_t* d_atom_pt0,
