@@ -13,6 +13,7 @@
 //     fold into one accumulator M with dJK = M + M^T (6 scatters per ERI).
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "batch.h"
 #include "common.h"
@@ -900,7 +901,8 @@ extern "C" int pscf_jk_blocks(int dtype, const void* d_eri, const int* d_blocks,
 //     q of M), (p, r) and (q, r) (segmented sums over runs of equal r);
 //     rows p and q of D sit in the wave's LDS, D[r][s] comes from a packed
 //     copy of D (index rs, coalesced).  After the row, the two row
-//     accumulators and the dot go to M with global atomics.
+//     accumulators and the dot go to M with global atomics.  (Up to nao 256:
+//     jk8l_rows_wave_kernel, whose lanes keep their columns in registers.)
 //   columns pass: the remaining J target (r, s) += 2 w D[p][q], one wave per
 //     (block of 64 rs, block of rows pq): lane rs sums over the rows in a
 //     register, then adds to M once.
@@ -992,6 +994,150 @@ __global__ void __launch_bounds__(64 * JK8L_WAVES) jk8l_rows_kernel(const T* __r
   }
 }
 
+// The rows pass for nao <= 64 NS: lanes keep columns s = lane + 64 c, so D[p][s],
+// D[q][s] and the row sums (p, s), (q, s) are registers; r is wave-uniform, and
+// the sums over s for (p, r), (q, r) are reduced 16 at a time (8 r).  Only a
+// row's last 64 columns and last r need masks.  DLDS: D packed in LDS, where it
+// fits.  About 45 instructions per (row, r) against 100 per 64 elements of
+// jk8l_rows_kernel (indices by square root, LDS atomics, segmented scans): nao
+// 161, FP64 391 -> 223 us, the ERIs' HBM time being 148.
+constexpr int JK8W_THREADS = 512;
+
+template <typename T, int NS, bool DLDS>
+__global__ void __launch_bounds__(JK8W_THREADS) jk8l_rows_wave_kernel(const T* __restrict__ eri, int N,
+                                                                      const double* __restrict__ dm,
+                                                                      const double* __restrict__ dpk, double hhalf,
+                                                                      double* __restrict__ M) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int lane = threadIdx.x & 63, P = (int)tri(N);
+  // the wave's sums (p, r) and (q, r), then D packed
+  double* rp = reinterpret_cast<double*>(smem) + (threadIdx.x >> 6) * 2 * N;
+  double* dl = reinterpret_cast<double*>(smem) + JK8W_THREADS / 64 * 2 * N;
+  if constexpr (DLDS) {
+    for (int x = threadIdx.x; x < P; x += JK8W_THREADS) dl[x] = dpk[x];
+    __syncthreads();
+  }
+  const int nw = gridDim.x * (JK8W_THREADS / 64);
+  for (int item = __builtin_amdgcn_readfirstlane(blockIdx.x * (JK8W_THREADS / 64) + (threadIdx.x >> 6)); item < P;
+       item += nw) {
+    const int pq = P - 1 - item;  // longest rows first
+    int p, q;
+    tri_split(pq, p, q);
+    p = __builtin_amdgcn_readfirstlane(p);
+    q = __builtin_amdgcn_readfirstlane(q);
+    const T* row = eri + tri(pq);
+    double dps[NS], dqs[NS], aps[NS], aqs[NS], jrow = 0.0;
+#pragma unroll
+    for (int c = 0; c < NS; ++c) {
+      const int s = 64 * c + lane;
+      dps[c] = s < N ? dm[(int64_t)p * N + s] : 0.0;
+      dqs[c] = s < N ? dm[(int64_t)q * N + s] : 0.0;
+      aps[c] = aqs[c] = 0.0;
+    }
+    const double fpq = p == q ? 0.5 : 1.0, fk = -hhalf * fpq;
+    // r = g .. g + 7 with 64 CR <= g < 64 CR + 64; END: the group that holds
+    // r = p, where columns end at q and later r have none
+    auto group = [&](auto cr_tag, auto end_tag, int g) {
+      constexpr int CR = decltype(cr_tag)::value;
+      constexpr bool END = decltype(end_tag)::value;
+      double w[8][CR + 1], d[8][CR + 1];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int r = g + u, lim = !END || r < p ? r : (r == p ? q : -1), base = r * (r + 1) / 2;
+#pragma unroll
+        for (int c = 0; c <= CR; ++c) {
+          const int s = 64 * c + lane, x = (!END && c < CR) || s <= lim ? base + s : 0;
+          w[u][c] = (double)row[x];
+          d[u][c] = DLDS ? dl[x] : dpk[x];
+        }
+      }
+      double t[16];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int r = g + u, lim = !END || r < p ? r : (r == p ? q : -1);
+        // weights: 1/2 on r = s and on rs = pq
+        const double h = !END || r < p || q < p ? 0.5 : 0.25;
+        const double dqr = lane_read(dqs[CR], r & 63), dpr = lane_read(dps[CR], r & 63);
+        t[u] = t[8 + u] = 0.0;
+#pragma unroll
+        for (int c = 0; c <= CR; ++c) {
+          const int s = 64 * c + lane;
+          double v = w[u][c];
+          if (END || c == CR) v = s < lim ? v : (s == lim ? v * h : 0.0);
+          jrow += v * d[u][c];
+          aps[c] += v * dqr;
+          aqs[c] += v * dpr;
+          t[u] += v * dqs[c];
+          t[8 + u] += v * dps[c];
+        }
+      }
+      const double tot = transpose_reduce16(t, lane);
+      const int r = g + (lane & 7);
+      if (lane < 16 && (!END || r <= p)) rp[(lane < 8 ? 0 : N) + r] = tot;
+    };
+    auto block = [&](auto cr_tag) {
+      constexpr int CR = decltype(cr_tag)::value;
+      int g = 64 * CR;
+#pragma unroll 1
+      for (; g < 64 * CR + 64 && g + 7 < p; g += 8) group(cr_tag, std::false_type{}, g);
+      if (g < 64 * CR + 64 && g <= p) group(cr_tag, std::true_type{}, g);
+    };
+    block(std::integral_constant<int, 0>{});
+    if constexpr (NS > 1)
+      if (p >= 64) block(std::integral_constant<int, 1>{});
+    if constexpr (NS > 2)
+      if (p >= 128) block(std::integral_constant<int, 2>{});
+    if constexpr (NS > 3)
+      if (p >= 192) block(std::integral_constant<int, 3>{});
+    jk8l_wave_sync();
+#pragma unroll
+    for (int c = 0; c < NS; ++c) {
+      const int s = 64 * c + lane;
+      if (s <= p) {  // (columns and r both end at p)
+        atomicAdd(M + (int64_t)p * N + s, jk_quant((aps[c] + rp[s]) * fk));
+        atomicAdd(M + (int64_t)q * N + s, jk_quant((aqs[c] + rp[N + s]) * fk));
+      }
+    }
+    jk8l_wave_sync();
+    jrow = wave_sum_last(jrow) * (2.0 * fpq);
+    if (lane == 63) atomicAdd(M + (int64_t)p * N + q, jk_quant(jrow));
+  }
+}
+
+static size_t jk8l_rows_lds(int N, bool dlds) {
+  return sizeof(double) * ((size_t)JK8W_THREADS / 64 * 2 * N + (dlds ? (size_t)tri(N) : 0));
+}
+
+template <typename T, int NS, bool DLDS>
+static int jk8l_rows_wave_launch(const T* eri, int N, const double* dm, const double* dpk, double hhalf, double* M,
+                                 hipStream_t st) {
+  const size_t lds = jk8l_rows_lds(N, DLDS);
+  const int per_cu = std::max(1, std::min(4, (int)((size_t)max_lds_bytes() / lds)));
+  const int64_t want = (tri(N) + JK8W_THREADS / 64 - 1) / (JK8W_THREADS / 64);
+  PSCF_SET_LDS((jk8l_rows_wave_kernel<T, NS, DLDS>), lds);
+  jk8l_rows_wave_kernel<T, NS, DLDS>
+      <<<(unsigned)std::min<int64_t>(want, 256 * per_cu), JK8W_THREADS, lds, st>>>(eri, N, dm, dpk, hhalf, M);
+  PSCF_HIP(hipGetLastError());
+  return PSCF_OK;
+}
+
+template <typename T>
+static int jk8l_rows(const T* eri, int N, const double* dm, const double* dpk, double hhalf, double* M,
+                     hipStream_t st) {
+  const bool fits = jk8l_rows_lds(N, true) <= (size_t)max_lds_bytes();  // nao <= 186
+  if (N <= 128) return jk8l_rows_wave_launch<T, 2, true>(eri, N, dm, dpk, hhalf, M, st);
+  if (N <= 192 && fits) return jk8l_rows_wave_launch<T, 3, true>(eri, N, dm, dpk, hhalf, M, st);
+  if (N <= 192) return jk8l_rows_wave_launch<T, 3, false>(eri, N, dm, dpk, hhalf, M, st);
+  if (N <= 256) return jk8l_rows_wave_launch<T, 4, false>(eri, N, dm, dpk, hhalf, M, st);
+  const size_t lds = sizeof(double) * 4 * (size_t)N * JK8L_WAVES;
+  const int64_t rows_wg = (tri(N) + JK8L_WAVES - 1) / JK8L_WAVES;
+  PSCF_SET_LDS(jk8l_rows_kernel<T>, lds);
+  jk8l_rows_kernel<T><<<(unsigned)std::min<int64_t>(rows_wg, 4096), 64 * JK8L_WAVES, lds, st>>>(eri, N, dm, dpk,
+                                                                                                hhalf, M);
+  PSCF_HIP(hipGetLastError());
+  return PSCF_OK;
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) jk8l_cols_kernel(const T* __restrict__ eri, int N,
                                                         const double* __restrict__ dpk, double* __restrict__ M) {
@@ -1010,16 +1156,35 @@ __global__ void __launch_bounds__(256) jk8l_cols_kernel(const T* __restrict__ er
     int r, s;
     tri_split(rs < P ? rs : P - 1, r, s);
     const double frs = r == s ? 0.5 : 1.0;
+    // eight rows' loads in flight, (p, q) not decoded per row: nao 161, FP64 241 ->
+    // 150 us, the ERIs' HBM time; diagonal rows pq = (p, p) are met in order
+    int p, q;
+    tri_split(row0, p, q);
+    p = __builtin_amdgcn_readfirstlane(p);
+    int diag = p * (p + 1) / 2 + p;
     double jt = 0.0;
-    for (int pq = row0; pq < row1; ++pq) {
-      int p, q;
-      tri_split(pq, p, q);
-      const double v = (rs <= pq) ? (double)eri[tri(pq) + rs] : 0.0;
-      double w = v * frs * (p == q ? 0.5 : 1.0);
-      if (rs == pq) w *= 0.5;
-      jt += 2.0 * w * dpk[pq];
+    for (int pq0 = row0; pq0 < row1; pq0 += 8) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int pq = min(pq0 + u, row1 - 1);
+        v[u] = (double)eri[tri(pq) + min(rs, pq)];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int pq = pq0 + u;
+        if (pq < row1) {  // uniform
+          double f = 2.0 * dpk[pq];
+          if (pq == diag) {
+            f *= 0.5;
+            ++p;
+            diag += p + 1;
+          }
+          jt += (rs < pq ? v[u] : (rs == pq ? 0.5 * v[u] : 0.0)) * f;
+        }
+      }
     }
-    if (rs < P) atomicAdd(M + (int64_t)r * N + s, jk_quant(jt));
+    if (rs < P) atomicAdd(M + (int64_t)r * N + s, jk_quant(jt * frs));
   }
 }
 
@@ -1049,19 +1214,15 @@ extern "C" int pscf_jk_s8_large(int dtype, const void* d_eri_s8, int N, const do
   const int64_t prep = ((int64_t)N * N + P + 255) / 256;
   jk8l_prep_kernel<<<(unsigned)(prep < 65536 ? prep : 65536), 256, 0, st>>>(d_dm, N, M, dpk);
   PSCF_HIP(hipGetLastError());
-  const int64_t rows_wg = (P + JK8L_WAVES - 1) / JK8L_WAVES;
-  const unsigned g1 = (unsigned)(rows_wg < 4096 ? rows_wg : 4096);
   const int64_t items = ((P + 63) / 64) * ((P + JK8L_ROWS - 1) / JK8L_ROWS);
   const unsigned g2 = (unsigned)((items + 3) / 4 < 8192 ? (items + 3) / 4 : 8192);
   if (dtype == PSCF_F64) {
-    PSCF_SET_LDS(jk8l_rows_kernel<double>, lds);
-    jk8l_rows_kernel<double><<<g1, 64 * JK8L_WAVES, lds, st>>>((const double*)d_eri_s8, N, d_dm, dpk, hyb / 2.0, M);
-    PSCF_HIP(hipGetLastError());
+    const int rc = jk8l_rows<double>((const double*)d_eri_s8, N, d_dm, dpk, hyb / 2.0, M, st);
+    if (rc) return rc;
     jk8l_cols_kernel<double><<<g2, 256, 0, st>>>((const double*)d_eri_s8, N, dpk, M);
   } else {
-    PSCF_SET_LDS(jk8l_rows_kernel<float>, lds);
-    jk8l_rows_kernel<float><<<g1, 64 * JK8L_WAVES, lds, st>>>((const float*)d_eri_s8, N, d_dm, dpk, hyb / 2.0, M);
-    PSCF_HIP(hipGetLastError());
+    const int rc = jk8l_rows<float>((const float*)d_eri_s8, N, d_dm, dpk, hyb / 2.0, M, st);
+    if (rc) return rc;
     jk8l_cols_kernel<float><<<g2, 256, 0, st>>>((const float*)d_eri_s8, N, dpk, M);
   }
   PSCF_HIP(hipGetLastError());
