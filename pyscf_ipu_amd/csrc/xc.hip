@@ -153,9 +153,10 @@ struct XCArgs {
   int64_t nzero;
 };
 
-// LDS layout: D[N][N] | phi0[N][TILE+1] | XY[N][TILE+1] | coef[4][TILE] | red[8]
 // ---- MFMA path ------------------------------------------------------------------
-// Per tile of XT points (64 in FP32, 32 in FP64), with the tile's AO values and
+// Workgroup-wide tiles, for FP64 batches above nao 48 with AO values evaluated in
+// the kernel (everything else: xc_wave.h).
+// Per tile of XT points (32), with the tile's AO values and
 // gradients staged in LDS as Phi[c][p][nu] (row stride XS = NP + 4, NP = N
 // rounded up to 16):
 //   GEMM 1 (v_mfma_{f32,f64}_16x16x4): X[p][nu] = sum_mu phi0[p][mu] D[mu][nu];
@@ -577,12 +578,13 @@ __device__ inline void xm_store_v(const XVacc<T, XT, NP>& vacc, int N, T* dst, i
   }
 }
 
+template <int WAVES = XC_THREADS / 64>
 __device__ inline double xc_block_energy(double e_loc, double* red) {
   for (int off = 32; off > 0; off >>= 1) e_loc += __shfl_xor(e_loc, off, 64);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = e_loc;
   __syncthreads();
   double s = 0.0;
-  for (int k = 0; k < XC_THREADS / 64; ++k) s += red[k];
+  for (int k = 0; k < WAVES; ++k) s += red[k];
   return s;
 }
 
@@ -603,19 +605,20 @@ constexpr int xw_min_blocks() {
 // FP64 adds the workgroup's V + V^T and energy into the zeroed outputs (exact
 // atomics), FP32 leaves V and the energy in part_v and part_e.
 template <typename T, int NP>
-__global__ void __launch_bounds__(XC_THREADS, (xw_min_blocks<T, NP>())) xc_wave_kernel(XCArgs<T> a) {
+__global__ void __launch_bounds__((XW<T, NP, true>::THREADS), (xw_min_blocks<T, NP>())) xc_wave_kernel(XCArgs<T> a) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T* smem = reinterpret_cast<T*>(smem_raw);
   typedef XW<T, NP, true> L;
   T dreg[L::ND];
-  typename L::v4 vacc[L::NB * L::NB];
+  typename L::v4 vacc[L::NB * L::NBH];
   XwAO<T, NP> ao;
   double e_loc = 0.0;
-  for (int64_t x = (int64_t)blockIdx.x * XC_THREADS + threadIdx.x; x < a.nzero; x += (int64_t)gridDim.x * XC_THREADS)
+  for (int64_t x = (int64_t)blockIdx.x * L::THREADS + threadIdx.x; x < a.nzero; x += (int64_t)gridDim.x * L::THREADS)
     a.zero[x] = 0.0;
   XwStored<T, NP> stage{a.ao, (int)a.sc, (int)a.smu, (int)a.sp, a.g, a.N};
-  stage.init();
-  const int ntiles = (a.g + 63) / 64, p0 = blockIdx.x * 64 + (int)(threadIdx.x >> 6) * 16;
+  const int wave = threadIdx.x >> 6;
+  stage.init(wave % L::HS * L::NBH * 16);
+  const int ntiles = (a.g + 63) / 64, p0 = blockIdx.x * 64 + wave / L::HS * 16;
   stage.template load<0, 1>(p0, ao.f0);
   stage.template load<1, 4>(p0, ao.fg);
   xw_load_d<T, NP, true>(a.dm, a.N, dreg);
@@ -623,7 +626,7 @@ __global__ void __launch_bounds__(XC_THREADS, (xw_min_blocks<T, NP>())) xc_wave_
   xw_tiles_stored<T, NP>(a, smem, blockIdx.x, gridDim.x, ntiles, -1, stage, ao, dreg, vacc, e_loc);
   double* red = reinterpret_cast<double*>(smem + L::MAIN);
   __syncthreads();
-  const double e = xc_block_energy(e_loc, red);
+  const double e = xc_block_energy<L::THREADS / 64>(e_loc, red);
   const int N = a.N;
   if (a.vout != nullptr) {
     if (threadIdx.x == 0) atomicAdd(a.eout, quant40(e));
@@ -750,7 +753,7 @@ __global__ void __launch_bounds__(XC_THREADS) xc_batch_kernel(
 // xc_batch_kernel with wave-private tiles: the same chunks and outputs; a
 // chunk's slot holds the lower triangle of its V + V^T, packed.
 template <typename T, int NP, bool DIRECT>
-__global__ void __launch_bounds__(XC_THREADS, (xw_min_blocks<T, NP>())) xc_wave_batch_kernel(
+__global__ void __launch_bounds__((XW<T, NP, !DIRECT>::THREADS), (xw_min_blocks<T, NP>())) xc_wave_batch_kernel(
     const BatchMol* __restrict__ mols, const int* __restrict__ order, int max_nao, const double* __restrict__ ctl,
     const T* __restrict__ ao, XcDirect da, const T* __restrict__ dm, const T* __restrict__ w, T eps,
     T* __restrict__ vxc, double* __restrict__ exc, T* __restrict__ part_v, double* __restrict__ part_e,
@@ -779,15 +782,15 @@ __global__ void __launch_bounds__(XC_THREADS, (xw_min_blocks<T, NP>())) xc_wave_
                   : part >= nchunk || !xc_parts_fit(nchunk, gridDim.x, max_nao, part_v_elems, part_e_elems))
     return;  // buffers that do not fit are marked by the reduction
   constexpr int TPC = XC_CHUNK_PTS / 64;  // tiles per chunk
-  const int wp = (int)(threadIdx.x >> 6) * 16, nrun = nchunk > 1 ? nchunk : 1;
+  const int wave = threadIdx.x >> 6, wp = wave / L::HS * 16, nrun = nchunk > 1 ? nchunk : 1;
   const T* D = dm + Mo.mat0;
   double* red = reinterpret_cast<double*>(smem + L::MAIN);
   T dreg[L::ND];
-  typename L::v4 vacc[L::NB * L::NB];
+  typename L::v4 vacc[L::NB * L::NBH];
   xw_load_d<T, NP, !DIRECT>(D, N, dreg);
   auto flush = [&](int c, double e_loc) {
     __syncthreads();
-    const double e = xc_block_energy(e_loc, red);
+    const double e = xc_block_energy<L::THREADS / 64>(e_loc, red);
     if (nchunk > 1) {
       const int64_t slot = (int64_t)c * gridDim.x + blockIdx.x;
       if (threadIdx.x == 0) part_e[slot] = e;
@@ -817,7 +820,7 @@ __global__ void __launch_bounds__(XC_THREADS, (xw_min_blocks<T, NP>())) xc_wave_
   } else {
     XwStored<T, NP> stage{ao + Mo.ao0, N * a.g, a.g, 1, a.g, N};
     XwAO<T, NP> f;
-    stage.init();
+    stage.init(wave % L::HS * L::NBH * 16);
     if (part * TPC < ntiles) {
       stage.template load<0, 1>(part * XC_CHUNK_PTS + wp, f.f0);
       stage.template load<1, 4>(part * XC_CHUNK_PTS + wp, f.fg);
@@ -1209,7 +1212,7 @@ static int xc_launch(const XCArgs<T>& a, int nb, hipStream_t st) {
   const size_t lds = XW<T, NP, true>::lds_bytes;
   PSCF_REQUIRE((int)lds <= xc_max_lds(), "pscf_xc: N=%d needs %zu B LDS", a.N, lds);
   PSCF_SET_LDS((xc_wave_kernel<T, NP>), lds);
-  xc_wave_kernel<T, NP><<<nb, XC_THREADS, lds, st>>>(a);
+  xc_wave_kernel<T, NP><<<nb, XW<T, NP, true>::THREADS, lds, st>>>(a);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
 }
@@ -1645,12 +1648,12 @@ static int batch_xc_launch(const void* d_mols, const int* d_order, int nmol, int
   a.tab_off = (int)lds;
   if (DIRECT) lds += xc_shell_bytes(a.nsh_max, a.kp, sizeof(T));
   PSCF_REQUIRE((int)lds <= xc_max_lds(), "pscf_batch_xc: nao %d needs %zu B LDS", max_nao, lds);
+  constexpr int THREADS = WAVE ? XW<T, NP, !DIRECT>::THREADS : XC_THREADS;
   auto run = [&](auto kernel) -> int {
     PSCF_SET_LDS(kernel, lds);
-    kernel<<<dim3(nmol, WAVE && split < XW_PARTS ? XW_PARTS : split), XC_THREADS, lds, st>>>((const BatchMol*)d_mols, d_order, max_nao, d_ctl,
-                                                       (const T*)d_ao, a, (const T*)d_dm, (const T*)d_w, (T)eps,
-                                                       (T*)d_vxc, d_exc, (T*)d_part_v, d_part_e, part_v_elems,
-                                                       part_e_elems);
+    kernel<<<dim3(nmol, WAVE && split < XW_PARTS ? XW_PARTS : split), THREADS, lds, st>>>(
+        (const BatchMol*)d_mols, d_order, max_nao, d_ctl, (const T*)d_ao, a, (const T*)d_dm, (const T*)d_w, (T)eps,
+        (T*)d_vxc, d_exc, (T*)d_part_v, d_part_e, part_v_elems, part_e_elems);
     PSCF_HIP(hipGetLastError());
     return PSCF_OK;
   };

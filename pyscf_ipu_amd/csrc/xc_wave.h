@@ -7,6 +7,14 @@
 // (the points of a k step are the rows row(lg, k) of GEMM 1's accumulators), so
 // Y never goes to LDS.  A wave keeps its whole V in registers, and its whole D
 // operand too where both fit (DLDS otherwise).
+//
+// Measured against workgroup-wide tiles (five barriers per 32 points): 1024
+// 9-heavy molecules, FP32, AO values evaluated in the kernel, one XC pass 9.3 ->
+// 6.0 ms; one 9-heavy molecule at level 1 from a stored block, FP32, 62 -> 32 us.
+// The direct form is bound by the sum of AO evaluation (a third of the time), matrix
+// products (a third; their peak-rate time is 1.9 ms) and LDS traffic, which two
+// waves a SIMD overlap only in part; the stored form in FP64 by matrix products and
+// the functional, HBM time about a third.
 #pragma once
 #include "common.h"
 
@@ -23,13 +31,18 @@ struct XW {
   static constexpr int NB = NP / 16, NK = NP / 4;
   // row stride: 16 consecutive rows spread over all 64 banks
   static constexpr int XS = NP + (STORED && sizeof(T) == 8 ? 2 : 4), XD = NP <= 16 ? 16 : (NP == 48 ? 48 : 80);
-  static constexpr int PHI = (STORED ? 1 : 4) * 16 * XS;
+  // HS = 2: two waves share 16 points, each with half of the columns of X, Y and
+  // V, where all of them (FP64, nao 64: 128 registers of V, 128 of AO values) leave
+  // a wave nothing for the functional; 512 threads, two waves a SIMD (22 molecules
+  // of nao 63, one XC pass: 464 us, 655 with a wave per 16 points)
+  static constexpr int HS = STORED && sizeof(T) == 8 && NP == 64 ? 2 : 1, THREADS = XC_THREADS * HS, NBH = NB / HS;
+  static constexpr int PHI = (STORED ? HS : 4) * 16 * XS;  // HS = 2: phi0 of this tile and the last
   static constexpr bool DLDS = STORED && (sizeof(T) == 8 ? NP >= 48 : NP >= 64);
   static constexpr int ND = DLDS ? 1 : NB * NK;  // D registers
   static constexpr int NV = 2;                   // partial V matrices of a flush
   static constexpr int MAIN0 = 4 * PHI + (DLDS ? NP * XD : 0);
   static constexpr int MAIN = MAIN0 > NV * NP * NP ? MAIN0 : NV * NP * NP;
-  static constexpr int RHO = 2 * 4 * 64, PART = 9 * 64, COEF = 4 * 64;
+  static constexpr int RHO = 2 * HS * 4 * 64, PART = 9 * 64, COEF = HS * 4 * 64;
   static constexpr size_t lds_elems = (size_t)MAIN + RHO + PART + COEF;
   static constexpr size_t lds_bytes = (sizeof(T) * lds_elems + 31) & ~(size_t)31;
 };
@@ -60,7 +73,7 @@ __device__ inline void xw_load_d(const T* __restrict__ dm, int N, T (&dreg)[XW<T
 // overwrites it); in the direct form the padding columns of the wave's Phi = 0.
 template <typename T, int NP, bool STORED>
 __device__ inline void xw_begin(T* smem, const T* __restrict__ dm, int N,
-                                typename XW<T, NP, STORED>::v4 (&vacc)[XW<T, NP, STORED>::NB * XW<T, NP, STORED>::NB]) {
+                                typename XW<T, NP, STORED>::v4 (&vacc)[XW<T, NP, STORED>::NB * XW<T, NP, STORED>::NBH]) {
   typedef XW<T, NP, STORED> L;
   if constexpr (!STORED) {
     T* Phi = smem + (threadIdx.x >> 6) * L::PHI + (threadIdx.x & 63) * L::XS;
@@ -68,31 +81,31 @@ __device__ inline void xw_begin(T* smem, const T* __restrict__ dm, int N,
   }
   if constexpr (L::DLDS) {
     T* Dm = smem + 4 * L::PHI;
-    for (int x = threadIdx.x; x < NP * NP; x += XC_THREADS) {
+    for (int x = threadIdx.x; x < NP * NP; x += L::THREADS) {
       const int i = x / NP, j = x - i * NP;
       Dm[i * L::XD + j] = i < N && j < N ? dm[i * N + j] : T(0);
     }
     __syncthreads();
   }
 #pragma unroll
-  for (int u = 0; u < L::NB * L::NB; ++u) vacc[u] = (typename L::v4){T(0), T(0), T(0), T(0)};
+  for (int u = 0; u < L::NB * L::NBH; ++u) vacc[u] = (typename L::v4){T(0), T(0), T(0), T(0)};
 }
 
 // X = phi0 D of the wave's 16 points (A operand from LDS, read once per k step
 // for all column blocks).
 template <typename T, int NP, bool STORED>
 __device__ inline void xw_gemm1(const T* Phi, const T* Dm, const T (&dreg)[XW<T, NP, STORED>::ND],
-                                typename XMTraits<T>::v4 (&x)[NP / 16]) {
+                                typename XMTraits<T>::v4 (&x)[XW<T, NP, STORED>::NBH], int col0) {
   typedef XW<T, NP, STORED> L;
   const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
 #pragma unroll
-  for (int cb = 0; cb < L::NB; ++cb) x[cb] = (typename L::v4){T(0), T(0), T(0), T(0)};
+  for (int cb = 0; cb < L::NBH; ++cb) x[cb] = (typename L::v4){T(0), T(0), T(0), T(0)};
 #pragma unroll
   for (int k = 0; k < L::NK; ++k) {
     const T av = Phi[li * L::XS + 4 * k + lg];
 #pragma unroll
-    for (int cb = 0; cb < L::NB; ++cb)
-      x[cb] = XMTraits<T>::mfma(av, L::DLDS ? Dm[(4 * k + lg) * L::XD + 16 * cb + li] : dreg[L::DLDS ? 0 : cb * L::NK + k],
+    for (int cb = 0; cb < L::NBH; ++cb)
+      x[cb] = XMTraits<T>::mfma(av, L::DLDS ? Dm[(4 * k + lg) * L::XD + col0 + 16 * cb + li] : dreg[L::DLDS ? 0 : cb * L::NK + k],
                                 x[cb]);
   }
 }
@@ -101,16 +114,17 @@ __device__ inline void xw_gemm1(const T* Phi, const T* Dm, const T (&dreg)[XW<T,
 // row(lg, j) of the wave's 16; on return coef[4][16] holds c_0 .. c_3 of the
 // wave's points.  odd alternates from tile to tile: a wave may write the next
 // tile's rho while another still reads this one's.
-template <typename T>
+template <typename T, int HS>
 __device__ inline void xw_point(T (&s)[16], T* rho, T* part, T* coef, int p0, int g, T wt, T eps, double& e_loc) {
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), slot = wave / HS;
   const int li = lane & 15, lg = lane >> 4;
   const T tot = transpose_reduce16_row(s, lane);
-  rho[(li >> 2) * 64 + wave * 16 + XMTraits<T>::row(lg, li & 3)] = tot;
+  rho[((wave % HS) * 4 + (li >> 2)) * 64 + slot * 16 + XMTraits<T>::row(lg, li & 3)] = tot;
   __syncthreads();
+  auto rc = [&](int c, int q) { return HS == 1 ? rho[c * 64 + q] : rho[c * 64 + q] + rho[(4 + c) * 64 + q]; };
   if (wave < 3) {  // part `wave` of the functional (Slater + VWN, B88, LYP) at 64 points
     T r, gam, e = T(0), vr = T(0), vn = T(0);
-    b3lyp_inputs<T>(rho[lane], rho[64 + lane], rho[128 + lane], rho[192 + lane], eps, r, gam);
+    b3lyp_inputs<T>(rc(0, lane), rc(1, lane), rc(2, lane), rc(3, lane), eps, r, gam);
     if (wave == 0)
       b3lyp_part<T, 0>(r, gam, e, vr, vn);
     else if (wave == 1)
@@ -123,18 +137,18 @@ __device__ inline void xw_point(T (&s)[16], T* rho, T* part, T* coef, int p0, in
   }
   __syncthreads();
   if (lane < 16) {
-    const int q = wave * 16 + lane;
+    const int q = slot * 16 + lane;
     T c[4] = {T(0), T(0), T(0), T(0)};
     if (p0 + lane < g) {
       const T e = part[q] + part[3 * 64 + q] + part[6 * 64 + q];
       const T vr = part[64 + q] + part[4 * 64 + q] + part[7 * 64 + q];
       const T vn = part[2 * 64 + q] + part[5 * 64 + q] + part[8 * 64 + q];
-      e_loc += (double)rho[q] * (double)wt * (double)e;
+      if (wave % HS == 0) e_loc += (double)rc(0, q) * (double)wt * (double)e;
       const T f = T(4) * vn * wt;
       c[0] = T(0.5) * vr * wt;
-      c[1] = f * rho[64 + q];
-      c[2] = f * rho[128 + q];
-      c[3] = f * rho[192 + q];
+      c[1] = f * rc(1, q);
+      c[2] = f * rc(2, q);
+      c[3] = f * rc(3, q);
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) coef[k * 16 + lane] = c[k];
@@ -153,23 +167,24 @@ template <typename T, int NP>
 struct XwStored {
   const T* ao;
   int sc, smu, sp, g, N;
-  int moff[NP / 16];
-  __device__ inline void init() {
+  static constexpr int NBH = XW<T, NP, true>::NBH;
+  int moff[NBH];
+  __device__ inline void init(int col0) {
 #pragma unroll
-    for (int b = 0; b < NP / 16; ++b) {
-      const int mu = 16 * b + (int)(threadIdx.x & 15);
+    for (int b = 0; b < NBH; ++b) {
+      const int mu = col0 + 16 * b + (int)(threadIdx.x & 15);
       moff[b] = (mu < N ? mu : N - 1) * smu;
     }
   }
   template <int C0, int C1>
-  __device__ inline void load(int p0, T (&f)[C1 - C0][NP / 16][4]) const {
+  __device__ inline void load(int p0, T (&f)[C1 - C0][NBH][4]) const {
     const int lg = (threadIdx.x & 63) >> 4;
     if (sizeof(T) == 4 && sp == 1 && p0 + 16 <= g) {
       const int po = p0 + 4 * lg;
 #pragma unroll
       for (int c = C0; c < C1; ++c)
 #pragma unroll
-        for (int b = 0; b < NP / 16; ++b) __builtin_memcpy(f[c - C0][b], ao + (c * sc + moff[b] + po), 4 * sizeof(T));
+        for (int b = 0; b < NBH; ++b) __builtin_memcpy(f[c - C0][b], ao + (c * sc + moff[b] + po), 4 * sizeof(T));
     } else {
       int po[4];
 #pragma unroll
@@ -180,7 +195,7 @@ struct XwStored {
 #pragma unroll
       for (int c = C0; c < C1; ++c)
 #pragma unroll
-        for (int b = 0; b < NP / 16; ++b)
+        for (int b = 0; b < NBH; ++b)
 #pragma unroll
           for (int j = 0; j < 4; ++j) f[c - C0][b][j] = ao[c * sc + moff[b] + po[j]];
     }
@@ -190,7 +205,7 @@ struct XwStored {
 // AO registers of the tile at hand, loaded one tile ahead.
 template <typename T, int NP>
 struct XwAO {
-  T f0[1][NP / 16][4], fg[3][NP / 16][4];
+  T f0[1][XW<T, NP, true>::NBH][4], fg[3][XW<T, NP, true>::NBH][4];
 };
 
 // Tiles tile, tile + tstride, ... (64 points each) below tile_end, from a
@@ -200,29 +215,32 @@ template <typename T, int NP>
 __device__ inline void xw_tiles_stored(const XCArgs<T>& a, T* smem, int tile, int tstride, int tile_end, int next,
                                        const XwStored<T, NP>& st, XwAO<T, NP>& ao,
                                        const T (&dreg)[XW<T, NP, true>::ND],
-                                       typename XMTraits<T>::v4 (&vacc)[XW<T, NP, true>::NB * XW<T, NP, true>::NB],
+                                       typename XMTraits<T>::v4 (&vacc)[XW<T, NP, true>::NB * XW<T, NP, true>::NBH],
                                        double& e_loc) {
   typedef XW<T, NP, true> L;
-  constexpr int NB = L::NB;
+  constexpr int NB = L::NB, NBH = L::NBH, HS = L::HS;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int li = lane & 15, lg = lane >> 4;
-  T* Phi = smem + wave * L::PHI;
+  const int li = lane & 15, lg = lane >> 4, slot = wave / HS, col0 = wave % HS * NBH * 16;
   const T* Dm = smem + 4 * L::PHI;
   T* rho = smem + L::MAIN;
   T* part = rho + L::RHO;
   T* coef = part + L::PART + wave * 64;
   for (int odd = 0; tile < tile_end; tile += tstride, odd ^= 1) {
-    const int p0 = tile * 64 + wave * 16;
+    const int p0 = tile * 64 + slot * 16;
+    T* Phi = smem + slot * L::PHI + (HS == 2 ? odd * 16 * L::XS : 0);
     const T wt = lane < 16 && p0 + lane < a.g ? a.w[p0 + lane] : T(0);
     xw_fence();  // the last tile's reads of Phi and coef
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
+    for (int b = 0; b < NBH; ++b)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) Phi[XMTraits<T>::row(lg, j) * L::XS + 16 * b + li] = ao.f0[0][b][j];
-    xw_fence();
+      for (int j = 0; j < 4; ++j) Phi[XMTraits<T>::row(lg, j) * L::XS + col0 + 16 * b + li] = ao.f0[0][b][j];
+    if constexpr (HS == 2)
+      __syncthreads();  // the other wave's half
+    else
+      xw_fence();
     {
-      typename L::v4 x[NB];
-      xw_gemm1<T, NP, true>(Phi, Dm, dreg, x);
+      typename L::v4 x[NBH];
+      xw_gemm1<T, NP, true>(Phi, Dm, dreg, x, col0);
       T s[16];
 #pragma unroll
       for (int c = 0; c < 4; ++c)
@@ -230,40 +248,41 @@ __device__ inline void xw_tiles_stored(const XCArgs<T>& a, T* smem, int tile, in
         for (int j = 0; j < 4; ++j) {
           T v = T(0);
 #pragma unroll
-          for (int b = 0; b < NB; ++b) v += x[b][j] * (c == 0 ? ao.f0[0][b][j] : ao.fg[c > 0 ? c - 1 : 0][b][j]);
+          for (int b = 0; b < NBH; ++b) v += x[b][j] * (c == 0 ? ao.f0[0][b][j] : ao.fg[c > 0 ? c - 1 : 0][b][j]);
           s[c * 4 + j] = v;
         }
-      xw_point<T>(s, rho + odd * 4 * 64, part, coef, p0, a.g, wt, a.eps, e_loc);
+      xw_point<T, HS>(s, rho + odd * HS * 4 * 64, part, coef, p0, a.g, wt, a.eps, e_loc);
     }
-    T y[NB][4];
+    T y[NBH][4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       T c[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) c[q] = coef[q * 16 + XMTraits<T>::row(lg, j)];
 #pragma unroll
-      for (int b = 0; b < NB; ++b)
+      for (int b = 0; b < NBH; ++b)
         y[b][j] = c[0] * ao.f0[0][b][j] + c[1] * ao.fg[0][b][j] + c[2] * ao.fg[1][b][j] + c[3] * ao.fg[2][b][j];
     }
     const int nt = tile + tstride < tile_end ? tile + tstride : next;
-    T fn[1][NB][4];
+    T fn[1][NBH][4];
     __builtin_amdgcn_sched_barrier(0);
     if (nt >= 0) {
-      st.template load<0, 1>(nt * 64 + wave * 16, fn);
-      st.template load<1, 4>(nt * 64 + wave * 16, ao.fg);
+      st.template load<0, 1>(nt * 64 + slot * 16, fn);
+      st.template load<1, 4>(nt * 64 + slot * 16, ao.fg);
     }
     __builtin_amdgcn_sched_barrier(0);
     // GEMM 2: V[mu][nu] += sum_p phi0[p][mu] Y[p][nu]
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int m = 0; m < NB; ++m)
+      for (int m = 0; m < NB; ++m) {
+        const T f0 = HS == 2 ? Phi[XMTraits<T>::row(lg, j) * L::XS + 16 * m + li] : ao.f0[0][m % NBH][j];
 #pragma unroll
-        for (int n = 0; n < NB; ++n)
-          vacc[m * NB + n] = XMTraits<T>::mfma(ao.f0[0][m][j], y[n][j], vacc[m * NB + n]);
+        for (int n = 0; n < NBH; ++n) vacc[m * NBH + n] = XMTraits<T>::mfma(f0, y[n][j], vacc[m * NBH + n]);
+      }
     if (nt >= 0) {
 #pragma unroll
-      for (int b = 0; b < NB; ++b)
+      for (int b = 0; b < NBH; ++b)
 #pragma unroll
         for (int j = 0; j < 4; ++j) ao.f0[0][b][j] = fn[0][b][j];
     }
@@ -320,7 +339,7 @@ __device__ inline void xw_tiles_direct(const XCArgs<T>& a, T* smem, int tile, in
     xw_fence();
     {
       typename L::v4 x[NB];
-      xw_gemm1<T, NP, false>(Phi, nullptr, dreg, x);
+      xw_gemm1<T, NP, false>(Phi, nullptr, dreg, x, 0);
       T s[16];
 #pragma unroll
       for (int c = 0; c < 4; ++c)
@@ -332,7 +351,7 @@ __device__ inline void xw_tiles_direct(const XCArgs<T>& a, T* smem, int tile, in
           for (int b = 0; b < NB; ++b) v += x[b][j] * f[16 * b];
           s[c * 4 + j] = v;
         }
-      xw_point<T>(s, rho + odd * 4 * 64, part, coef, p0, a.g, wt, a.eps, e_loc);
+      xw_point<T, 1>(s, rho + odd * 4 * 64, part, coef, p0, a.g, wt, a.eps, e_loc);
     }
     // GEMM 2: V[mu][nu] += sum_p phi0[p][mu] Y[p][nu], points 4 k + lg
 #pragma unroll
@@ -359,28 +378,29 @@ __device__ inline void xw_tiles_direct(const XCArgs<T>& a, T* smem, int tile, in
 // of i, j < N to out.  Begins and ends with a barrier; overwrites Phi and D.
 template <typename T, int NP, bool STORED, class Out>
 __device__ inline void xw_flush(T* smem, int N,
-                                const typename XMTraits<T>::v4 (&vacc)[XW<T, NP, STORED>::NB * XW<T, NP, STORED>::NB],
+                                const typename XMTraits<T>::v4 (&vacc)[XW<T, NP, STORED>::NB * XW<T, NP, STORED>::NBH],
                                 Out out) {
   typedef XW<T, NP, STORED> L;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lg = lane >> 4;
-  T* V = smem + (wave & 1) * NP * NP;
+  const int slot = wave / L::HS, col0 = wave % L::HS * L::NBH * 16;
+  T* V = smem + (slot & 1) * NP * NP + col0;
   __syncthreads();
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    if ((wave >> 1) == h) {
+    if ((slot >> 1) == h) {
 #pragma unroll
       for (int m = 0; m < L::NB; ++m)
 #pragma unroll
-        for (int n = 0; n < L::NB; ++n)
+        for (int n = 0; n < L::NBH; ++n)
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             T* v = V + (16 * m + XMTraits<T>::row(lg, j)) * NP + 16 * n + li;
-            *v = h ? *v + vacc[m * L::NB + n][j] : vacc[m * L::NB + n][j];
+            *v = h ? *v + vacc[m * L::NBH + n][j] : vacc[m * L::NBH + n][j];
           }
     }
     __syncthreads();
   }
-  for (int x = threadIdx.x; x < N * N; x += XC_THREADS) {
+  for (int x = threadIdx.x; x < N * N; x += L::THREADS) {
     const int i = x / N, j = x - i * N;
     out(i, j, smem[i * NP + j] + smem[NP * NP + i * NP + j], smem[j * NP + i] + smem[NP * NP + j * NP + i]);
   }
