@@ -287,12 +287,13 @@ int pscf_batch_becke(int dtype, const void* d_mols, const int* d_ptmol, const in
 int pscf_batch_ao(int dtype, const void* d_mols, const int* d_ptmol, const double* d_coords, int64_t G,
                   const int* d_atm, const int* d_bas, const double* d_env, void* d_ao, void* stream);
 /* E_xc (d_exc[m]) and V_xc of the active molecules d_order[0..nmol)
- * (nanoDFT.py:105-123), grid tiles of `tile` points (32, or 64 in FP32);
+ * (nanoDFT.py:105-123); tile (32, or 64 in FP32) is checked but chooses
+ * nothing any more, the kernels' tiles having one shape;
  * max_nao bounds the nao of these molecules (it sizes the LDS and the tile
  * shapes; a larger molecule gets NaN).  Each molecule's grid is cut into
  * chunks of PSCF_XC_CHUNK_PTS points whose V and E_xc partials are summed in
  * chunk order, so the result does not depend on `split` (workgroups sharing a
- * molecule's chunks).  Chunk partials go to d_part_v (part_v_elems >=
+ * molecule's chunks; a launch may use more).  Chunk partials go to d_part_v (part_v_elems >=
  * nchunk_max * nmol * max_nao^2 elements of dtype) and d_part_e (part_e_elems
  * >= nchunk_max * nmol doubles), nchunk_max = ceil(largest grid /
  * PSCF_XC_CHUNK_PTS); a molecule whose chunks do not fit gets NaN. */
