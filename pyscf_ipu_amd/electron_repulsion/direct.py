@@ -144,11 +144,12 @@ def prepare_integrals_2_inputs(mol):
 prepare_electron_repulsion_integrals = prepare_integrals_2_inputs
 
 
+def _mol_host(mol):
+    return mol._atm.astype(np.int32), mol._bas.astype(np.int32), mol._env.astype(np.float64)
+
+
 def _mol_device(mol):
-    atm = device.to_dev(mol._atm.astype(np.int32))
-    bas = device.to_dev(mol._bas.astype(np.int32))
-    env = device.to_dev(mol._env.astype(np.float64))
-    return atm, bas, env
+    return tuple(device.upload_many(*_mol_host(mol)))
 
 
 def eri_quartets(mol, quartets: np.ndarray, dtype: str = "fp32") -> torch.Tensor:
@@ -286,17 +287,22 @@ def eri_s8(mol, dtype: str = "fp64", out: torch.Tensor = None, dev_mol=None, dev
     """All unique ERIs in PySCF's aosym='s8' packing, on the device.
     `dev_pairs` = (device pairs, counts) of shell_pairs_by_class, if uploaded."""
     tdt, code, _ = device.DTYPES[dtype]
-    if any(mol._bas[:, ANG_OF] > 1):
+    if (mol._bas[:, ANG_OF] > 1).any():
         raise _lib.HIPError("eri_s8: only s and p shells are supported")
+    # one copy for what is not on the device yet: each from pageable memory
+    # costs 10 us and more
+    if dev_pairs is None:
+        pairs, counts = shell_pairs_by_class(mol)
+        if dev_mol is None:
+            *dev_mol, dp = device.upload_many(*_mol_host(mol), pairs)
+        else:
+            dp = device.to_dev(pairs)
+    else:
+        dp, counts = dev_pairs
     atm, bas, env = dev_mol if dev_mol is not None else _mol_device(mol)
     nao = mol.nao_nr()
     if out is None:
         out = device.empty(s8_size(nao), tdt)
-    if dev_pairs is None:
-        pairs, counts = shell_pairs_by_class(mol)
-        dp = device.to_dev(pairs)
-    else:
-        dp, counts = dev_pairs
     cc = (ctypes.c_int * 3)(*counts)
     _lib.call("pscf_eri_s8", code, device.ptr(atm), len(mol._atm), device.ptr(bas), len(mol._bas), device.ptr(env),
               device.ptr(dp), cc, nao, device.ptr(out), device.stream())

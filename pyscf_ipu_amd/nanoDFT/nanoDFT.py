@@ -474,31 +474,28 @@ def grad(mol, coords, weight, mo_coeff, mo_energy):
     nocc = mol.nelectron // 2
     mo_coeff = np.asarray(mo_coeff, dtype=np.float64)
     e_occ = np.asarray(mo_energy, dtype=np.float64)[:nocc]
-    c_occ = device.to_dev(np.ascontiguousarray(mo_coeff[:, :nocc]))
-    c2 = device.to_dev(np.ascontiguousarray(2.0 * mo_coeff[:, :nocc]))           # 2 C_occ
-    c2e = device.to_dev(np.ascontiguousarray(2.0 * mo_coeff[:, :nocc] * e_occ))  # 2 C_occ e_occ
+    pairs, counts = direct.shell_pairs_by_class(mol)
+    # all inputs in one copy; c2 = 2 C_occ, c2e = 2 C_occ e_occ
+    atm, bas, env, dp, coords_d, w_d, c_occ, c2, c2e = device.upload_many(
+        *direct._mol_host(mol), pairs, np.asarray(coords, dtype=np.float64), np.asarray(weight, dtype=np.float64),
+        mo_coeff[:, :nocc], 2.0 * mo_coeff[:, :nocc], 2.0 * mo_coeff[:, :nocc] * e_occ)
     f64 = torch.float64
     dm0, dme0 = device.empty((N, N), f64), device.empty((N, N), f64)
     P, st = device.ptr, device.stream()
     G_F64 = 3
     _lib.call("pscf_gemm", G_F64, 1, 0, 1, 0, N, N, nocc, P(c2), nocc, P(c_occ), nocc, P(dm0), N, 1, st)
     _lib.call("pscf_gemm", G_F64, 1, 0, 1, 0, N, N, nocc, P(c2e), nocc, P(c_occ), nocc, P(dme0), N, 1, st)
-    atm, bas, env = direct._mol_device(mol)
     g_dev = device.zeros((natm, 3), f64)
     _lib.call("pscf_grad_int1e", P(atm), natm, P(bas), mol.nbas, P(env), N, P(dm0), P(dme0), P(g_dev), st)
-    pairs, counts = direct.shell_pairs_by_class(mol)
-    dp = device.to_dev(pairs)
     _lib.call("pscf_grad_eri", P(atm), natm, P(bas), mol.nbas, P(env), P(dp), (ctypes.c_int * 3)(*counts), N,
               P(dm0), HYB_B3LYP, P(g_dev), st)
-    coords_d = device.to_dev(np.ascontiguousarray(coords, dtype=np.float64))
-    w_d = device.to_dev(np.ascontiguousarray(weight, dtype=np.float64))
     g = len(w_d)
     wsb = _lib.lib().pscf_grad_xc_workspace_bytes(N, mol.nbas, g)
     ws = device.workspace(wsb)
     _lib.call("pscf_grad_xc", P(coords_d), P(w_d), g, P(atm), natm, P(bas), mol.nbas, P(env), N, P(dm0),
               EPSILON_B3LYP, P(ws), wsb, P(g_dev), st)
-    out = g_dev.cpu().numpy()
-    return out + grad_nuc(mol.atom_charges(), mol.atom_coords())
+    nuc = grad_nuc(mol.atom_charges(), mol.atom_coords())  # while the kernels run
+    return g_dev.cpu().numpy() + nuc
 
 
 def structure_optimization(opts, steps: int = 20, mol_str: str = None):
