@@ -5,8 +5,8 @@
 // recurrence CINTg0_2e_2d :1475-1600, primitive loop CINT2e_loop_nopt
 // :2452-2723, one shell quartet per IPU tile).  The packed s8 arrays come from
 // the shell-pair engine of eri_pairs.h, the gradient from eri_grad.h.  The same
-// quadrature as libcint's, one contracted shell quartet per lane, serves
-// explicit quartet lists (pscf_eri_quartets):
+// quadrature as libcint's, one contracted shell quartet per lane, serves FP64
+// batches and explicit quartet lists (pscf_eri_quartets):
 //   * Boys F_m(T) from a Taylor table staged in LDS (F_0..F_14 on a 0.1 grid
 //     up to T = 39.9, asymptote above),
 //   * Rys roots/weights from the Boys moments in closed form (1-3 roots), FP64,
@@ -605,6 +605,80 @@ __global__ void __launch_bounds__(256) int1e_kernel(const int* __restrict__ atm,
 }
 
 // ------------------------------------------------------------ batched form ---
+// ERIs of FP64 batches, one contracted quartet per lane (shell_quartet): a
+// workgroup takes the chunk of <= 256 quartets of class (X, Y) that its work
+// entry names or, without a list, chunks part, part + per, ... of its molecule.
+// FP64 batches do not take the shell-pair engine, although its ERIs differ by
+// rounding only and take 3 of 54 ms less (96 molecules of 1-9 heavy atoms): a molecule
+// that does not converge amplifies a last bit of its integrals by up to seven
+// orders within 20 iterations, and FP64 is the form that results are compared
+// and reproduced with.
+template <int X, int Y>
+__global__ void __launch_bounds__(256) eri_s8_rys_batch_kernel(
+    const BatchMol* __restrict__ mols, const int* __restrict__ work, const int* __restrict__ order, int per,
+    const int* __restrict__ atm, const int* __restrict__ bas, const double* __restrict__ env,
+    const int* __restrict__ shell_ao, const int* __restrict__ shl_sorted, double* __restrict__ out, int div) {
+  constexpr int LI = PairL<X>::a, LJ = PairL<X>::b, LK = PairL<Y>::a, LL = PairL<Y>::b;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int mo = blockIdx.x / per, part = blockIdx.x - mo * per;
+  const int m = work ? work[2 * blockIdx.x] : (order ? order[mo] : mo);
+  const BatchMol M = mols[m];
+  const int ns = (int)M.ns, np = (int)M.np;
+  const int64_t nx = ep_count(X, ns, np), ny = ep_count(Y, ns, np);
+  const bool tri_launch = (X == Y);
+  const int64_t total = tri_launch ? tri(nx) : nx * ny;
+  const int64_t q0 = work ? (int64_t)work[2 * blockIdx.x + 1] : (int64_t)part * 256;
+  if (q0 >= total) return;
+  double* tab = reinterpret_cast<double*>(smem);
+  for (int i = threadIdx.x; i < BOYS_NT * BOYS_NM; i += blockDim.x) tab[i] = g_boys[i];
+  __syncthreads();
+  const EpMol E{atm, bas, env, shell_ao, nullptr, shl_sorted + M.shl0, ns};
+  const int64_t step = work ? total : (int64_t)per * 256;
+  for (int64_t q = q0 + threadIdx.x; q < total; q += step) {
+    int64_t a, b;
+    if (tri_launch) {
+      a = (int64_t)((sqrt(8.0 * (double)q + 1.0) - 1.0) * 0.5);
+      while (tri(a + 1) <= q) ++a;
+      while (tri(a) > q) --a;
+      b = q - tri(a);
+    } else {
+      a = q / ny;
+      b = q - a * ny;
+    }
+    int i, j, k, l;
+    ep_pair<X>(E, 0, (int)a, i, j);
+    ep_pair<Y>(E, 0, (int)b, k, l);
+    // shell_ao holds each shell's first AO within its molecule
+    const ShellD A = load_shell(atm, bas, env, shell_ao, i), B = load_shell(atm, bas, env, shell_ao, j);
+    const ShellD C = load_shell(atm, bas, env, shell_ao, k), D = load_shell(atm, bas, env, shell_ao, l);
+    constexpr int NI = NComp<LI>::v, NJ = NComp<LJ>::v, NK = NComp<LK>::v, NL = NComp<LL>::v;
+    double acc[NI * NJ * NK * NL];
+    shell_quartet<double, double, BoysTerms<double>::v, LI, LJ, LK, LL>(A, B, C, D, tab, acc);
+    const bool diag_bra = (i == j), diag_ket = (k == l), same_pair = tri_launch && (a == b);
+    double* dst = out + M.eri0;
+#pragma unroll
+    for (int fi = 0; fi < NI; ++fi)
+#pragma unroll
+      for (int fj = 0; fj < NJ; ++fj)
+#pragma unroll
+        for (int fk = 0; fk < NK; ++fk)
+#pragma unroll
+          for (int fl = 0; fl < NL; ++fl) {
+            const int64_t p = A.ao0 + fi, qq = B.ao0 + fj, r = C.ao0 + fk, s = D.ao0 + fl;
+            if (diag_bra && qq > p) continue;
+            if (diag_ket && s > r) continue;
+            const int64_t pq = p >= qq ? tri(p) + qq : tri(qq) + p;
+            const int64_t rs = r >= s ? tri(r) + s : tri(s) + r;
+            if (same_pair && rs > pq) continue;
+            const int64_t idx = pq >= rs ? tri(pq) + rs : tri(rs) + pq;
+            double v = acc[((fi * NJ + fj) * NK + fk) * NL + fl];
+            // div: over the element's multiplicity 2^([p==q] + [r==s] + [pq==rs])
+            if (div) v *= 1.0 / (double)(1 << ((p == qq) + (r == s) + (pq == rs)));
+            dst[idx] = v;
+          }
+  }
+}
+
 // gridDim.y workgroups per molecule, one wave per shell pair: S and H_core = T + V.
 __global__ void __launch_bounds__(256) int1e_batch_kernel(const BatchMol* __restrict__ mols,
                                                           const int* __restrict__ atm, const int* __restrict__ bas,
@@ -992,29 +1066,63 @@ extern "C" int pscf_int1e(const int* d_atm, int natm, const int* d_bas, int nbas
   return PSCF_OK;
 }
 
+// Workgroups that share a molecule where a launch enumerates the molecules itself.
+static int mols_per(int nmol) { return (nmol >= 8192 ? 4 : (nmol <= 256 ? 128 : 32768 / nmol)) - 1; }
+
+// FP64 batch ERIs: work lists (h_work, lightest class first) or, if null, every molecule.
+template <int X, int Y>
+static int launch_rys(const BatchMol* mols, const int* work, int nwork, const int* order, int nmol, const int* atm,
+                      const int* bas, const double* env, const int* shell_ao, const int* shl, double* out, int div,
+                      hipStream_t st) {
+  const int per = work ? 1 : mols_per(nmol);
+  const int64_t blocks = work ? nwork : (int64_t)nmol * per;
+  PSCF_REQUIRE(blocks < (1ll << 31), "pscf_batch_eri_s8: too many molecules");
+  if (blocks == 0) return PSCF_OK;
+  eri_s8_rys_batch_kernel<X, Y><<<(unsigned)blocks, 256, sizeof(double) * BOYS_NT * BOYS_NM, st>>>(
+      mols, work, order, per, atm, bas, env, shell_ao, shl, out, div);
+  PSCF_HIP(hipGetLastError());
+  return PSCF_OK;
+}
+static int rys_all(const BatchMol* mols, const int* const* work, const int* nwork, const int* order, int nmol,
+                   const int* atm, const int* bas, const double* env, const int* shell_ao, const int* shl, double* out,
+                   int div, hipStream_t st) {
+  // a class without quartets has an empty list, whose pointer may be null
+  auto run = [&](auto launch, int l) {
+    if (nwork && nwork[l] == 0) return (int)PSCF_OK;
+    return launch(mols, work ? work[l] : nullptr, nwork ? nwork[l] : 0, order, nmol, atm, bas, env, shell_ao, shl, out,
+                  div, st);
+  };
+  int rc = run(launch_rys<0, 0>, 0);
+  if (!rc) rc = run(launch_rys<1, 0>, 1);
+  if (!rc) rc = run(launch_rys<1, 1>, 2);
+  if (!rc) rc = run(launch_rys<2, 0>, 3);
+  if (!rc) rc = run(launch_rys<2, 1>, 4);
+  if (!rc) rc = run(launch_rys<2, 2>, 5);
+  return rc;
+}
+
 // The lists come lightest class first: list l holds class EP_CLASSES - 1 - l.
-template <typename T, int C>
+template <int C>
 static int launch_list(const BatchMol* mols, const int* const* work, const int* nwork, const int* atm, const int* bas,
-                       const double* env, const int* shell_ao, const int* shl, T* out, int div, hipStream_t st) {
+                       const double* env, const int* shell_ao, const int* shl, float* out, int div, hipStream_t st) {
   const int n = nwork[EP_CLASSES - 1 - C];
   if (n == 0) return PSCF_OK;
-  const size_t shm = ep_lds<T, C>();
-  PSCF_SET_LDS((eri_s8_list_kernel<T, C>), shm);
-  eri_s8_list_kernel<T, C><<<(n + EP_GROUP - 1) / EP_GROUP, EP_THREADS, shm, st>>>(
+  const size_t shm = ep_lds<float, C>();
+  PSCF_SET_LDS(eri_s8_list_kernel<C>, shm);
+  eri_s8_list_kernel<C><<<(n + EP_GROUP - 1) / EP_GROUP, EP_THREADS, shm, st>>>(
       mols, work[EP_CLASSES - 1 - C], n, atm, bas, env, shell_ao, shl, out, div);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
 }
 
-template <typename T>
-static int batch_s8_all(const BatchMol* mols, const int* const* work, const int* nwork, const int* atm, const int* bas,
-                        const double* env, const int* shell_ao, const int* shl, T* out, int div, hipStream_t st) {
-  int rc = launch_list<T, 0>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
-  if (!rc) rc = launch_list<T, 1>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
-  if (!rc) rc = launch_list<T, 2>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
-  if (!rc) rc = launch_list<T, 3>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
-  if (!rc) rc = launch_list<T, 4>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
-  if (!rc) rc = launch_list<T, 5>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
+static int lists_all(const BatchMol* mols, const int* const* work, const int* nwork, const int* atm, const int* bas,
+                     const double* env, const int* shell_ao, const int* shl, float* out, int div, hipStream_t st) {
+  int rc = launch_list<0>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_list<1>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_list<2>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_list<3>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_list<4>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_list<5>(mols, work, nwork, atm, bas, env, shell_ao, shl, out, div, st);
   return rc;
 }
 
@@ -1030,39 +1138,38 @@ static int batch_eri_s8_any(int dtype, const void* d_mols, int nmol, const int* 
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == PSCF_F64)
-    return batch_s8_all<double>((const BatchMol*)d_mols, h_work, h_nwork, d_atm, d_bas, d_env, d_shell_ao,
-                                d_shl_sorted, (double*)d_out, div, st);
-  return batch_s8_all<float>((const BatchMol*)d_mols, h_work, h_nwork, d_atm, d_bas, d_env, d_shell_ao, d_shl_sorted,
-                             (float*)d_out, div, st);
+    return rys_all((const BatchMol*)d_mols, h_work, h_nwork, nullptr, nmol, d_atm, d_bas, d_env, d_shell_ao,
+                   d_shl_sorted, (double*)d_out, div, st);
+  return lists_all((const BatchMol*)d_mols, h_work, h_nwork, d_atm, d_bas, d_env, d_shell_ao, d_shl_sorted,
+                   (float*)d_out, div, st);
 }
 
 // Tiles: the heavy classes have few pairs per molecule, so theirs are small; a
 // small batch takes smaller tiles still, to spread over the chip.
-template <typename T, int C>
+template <int C>
 static int launch_mols(const BatchMol* mols, const int* order, int nmol, const int* atm, const int* bas,
-                       const double* env, const int* shell_ao, const int* shl, T* out, int div, hipStream_t st) {
+                       const double* env, const int* shell_ao, const int* shl, float* out, int div, hipStream_t st) {
   static const int big[EP_CLASSES][2] = {{4, 64}, {8, 64}, {16, 64}, {16, 64}, {32, 64}, {32, 64}};
   static const int small[EP_CLASSES][2] = {{4, 16}, {4, 16}, {16, 32}, {8, 32}, {16, 32}, {16, 32}};
   const int* tile = nmol >= 32 ? big[C] : small[C];
-  const int per = (nmol >= 8192 ? 4 : (nmol <= 256 ? 128 : 32768 / nmol)) - 1;
+  const int per = mols_per(nmol);
   PSCF_REQUIRE((int64_t)nmol * per < (1ll << 31), "pscf_batch_eri_s8_all: too many molecules");
-  const size_t shm = ep_lds<T, C>();
-  PSCF_SET_LDS((eri_s8_mols_kernel<T, C>), shm);
-  eri_s8_mols_kernel<T, C><<<(unsigned)nmol * per, EP_THREADS, shm, st>>>(mols, order, per, atm, bas, env, shell_ao,
+  const size_t shm = ep_lds<float, C>();
+  PSCF_SET_LDS(eri_s8_mols_kernel<C>, shm);
+  eri_s8_mols_kernel<C><<<(unsigned)nmol * per, EP_THREADS, shm, st>>>(mols, order, per, atm, bas, env, shell_ao,
                                                                           shl, tile[0], tile[1], out, div);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
 }
 
-template <typename T>
 static int mols_all(const BatchMol* mols, const int* order, int nmol, const int* atm, const int* bas, const double* env,
-                    const int* shell_ao, const int* shl, T* out, int div, hipStream_t st) {
-  int rc = launch_mols<T, 0>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
-  if (!rc) rc = launch_mols<T, 1>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
-  if (!rc) rc = launch_mols<T, 2>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
-  if (!rc) rc = launch_mols<T, 3>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
-  if (!rc) rc = launch_mols<T, 4>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
-  if (!rc) rc = launch_mols<T, 5>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
+                    const int* shell_ao, const int* shl, float* out, int div, hipStream_t st) {
+  int rc = launch_mols<0>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_mols<1>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_mols<2>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_mols<3>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_mols<4>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
+  if (!rc) rc = launch_mols<5>(mols, order, nmol, atm, bas, env, shell_ao, shl, out, div, st);
   return rc;
 }
 
@@ -1076,10 +1183,10 @@ extern "C" int pscf_batch_eri_s8_all(int dtype, const void* d_mols, const int* d
   if (rc) return rc;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == PSCF_F64)
-    return mols_all<double>((const BatchMol*)d_mols, d_order, nmol, d_atm, d_bas, d_env, d_shell_ao, d_shl_sorted,
-                            (double*)d_out, div, st);
-  return mols_all<float>((const BatchMol*)d_mols, d_order, nmol, d_atm, d_bas, d_env, d_shell_ao, d_shl_sorted,
-                         (float*)d_out, div, st);
+    return rys_all((const BatchMol*)d_mols, nullptr, nullptr, d_order, nmol, d_atm, d_bas, d_env, d_shell_ao,
+                   d_shl_sorted, (double*)d_out, div, st);
+  return mols_all((const BatchMol*)d_mols, d_order, nmol, d_atm, d_bas, d_env, d_shell_ao, d_shl_sorted,
+                  (float*)d_out, div, st);
 }
 
 extern "C" int pscf_batch_eri_s8(int dtype, const void* d_mols, int nmol, const int* const* h_work,
@@ -1127,9 +1234,10 @@ extern "C" int pscf_batch_chunks(const int64_t* d_first, int n, int size, int* d
   return PSCF_OK;
 }
 
-// Nuclear repulsion of every molecule, one wave per molecule (256 molecules: 147 ->
-// 19 us; a thread each ran through all atom pairs), atom pairs
-// i > j in order (nanoDFT.py: mol.energy_nuc()).
+// Nuclear repulsion of every molecule, one wave per molecule, atom pairs i > j
+// in order (nanoDFT.py: mol.energy_nuc()): the lanes form the terms of 64 j at
+// once, which are then added one after the other, so that the sum has the bits
+// of a plain loop (a thread per molecule, 256 molecules: 132 us, 31 now).
 __global__ void __launch_bounds__(256) enuc_kernel(const BatchMol* __restrict__ mols, int nmol,
                                                    const int* __restrict__ atm, const double* __restrict__ env,
                                                    double* __restrict__ out) {
@@ -1140,14 +1248,15 @@ __global__ void __launch_bounds__(256) enuc_kernel(const BatchMol* __restrict__ 
   for (int i = 1; i < na; ++i) {
     const double* Ri = env + atm[(a0 + i) * ATM_SLOTS + 1];
     const double Zi = (double)atm[(a0 + i) * ATM_SLOTS];
-    for (int j = lane; j < i; j += 64) {
+    for (int j0 = 0; j0 < i; j0 += 64) {
+      const int n = min(i - j0, 64), j = j0 + min(lane, n - 1);
       const double* Rj = env + atm[(a0 + j) * ATM_SLOTS + 1];
       const double dx = Ri[0] - Rj[0], dy = Ri[1] - Rj[1], dz = Ri[2] - Rj[2];
-      e += Zi * (double)atm[(a0 + j) * ATM_SLOTS] / sqrt(dx * dx + dy * dy + dz * dz);
+      const double t = Zi * (double)atm[(a0 + j) * ATM_SLOTS] / sqrt(dx * dx + dy * dy + dz * dz);
+      for (int k = 0; k < n; ++k) e += __shfl(t, k);
     }
   }
-  e = wave_sum_last(e);
-  if (lane == 63) out[m] = e;
+  if (lane == 0) out[m] = e;
 }
 
 extern "C" int pscf_batch_enuc(const void* d_mols, int nmol, const int* d_atm, const double* d_env, double* d_enuc,

@@ -1,5 +1,5 @@
 // Packed s8 ERIs from shell-pair primitive lists (McMurchie-Davidson), the
-// engine of pscf_eri_s8 and pscf_batch_eri_s8_all.
+// engine of pscf_eri_s8 and, in FP32, of the batched entries.
 //
 // The ERI work is bound by VALU issue, so the layout removes what a
 // lane-per-contracted-quartet Rys form spends beyond the arithmetic itself:
@@ -796,27 +796,27 @@ __host__ __device__ inline int ep_count(int X, int ns, int np) {
   return X == 0 ? ns * (ns + 1) / 2 : (X == 1 ? ns * np : np * (np + 1) / 2);
 }
 
-// All molecules of a batch, one class: `per` workgroups share a molecule's
+// All molecules of an FP32 batch, one class: `per` workgroups share a molecule's
 // tiles.  `per` is odd: neighbouring workgroups go to different XCDs, and with
 // an even count the parts of molecules with few tiles all fell on the same few
 // XCDs (1024 nine-heavy-atom molecules: 69 ms with 32, 51 ms with 31).  The
 // classes have a launch each: in one launch they would all take the registers
 // and LDS of the heaviest (74 ms).
-template <typename T, int C>
+template <int C>
 __global__ void __launch_bounds__(EP_THREADS, 2) eri_s8_mols_kernel(
     const BatchMol* __restrict__ mols, const int* __restrict__ order, int per, const int* __restrict__ atm,
     const int* __restrict__ bas, const double* __restrict__ env, const int* __restrict__ shell_ao,
-    const int* __restrict__ shl, int na, int nb, T* __restrict__ out, int div) {
-  using Run = EpRun<T, C, sizeof(T) == 8>;
+    const int* __restrict__ shl, int na, int nb, float* __restrict__ out, int div) {
+  using Run = EpRun<float, C, false>;
   extern __shared__ __align__(16) unsigned char smem[];
   const int mo = blockIdx.x / per, part = blockIdx.x - mo * per;
   const BatchMol B = mols[order ? order[mo] : mo];
   const int ns = (int)B.ns, np = (int)B.np, nx = ep_count(Run::X, ns, np), ny = ep_count(Run::Y, ns, np);
   const int64_t tiles = Run::tiles(nx, ny, na, nb);
   if (part >= tiles) return;
-  auto* tab = reinterpret_cast<typename EpTable<T>::type*>(smem);
+  auto* tab = reinterpret_cast<float4*>(smem);
   ep_stage_table<Run::X + Run::Y>(tab, g_boys);
-  auto& sh = *reinterpret_cast<EpShared<T, Run::X, Run::Y>*>(smem + EpTable<T>::bytes);
+  auto& sh = *reinterpret_cast<EpShared<float, Run::X, Run::Y>*>(smem + EpTable<float>::bytes);
   const EpMol M{atm, bas, env, shell_ao, nullptr, shl + B.shl0, ns};
   for (int64_t t = part; t < tiles; t += per) Run::tile(M, 0, 0, nx, ny, na, nb, t, tab, sh, out + B.eri0, div != 0);
 }
@@ -827,17 +827,17 @@ __global__ void __launch_bounds__(EP_THREADS, 2) eri_s8_mols_kernel(
 // EP_GROUP entries and merges neighbours, so that a range of quartets is a few
 // whole rows and a part of a row at either end.
 constexpr int EP_LIST = 256, EP_GROUP = 16;
-template <typename T, int C>
+template <int C>
 __global__ void __launch_bounds__(EP_THREADS, 2) eri_s8_list_kernel(
     const BatchMol* __restrict__ mols, const int* __restrict__ work, int nwork, const int* __restrict__ atm,
     const int* __restrict__ bas, const double* __restrict__ env, const int* __restrict__ shell_ao,
-    const int* __restrict__ shl, T* __restrict__ out, int div) {
-  using Run = EpRun<T, C, sizeof(T) == 8>;
+    const int* __restrict__ shl, float* __restrict__ out, int div) {
+  using Run = EpRun<float, C, false>;
   constexpr bool TRI = Run::X == Run::Y;
   extern __shared__ __align__(16) unsigned char smem[];
-  auto* tab = reinterpret_cast<typename EpTable<T>::type*>(smem);
+  auto* tab = reinterpret_cast<float4*>(smem);
   ep_stage_table<Run::X + Run::Y>(tab, g_boys);
-  auto& sh = *reinterpret_cast<EpShared<T, Run::X, Run::Y>*>(smem + EpTable<T>::bytes);
+  auto& sh = *reinterpret_cast<EpShared<float, Run::X, Run::Y>*>(smem + EpTable<float>::bytes);
   const int w1 = min((int)(blockIdx.x + 1) * EP_GROUP, nwork);
   for (int w = blockIdx.x * EP_GROUP; w < w1;) {
     const int m = work[2 * w];
@@ -867,12 +867,10 @@ __global__ void __launch_bounds__(EP_THREADS, 2) eri_s8_list_kernel(
         c1 = TRI ? r1 : ncol;
       }
       // rows are bra pairs in the triangle, else the lanes' ket pairs
-      for (int i = 0; i < Run::parts; ++i) {
-        if (TRI)
-          Run::rect(M, 0, 0, (int)r, (int)r1, (int)c0, (int)c1, i, tab, sh, out + B.eri0, div != 0);
-        else
-          Run::rect(M, 0, 0, (int)c0, (int)c1, (int)r, (int)r1, i, tab, sh, out + B.eri0, div != 0);
-      }
+      if (TRI)
+        Run::rect(M, 0, 0, (int)r, (int)r1, (int)c0, (int)c1, 0, tab, sh, out + B.eri0, div != 0);
+      else
+        Run::rect(M, 0, 0, (int)c0, (int)c1, (int)r, (int)r1, 0, tab, sh, out + B.eri0, div != 0);
     }
   }
 }

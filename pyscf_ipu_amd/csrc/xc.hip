@@ -154,8 +154,7 @@ struct XCArgs {
 };
 
 // ---- MFMA path ------------------------------------------------------------------
-// Workgroup-wide tiles, for FP64 batches above nao 48 with AO values evaluated in
-// the kernel (everything else: xc_wave.h).
+// Workgroup-wide tiles, for FP64 batches (everything else: xc_wave.h).
 // Per tile of XT points (32), with the tile's AO values and
 // gradients staged in LDS as Phi[c][p][nu] (row stride XS = NP + 4, NP = N
 // rounded up to 16):
@@ -209,6 +208,44 @@ struct XTile {
 
 template <typename T, int XT, int NP>
 using XVacc = typename XMTraits<T>::v4[XTile<XT, NP>::NBW];
+
+// Staging of a tile's AO values and gradients into Phi[c][p][mu] (row stride
+// XS), mu < N; padding columns are left as they are.
+// Stored form: read from ao[c * sc + mu * smu + p * sp] in HBM.  Each wave
+// moves one (c, mu) row of XT points per 64 / XT rows and instruction (lanes
+// walk points, coalesced), eight rows' loads in flight before their LDS
+// stores; c = row / N comes from three compares, not a division.
+template <typename T, int XT, int NP>
+struct XcStageStored {
+  const T* ao;
+  int sc, smu, sp, g, N;
+  __device__ inline void load(int) {}
+  __device__ inline void operator()(T* Phi, int p0, int /*p0_next*/) {
+    constexpr int XS = XTile<XT, NP>::XS;
+    constexpr int RPW = 64 / XT;  // rows per wave instruction
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int p = lane % XT, sub = lane / XT, nrow = 4 * N, rstride = 4 * RPW;
+    const int pt = p0 + p;
+    const bool in = pt < g;
+    const int ptoff = pt * sp;
+    for (int base = wave * RPW + sub; base < nrow; base += 8 * rstride) {
+      T v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int row = base + u * rstride;
+        const int c = (row >= N) + (row >= 2 * N) + (row >= 3 * N), mu = row - c * N;
+        v[u] = (row < nrow && in) ? ao[c * sc + mu * smu + ptoff] : T(0);
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int row = base + u * rstride;
+        const int c = (row >= N) + (row >= 2 * N) + (row >= 3 * N), mu = row - c * N;
+        if (row < nrow) Phi[(c * XT + p) * XS + mu] = v[u];
+      }
+    }
+  }
+};
 
 // One molecule's shells in LDS for the direct form, as records: an s shell,
 // a p shell, or an s shell and the p shell after it on the same atom with the
@@ -677,10 +714,10 @@ __device__ inline bool xc_mol_outside(const BatchMol& Mo, int max_nao, int nsh_m
          (nsh_max > 0 && Mo.nbas > nsh_max);
 }
 
-template <typename T, int XT, int NP>
+template <typename T, int XT, int NP, bool DIRECT>
 __global__ void __launch_bounds__(XC_THREADS) xc_batch_kernel(
     const BatchMol* __restrict__ mols, const int* __restrict__ order, int max_nao, const double* __restrict__ ctl,
-    const T* __restrict__ /*ao*/, XcDirect da, const T* __restrict__ dm, const T* __restrict__ w, T eps,
+    const T* __restrict__ ao, XcDirect da, const T* __restrict__ dm, const T* __restrict__ w, T eps,
     T* __restrict__ vxc, double* __restrict__ exc, T* __restrict__ part_v, double* __restrict__ part_e,
     int64_t part_v_elems, int64_t part_e_elems) {
   static_assert(XC_CHUNK_PTS % XT == 0, "a chunk is a whole number of tiles");
@@ -692,7 +729,7 @@ __global__ void __launch_bounds__(XC_THREADS) xc_batch_kernel(
   const int part = blockIdx.y, nparts = gridDim.y;
   // LDS and tiles were sized for max_nao (and nsh_max shells), offsets are
   // 32-bit: flag a molecule outside those bounds
-  if (xc_mol_outside(Mo, max_nao, da.nsh_max)) {
+  if (xc_mol_outside(Mo, max_nao, DIRECT ? da.nsh_max : 0)) {
     if (part == 0) {
       for (int x = threadIdx.x; x < N * N; x += blockDim.x) vxc[Mo.mat0 + x] = T(NAN);
       if (threadIdx.x == 0) exc[m] = NAN;
@@ -742,12 +779,17 @@ __global__ void __launch_bounds__(XC_THREADS) xc_batch_kernel(
       if (threadIdx.x == 0) part_e[slot] = e;
     }
   };
-  XcStageDirect<T, XT, NP> stage;
-  stage.sh = xc_build_shells<T>(smem + da.tab_off, da.nsh_max, da.kp, (int)Mo.bas0, (int)Mo.nbas, da.atm, da.bas,
-                                da.env);
-  stage.coords = da.coords + 3 * Mo.grid0;
-  stage.g = a.g;
-  run(stage);
+  if constexpr (DIRECT) {
+    XcStageDirect<T, XT, NP> stage;
+    stage.sh = xc_build_shells<T>(smem + da.tab_off, da.nsh_max, da.kp, (int)Mo.bas0, (int)Mo.nbas, da.atm, da.bas,
+                                  da.env);
+    stage.coords = da.coords + 3 * Mo.grid0;
+    stage.g = a.g;
+    run(stage);
+  } else {
+    XcStageStored<T, XT, NP> stage{ao + Mo.ao0, N * a.g, a.g, 1, a.g, N};
+    run(stage);
+  }
 }
 
 // xc_batch_kernel with wave-private tiles: the same chunks and outputs; a
@@ -1631,14 +1673,17 @@ extern "C" int pscf_batch_ao(int dtype, const void* d_mols, const int* d_ptmol, 
 // molecules, all active: 6.18 ms per XC pass with one each, 5.98 with four.
 constexpr int XW_PARTS = 4;
 
-// FP64 direct launches above nao 48 keep xc_batch_kernel: four AO components
-// of 64 points and a wave's FP64 D and V do not fit a CU and its registers.
+// FP64 batches keep xc_batch_kernel, although the wave tiles are faster (22
+// molecules of nao 63, one pass: 464 us instead of 655): they add a point's
+// products in another order, and a molecule that does not converge amplifies a
+// last bit by up to seven orders within 20 iterations, where FP64 is the form
+// that results are compared and reproduced with.
 template <typename T, int NP, bool DIRECT>
 static int batch_xc_launch(const void* d_mols, const int* d_order, int nmol, int max_nao, const double* d_ctl,
                            const void* d_ao, const XcDirect* da, const void* d_dm, const void* d_w, double eps,
                            void* d_vxc, double* d_exc, int split, void* d_part_v, double* d_part_e,
                            int64_t part_v_elems, int64_t part_e_elems, hipStream_t st) {
-  constexpr bool WAVE = !(DIRECT && sizeof(T) == 8 && NP > 48);
+  constexpr bool WAVE = sizeof(T) == 4;
   XcDirect a = DIRECT ? *da : XcDirect{};
   size_t lds;
   if constexpr (WAVE)
@@ -1661,7 +1706,7 @@ static int batch_xc_launch(const void* d_mols, const int* d_order, int nmol, int
   if constexpr (WAVE)
     rc = run(xc_wave_batch_kernel<T, NP, DIRECT>);
   else
-    rc = run(xc_batch_kernel<T, 32, NP>);
+    rc = run(xc_batch_kernel<T, 32, NP, DIRECT>);
   if (rc) return rc;
   const dim3 rgrid(nmol, WAVE ? (max_nao * (max_nao + 1) / 2 + 255) / 256 : 1);
   xc_batch_reduce_kernel<T, WAVE><<<rgrid, 256, WAVE ? 0 : sizeof(T) * (size_t)max_nao * max_nao, st>>>(

@@ -33,8 +33,8 @@ struct XW {
   static constexpr int XS = NP + (STORED && sizeof(T) == 8 ? 2 : 4), XD = NP <= 16 ? 16 : (NP == 48 ? 48 : 80);
   // HS = 2: two waves share 16 points, each with half of the columns of X, Y and
   // V, where all of them (FP64, nao 64: 128 registers of V, 128 of AO values) leave
-  // a wave nothing for the functional; 512 threads, two waves a SIMD (22 molecules
-  // of nao 63, one XC pass: 464 us, 655 with a wave per 16 points)
+  // a wave nothing for the functional; 512 threads, two waves a SIMD (the SCF of a
+  // molecule of nao 60: 4.39 ms, 4.50 with a wave per 16 points)
   static constexpr int HS = STORED && sizeof(T) == 8 && NP == 64 ? 2 : 1, THREADS = XC_THREADS * HS, NBH = NB / HS;
   static constexpr int PHI = (STORED ? HS : 4) * 16 * XS;  // HS = 2: phi0 of this tile and the last
   static constexpr bool DLDS = STORED && (sizeof(T) == 8 ? NP >= 48 : NP >= 64);
