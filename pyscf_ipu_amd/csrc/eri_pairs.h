@@ -27,6 +27,7 @@
 // rest staging, segmented sums and the ends of tiles.
 #pragma once
 #include "batch.h"
+#include "boys_fp64.h"
 #include "common.h"
 #include "wave.h"
 
@@ -67,14 +68,10 @@ constexpr int EP_CAP_BRA = 288;
 // ------------------------------------------------------------ Boys values ----
 // FP32: cubic Taylor about nodes 1/16 apart (error below 2e-8), one 16-byte
 // LDS read; FP64: 10 terms about nodes 0.2 apart, with exp(-T_i) beside them
-// (19 KB; nodes 0.1 apart with 8 terms take 32 KB and a workgroup per CU).
+// (19 KB; nodes 0.1 apart with 8 terms take 32 KB and a workgroup per CU), see
+// boys_fp64.h.
 constexpr int BOYSF_NT = 640, BOYSF_LMAX = 4;
-constexpr int BOYSD_NT = 200, BOYSD_TERMS = 10, BOYSD_COLS = BOYSD_TERMS + 2;
-constexpr double BOYSD_H = 0.2;
 __device__ float4 g_boysf[(BOYSF_LMAX + 1) * BOYSF_NT];
-
-__device__ constexpr double INV_FACT[11] = {1.0,       1.0,        1.0 / 2,     1.0 / 6,      1.0 / 24,     1.0 / 120,
-                                            1.0 / 720, 1.0 / 5040, 1.0 / 40320, 1.0 / 362880, 1.0 / 3628800};
 
 template <typename T>
 struct EpTable;
@@ -96,8 +93,6 @@ __device__ inline double rsq(double x) {  // hardware estimate and one third-ord
   return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
-constexpr double BOYS_EDGE = 39.9;  // the tables end here, the asymptote begins
-
 // F_0 .. F_L from the table; t is clamped to it.
 template <int L>
 __device__ __forceinline__ void ep_boys(float t, const float4* __restrict__ tab, float* f) {
@@ -110,25 +105,6 @@ __device__ __forceinline__ void ep_boys(float t, const float4* __restrict__ tab,
     const float e = __builtin_amdgcn_exp2f(-1.44269504f * t), t2 = t + t;
 #pragma unroll
     for (int m = L; m > 0; --m) f[m - 1] = (t2 * f[m] + e) * (1.0f / (2 * m - 1));
-  }
-}
-template <int L>
-__device__ __forceinline__ void ep_boys(double t, const double* __restrict__ tab, double* f) {
-  t = fmin(t, BOYS_EDGE);
-  const int i = (int)(t * (1.0 / BOYSD_H) + 0.5);
-  const double d = (double)i * BOYSD_H - t;
-  const double* c = tab + i * BOYSD_COLS;
-  double a = c[BOYSD_TERMS];
-#pragma unroll
-  for (int k = BOYSD_TERMS; k > 0; --k) a = fma(a, d, c[k - 1]);
-  f[L] = a;
-  if constexpr (L > 0) {
-    double e = INV_FACT[9];  // exp(d), |d| <= 0.1
-#pragma unroll
-    for (int k = 8; k >= 0; --k) e = fma(e, d, INV_FACT[k]);
-    e *= c[BOYSD_TERMS + 1];
-#pragma unroll
-    for (int m = L; m > 0; --m) f[m - 1] = fma(t + t, f[m], e) * (1.0 / (2 * m - 1));
   }
 }
 // F_0 = sqrt(pi / t) / 2 and upward recursion past the tables.
@@ -149,7 +125,7 @@ __device__ inline void ep_stage_table(double* tab, const double* __restrict__ g)
   for (int i = threadIdx.x; i < BOYSD_NT; i += EP_THREADS) {
     const double* s = g + 2 * i * BOYS_NM + L;  // every second node of the 0.1 grid
 #pragma unroll
-    for (int k = 0; k <= BOYSD_TERMS; ++k)  // (order 5: a term less, still below 1e-19)
+    for (int k = 0; k <= BOYSD_TERMS; ++k)  // (order 5: a term less, 9e-19 at most)
       tab[i * BOYSD_COLS + k] = L + k < BOYS_NM ? s[L + k < BOYS_NM ? k : 0] * INV_FACT[k] : 0.0;
     if constexpr (L > 0) tab[i * BOYSD_COLS + BOYSD_TERMS + 1] = exp(-(double)i * BOYSD_H);
   }
@@ -490,10 +466,10 @@ __device__ __forceinline__ void ep_prims(const EpPrim<T>* prim, const T (&AB)[3]
     tmax = u ? max(tmax, t[u]) : t[u];
     ep_boys<L>(t[u], tab, F[u]);
   }
-  if (__any(tmax > T(BOYS_EDGE))) {
+  if (__any(tmax >= T(BOYS_EDGE))) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (t[u] > T(BOYS_EDGE)) ep_boys_tail<L>(t[u], F[u]);
+      if (t[u] >= T(BOYS_EDGE)) ep_boys_tail<L>(t[u], F[u]);
   }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
