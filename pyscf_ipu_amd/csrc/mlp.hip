@@ -167,7 +167,8 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(int M, int N, int K, con
   const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
   const int steps = (K + TK - 1) / TK, per = (steps + gridDim.z - 1) / gridDim.z;
   const int s0 = blockIdx.z * per, s1 = min(steps, s0 + per);
-  if (s0 >= s1) return;
+  // nothing to add; the other epilogues store their result for K = 0 too
+  if (EPI == EPI_ATOMIC && s0 >= s1) return;
   float sum[FN];
 #pragma unroll
   for (int j = 0; j < FN; ++j) sum[j] = 0.f;
