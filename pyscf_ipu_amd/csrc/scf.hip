@@ -1830,7 +1830,7 @@ template <typename T>
 __global__ void __launch_bounds__(SCF_THREADS) scf_step_kernel(int it, int N, int nocc, const double* __restrict__ Hcore,
                                                                const double* __restrict__ S,
                                                                const double* __restrict__ Linv,
-                                                               const T* __restrict__ dJK, const T* __restrict__ Vxc,
+                                                               const T* __restrict__ dJK, const T* Vxc,
                                                                double* __restrict__ D, double* __restrict__ Hout,
                                                                double* __restrict__ mo_e, double* __restrict__ Cout,
                                                                double* __restrict__ state, int use_diis,
@@ -1839,7 +1839,8 @@ __global__ void __launch_bounds__(SCF_THREADS) scf_step_kernel(int it, int N, in
   const ScfLds L = scf_lds_carve(smem, N);
   scf_step_body<T, T>(L, it, N, nocc, Hcore, S, Linv, dJK, Vxc, D, (T*)nullptr, (T*)nullptr, Hout, mo_e, Cout, state,
                       use_diis);
-  // (Vxc was read before the step's first barriers)
+  // zero_v may be Vxc itself, which therefore promises nothing about aliases; it
+  // was read before the step's first barriers
   if (zero_v != nullptr) {
     __syncthreads();
     for (int x = threadIdx.x; x < N * N; x += SCF_THREADS) zero_v[x] = 0.0;
