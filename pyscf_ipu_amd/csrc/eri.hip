@@ -1066,8 +1066,17 @@ extern "C" int pscf_int1e(const int* d_atm, int natm, const int* d_bas, int nbas
   return PSCF_OK;
 }
 
-// Workgroups that share a molecule where a launch enumerates the molecules itself.
-static int mols_per(int nmol) { return (nmol >= 8192 ? 4 : (nmol <= 256 ? 128 : 32768 / nmol)) - 1; }
+// Workgroups that share a molecule where a launch enumerates the molecules
+// itself, about 32768 in all; odd for every number of molecules (eri_s8_mols_kernel).
+static constexpr int mols_per(int nmol) {
+  return ((nmol >= 8192 ? 4 : (nmol <= 256 ? 128 : 32768 / nmol)) - 1) | 1;
+}
+static constexpr bool mols_per_odd() {
+  for (int n = 1; n <= 10000; ++n)
+    if (mols_per(n) % 2 == 0) return false;
+  return true;
+}
+static_assert(mols_per_odd(), "workgroups per molecule: an odd number");
 
 // FP64 batch ERIs: work lists (h_work, lightest class first) or, if null, every molecule.
 template <int X, int Y>

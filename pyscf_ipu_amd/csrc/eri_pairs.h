@@ -775,7 +775,8 @@ __host__ __device__ inline int ep_count(int X, int ns, int np) {
 // All molecules of an FP32 batch, one class: `per` workgroups share a molecule's
 // tiles.  `per` is odd: neighbouring workgroups go to different XCDs, and with
 // an even count the parts of molecules with few tiles all fell on the same few
-// XCDs (1024 nine-heavy-atom molecules: 69 ms with 32, 51 ms with 31).  The
+// XCDs (1024 nine-heavy-atom molecules: 69 ms with 32, 51 ms with 31; 500: 33 ms
+// with 64, 25.5 with 65).  The
 // classes have a launch each: in one launch they would all take the registers
 // and LDS of the heaviest (74 ms).
 template <int C>
