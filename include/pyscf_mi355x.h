@@ -293,11 +293,12 @@ int pscf_batch_ao(int dtype, const void* d_mols, const int* d_ptmol, const doubl
  * shapes; a larger molecule gets NaN).  Each molecule's grid is cut into
  * chunks of PSCF_XC_CHUNK_PTS points whose V and E_xc partials are summed in
  * chunk order, so the result does not depend on `split` (workgroups sharing a
- * molecule's chunks; a launch may use more).  Chunk partials go to d_part_v (part_v_elems >=
+ * molecule's chunks; a launch takes pscf_batch_xc_split of them).  Chunk partials go to d_part_v (part_v_elems >=
  * nchunk_max * nmol * max_nao^2 elements of dtype) and d_part_e (part_e_elems
  * >= nchunk_max * nmol doubles), nchunk_max = ceil(largest grid /
  * PSCF_XC_CHUNK_PTS); a molecule whose chunks do not fit gets NaN. */
 #define PSCF_XC_CHUNK_PTS 512
+int pscf_batch_xc_split(int dtype, int split);
 int pscf_batch_xc(int dtype, const void* d_mols, const int* d_order, int nmol, int max_nao, const double* d_ctl,
                   const void* d_ao, const void* d_dm, const void* d_w, double eps, void* d_vxc, double* d_exc,
                   int split, int tile, void* d_part_v, double* d_part_e, int64_t part_v_elems, int64_t part_e_elems,
@@ -326,10 +327,12 @@ int pscf_batch_eri_scale(int dtype, const void* d_mols, int nmol, int max_nao, v
  * (sparse_symmetric_ERI.py:86-137); max_nao bounds their nao (it sizes the
  * LDS; a larger molecule gets NaN).  accumulate = 0: d_out (dtype) =
  * dJK(d_dm); accumulate = 1: d_out (FP64) += dJK(d_dm), the incremental build
- * from density changes.  split workgroups of `threads` (256 or 512) threads
- * share each molecule's ERI rows (atomic accumulation).  Each workgroup holds
+ * from density changes.  `split` workgroups of `threads` (256 or 512) threads,
+ * as many as pscf_batch_jk_split makes of it, share each molecule's ERI rows
+ * (atomic accumulation).  Each workgroup holds
  * dm (dtype) and an FP64 accumulator in LDS: max_nao^2 * (sizeof(dtype) + 8)
  * bytes, at most 160 KiB (max_nao <= 116 in FP32, 101 in FP64). */
+int pscf_batch_jk_split(int dtype, int nmol, int max_nao, int accumulate, int split, int threads);
 int pscf_batch_jk_s8(int dtype, const void* d_mols, const int* d_order, int nmol, int max_nao, const double* d_ctl,
                      const void* d_eri, const void* d_dm, double hyb, void* d_out, int accumulate, int split,
                      int threads, void* stream);

@@ -79,6 +79,8 @@ _SIGS = {
                                  c_void_p, c_void_p, c_void_p, c_void_p]),
     "pscf_batch_ao": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p,
                               c_void_p]),
+    "pscf_batch_xc_split": (c_int, [c_int, c_int]),
+    "pscf_batch_jk_split": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "pscf_batch_xc": (c_int, [c_int, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p,
                               c_double, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int64, c_int64,
                               c_void_p]),

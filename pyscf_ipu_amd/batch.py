@@ -368,14 +368,31 @@ class BatchRKS:
         dm = self.Dt if (first or not self.incremental) else self.dDt
         self._jk(ctl_ptr, self.split["jk"], self.jk_threads, dm)
 
+    def tune_candidates(self) -> dict:
+        """{"xc": [(tile, split)], "jk": [(threads, split)]}: one candidate for
+        each launch shape that the library makes of this batch (it raises a small
+        split and bounds a large one, so several may be one shape: the largest
+        of them is listed)."""
+        lib = _lib.lib()
+
+        def xc(c):
+            return c[0], *(lib.pscf_batch_xc_split(self.code, class_split(c[1], n)) for _, n, _ in self.nao_classes)
+
+        def jk(c):
+            return c[0], *(lib.pscf_batch_jk_split(self.code, n, cmax, int(self.dtype == "fp32"),
+                                                   class_split(c[1], n), c[0]) for _, n, cmax in self.nao_classes)
+
+        all_xc = [(t, k) for t in XC_TILES[self.dtype] for k in SPLITS[:3]]
+        all_jk = [(t, k) for t in JK_THREADS for k in SPLITS]
+        return {"xc": list({xc(c): c for c in all_xc}.values()), "jk": list({jk(c): c for c in all_jk}.values())}
+
     def tune(self, repeats: int = 2):
         """Autotuner: times the XC launch for every (tile, split) candidate and
-        the J/K launch for every (workgroup size, split) candidate on this
-        batch (all molecules active, current density, scratch outputs), keeps
-        the fastest, and caches the choice for batches of the same shape.
-        `self.tuning` records the timings (ms per launch) next to the fixed
-        tiling (32-point tiles, 256-thread J/K workgroups, one workgroup per
-        molecule)."""
+        the J/K launch for every (workgroup size, split) candidate of
+        tune_candidates on this batch (all molecules active, current density,
+        scratch outputs), keeps the fastest, and caches the choice for batches of
+        the same shape.  `self.tuning` records the timings (ms per launch) and,
+        as `fixed`, the smallest launch of each."""
         key = (self.dtype, self.M, self.max_nao, self.sizes["eri"], self.sizes["grid"], self.ao_direct)
         if key in _TUNE_CACHE:
             self.tuning = dict(_TUNE_CACHE[key], cached=True)
@@ -387,8 +404,7 @@ class BatchRKS:
         ctl = P(self.ctl)
         vxc, exc = torch.empty_like(self.Vxc), torch.empty_like(self.exc)
         out = torch.zeros_like(self.dJK)
-        cands = {"xc": [(t, k) for t in XC_TILES[self.dtype] for k in SPLITS[:3]],
-                 "jk": [(t, k) for t in JK_THREADS for k in SPLITS]}
+        cands = self.tune_candidates()
         fns = {"xc": lambda c: self._xc(ctl, c[1], c[0], vxc, exc),
                "jk": lambda c: self._jk(ctl, c[1], c[0], self.Dt, out)}
         names = {"xc": lambda c: f"tile{c[0]}/split{c[1]}", "jk": lambda c: f"threads{c[0]}/split{c[1]}"}
@@ -409,7 +425,7 @@ class BatchRKS:
         self.split = {"xc": best_xc[1], "jk": best_jk[1]}
         self.tuning = {"ms": res, "chosen_split": dict(self.split), "chosen_tile": self.xc_tile,
                        "chosen_jk_threads": self.jk_threads,
-                       "fixed": {"xc": "tile32/split1", "jk": "threads256/split1"}}
+                       "fixed": {n: names[n](cands[n][0]) for n in names}}
         _TUNE_CACHE[key] = dict(self.tuning)
         return self.tuning
 

@@ -1268,6 +1268,18 @@ static int batch_jk_launch(dim3 grid, int threads, size_t lds, hipStream_t st, c
   return PSCF_OK;
 }
 
+// With FP64 outputs the sums are exact for any split, so a launch takes at
+// least four workgroups per molecule (as molecules converge the others still
+// spread over the CUs) and about 2048 in all, up to one wave per row list of
+// jk_s8_cols_batch_kernel: 982 9-heavy molecules in FP32 4.75 -> 4.57 ms, 246
+// 2.43 -> 1.25 ms, 62 2.42 -> 0.37 ms a call against one workgroup each; 22
+// molecules in FP64 404 -> 341 us against 24 each.
+extern "C" int pscf_batch_jk_split(int dtype, int nmol, int max_nao, int accumulate, int split, int threads) {
+  const int cap = max_nao <= JKC_MAXN && threads >= 64 ? JKC_VWAVES / (threads / 64) : 64;
+  if ((dtype == PSCF_F64 || accumulate) && nmol > 0) split = std::max(split, std::max((2048 + nmol - 1) / nmol, 4));
+  return std::min(split, cap);
+}
+
 extern "C" int pscf_batch_jk_s8(int dtype, const void* d_mols, const int* d_order, int nmol, int max_nao,
                                 const double* d_ctl, const void* d_eri, const void* d_dm, double hyb, void* d_out,
                                 int accumulate, int split, int threads, void* stream) {
@@ -1279,17 +1291,7 @@ extern "C" int pscf_batch_jk_s8(int dtype, const void* d_mols, const int* d_orde
   const size_t lds = (size_t)max_nao * max_nao * ((dtype == PSCF_F64 ? 8 : 4) + sizeof(double));
   PSCF_REQUIRE((int)lds <= max_lds_bytes(), "pscf_batch_jk_s8: nao %d too large for LDS", max_nao);
   hipStream_t st = (hipStream_t)stream;
-  // With FP64 outputs the sums are exact for any split, so a launch takes at
-  // least four workgroups per molecule (as molecules converge the others still
-  // spread over the CUs) and about 2048 in all, up to one wave per row list of
-  // jk_s8_cols_batch_kernel: 982 9-heavy molecules in FP32 4.75 -> 4.57 ms, 246
-  // 2.43 -> 1.25 ms, 62 2.42 -> 0.37 ms a call against one workgroup each; 22
-  // molecules in FP64 404 -> 341 us against 24 each.
-  if (dtype == PSCF_F64 || accumulate) {
-    const int cap = max_nao <= JKC_MAXN ? JKC_VWAVES / (threads / 64) : 64;
-    const int want = std::min((2048 + nmol - 1) / nmol, cap);
-    split = std::max(split, std::max(want, 4));
-  }
+  split = pscf_batch_jk_split(dtype, nmol, max_nao, accumulate, split, threads);
   const dim3 grid(nmol, split);
   if (split > 1 && !accumulate) {
     if (dtype == PSCF_F64)

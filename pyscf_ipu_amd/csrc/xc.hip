@@ -1668,10 +1668,14 @@ extern "C" int pscf_batch_ao(int dtype, const void* d_mols, const int* d_ptmol, 
 
 // LDS of the batched kernel: the tile pipeline (or, after the tiles, V and
 // the energy partials), then in the direct form the shell table.
-// Workgroups per molecule at least: as molecules converge, the rest still
-// spread over the CUs (the sums do not depend on the split).  1024 9-heavy
-// molecules, all active: 6.18 ms per XC pass with one each, 5.98 with four.
+// Workgroups per molecule that a launch takes, in FP32 (wave tiles) at least
+// four: as molecules converge, the rest still spread over the CUs (the sums do
+// not depend on the split).  1024 9-heavy molecules, all active: 6.18 ms per XC
+// pass with one each, 5.98 with four.
 constexpr int XW_PARTS = 4;
+extern "C" int pscf_batch_xc_split(int dtype, int split) {
+  return dtype == PSCF_F32 && split < XW_PARTS ? XW_PARTS : split;
+}
 
 // FP64 batches keep xc_batch_kernel, although the wave tiles are faster (22
 // molecules of nao 63, one pass: 464 us instead of 655): they add a point's
@@ -1696,7 +1700,7 @@ static int batch_xc_launch(const void* d_mols, const int* d_order, int nmol, int
   constexpr int THREADS = WAVE ? XW<T, NP, !DIRECT>::THREADS : XC_THREADS;
   auto run = [&](auto kernel) -> int {
     PSCF_SET_LDS(kernel, lds);
-    kernel<<<dim3(nmol, WAVE && split < XW_PARTS ? XW_PARTS : split), THREADS, lds, st>>>(
+    kernel<<<dim3(nmol, pscf_batch_xc_split(WAVE ? PSCF_F32 : PSCF_F64, split)), THREADS, lds, st>>>(
         (const BatchMol*)d_mols, d_order, max_nao, d_ctl, (const T*)d_ao, a, (const T*)d_dm, (const T*)d_w, (T)eps,
         (T*)d_vxc, d_exc, (T*)d_part_v, d_part_e, part_v_elems, part_e_elems);
     PSCF_HIP(hipGetLastError());
