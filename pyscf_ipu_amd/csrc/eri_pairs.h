@@ -329,7 +329,7 @@ __device__ inline void ep_stage(const EpMol& M, int first, int s, int f, int e, 
         P[d] = ri[d] - w * x;
       }
       const double k = M.env[bi[6] + pi] * M.env[bj[6] + pj] * exp(-a * w * r2) * rp;
-      keep = fabs(k) >= EpCut<T>::v;
+      keep = !(fabs(k) < EpCut<T>::v);  // not-a-number stays
       r.p = (T)p;
       r.x = (T)P[0];
       r.y = (T)P[1];
