@@ -81,13 +81,24 @@ __device__ __forceinline__ float gemm_store(float v, int row, int col, int64_t o
 // the transposing writes fall on all banks.
 constexpr int tile_stride(int TK) { return TK == 32 ? 36 : TK + 16; }
 
-// Stages rows [r0, r0 + R) x k [k0, k0 + TK) of a [row][k] operand (T: stored [k][row]).
-template <int R, int TK, bool T>
+// Stages rows [r0, r0 + R) x k [k0, k0 + TK) of a [row][k] operand (T: stored
+// [k][row]).  TAIL: its stored rows are not whole 8-element pieces.
+template <int R, int TK, bool T, bool TAIL>
 struct TileLoad {
   static constexpr int KP = TK / 8, NT = (R * KP + 255) / 256;  // 16-byte pieces per row, per thread
   static constexpr int KQ = TK / 4, TASKS = KQ * R / 8;         // T: blocks of four k rows x eight rows
   static_assert(!T || TASKS <= 256, "one transposing block per thread");
   uint4 v[T ? 4 : NT];
+  // n elements from p, in one 16-byte load.  TAIL: n may be less than 8; what lies
+  // behind the elements is in the same row's padding or, in the last row, may be
+  // behind the allocation, so that its end is read element by element
+  __device__ static inline uint4 piece(const bf16_t* __restrict__ p, int n, bool last) {
+    if (!TAIL || n >= 8 || !last) return *reinterpret_cast<const uint4*>(p);
+    unsigned w[4] = {0, 0, 0, 0};
+#pragma unroll 1
+    for (int q = 0; q < n; ++q) w[q / 2] |= (unsigned)p[q] << (16 * (q % 2));
+    return uint4{w[0], w[1], w[2], w[3]};
+  }
   __device__ inline void load(const bf16_t* __restrict__ P, int ld, int r0, int rows, int k0, int kend) {
     const int tid = threadIdx.x;
     if constexpr (!T) {
@@ -96,8 +107,8 @@ struct TileLoad {
         const int e = tid + 256 * i, r = e / KP, k = k0 + (e % KP) * 8;
         uint4 x = {0, 0, 0, 0};
         if (r < R && r0 + r < rows && k < kend) {
-          x = *reinterpret_cast<const uint4*>(P + (int64_t)(r0 + r) * ld + k);
-          if (k + 8 > kend) {  // the tail of the last piece is not part of K
+          x = piece(P + (int64_t)(r0 + r) * ld + k, kend - k, r0 + r == rows - 1);
+          if (TAIL && k + 8 > kend) {  // the tail of the last piece is not part of K
             unsigned* w = reinterpret_cast<unsigned*>(&x);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -114,7 +125,7 @@ struct TileLoad {
       for (int q = 0; q < 4; ++q) {
         const int k = k0 + kq * 4 + q;
         v[q] = tid < TASKS && k < kend && r0 + r < rows
-                   ? *reinterpret_cast<const uint4*>(P + (int64_t)k * ld + r0 + r)
+                   ? piece(P + (int64_t)k * ld + r0 + r, rows - r0 - r, k == kend - 1)
                    : uint4{0, 0, 0, 0};
       }
     }
@@ -153,7 +164,7 @@ struct TileLoad {
 // (BN / (4 / WM)).  TA, TB as in gemm_bf16_kernel; blockIdx.z splits the K
 // steps (EPI_ATOMIC only).  A workgroup walks the row tiles blockIdx.y,
 // blockIdx.y + gridDim.y, ...
-template <int BM, int BN, int TK, int WM, bool TA, bool TB, int EPI>
+template <int BM, int BN, int TK, int WM, bool TA, bool TB, int EPI, bool TAIL>
 __global__ void __launch_bounds__(256) gemm_tile_kernel(int M, int N, int K, const bf16_t* __restrict__ A, int lda,
                                                         const bf16_t* __restrict__ B, int ldb,
                                                         const float* __restrict__ bias, const float* __restrict__ aux,
@@ -178,8 +189,8 @@ __global__ void __launch_bounds__(256) gemm_tile_kernel(int M, int N, int K, con
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int j = 0; j < FN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    TileLoad<BM, TK, TA> la;
-    TileLoad<BN, TK, !TB> lb;
+    TileLoad<BM, TK, TA, TAIL> la;
+    TileLoad<BN, TK, !TB, TAIL> lb;
     la.load(A, lda, m0, M, s0 * TK, K);
     lb.load(B, ldb, n0, N, s0 * TK, K);
     for (int s = s0; s < s1; ++s) {
@@ -462,12 +473,18 @@ template <int BM, int BN, int TK, int WM, bool TA, bool TB, int EPI>
 static void launch_tile(int M, int N, int K, const void* A, int lda, const void* B, int ldb, const float* bias,
                         const float* aux, float* out, void* out2, int ldc, int rows, int ksplit, hipStream_t st) {
   dim3 grid((N + BN - 1) / BN, rows, ksplit);
-  gemm_tile_kernel<BM, BN, TK, WM, TA, TB, EPI><<<grid, 256, 0, st>>>(M, N, K, (const bf16_t*)A, lda, (const bf16_t*)B,
-                                                                      ldb, bias, aux, out, (bf16_t*)out2, ldc);
+  auto run = [&](auto kernel) {
+    kernel<<<grid, 256, 0, st>>>(M, N, K, (const bf16_t*)A, lda, (const bf16_t*)B, ldb, bias, aux, out, (bf16_t*)out2,
+                                 ldc);
+  };
+  if ((TA ? M : K) % 8 || (TB ? K : N) % 8)
+    run(gemm_tile_kernel<BM, BN, TK, WM, TA, TB, EPI, true>);
+  else
+    run(gemm_tile_kernel<BM, BN, TK, WM, TA, TB, EPI, false>);
 }
 
-// Tiled form where every row starts 16-byte aligned and the rows reach to a
-// multiple of 8 elements (the pieces it loads): 64 x 64 tiles, 64 x 32 for the
+// Tiled form where every row starts 16-byte aligned and the rows are a multiple
+// of 8 elements apart (the pieces it loads): 64 x 64 tiles, 64 x 32 for the
 // narrow layer.
 template <bool TA, bool TB, int EPI>
 static int launch_gemm(int M, int N, int K, const void* A, int lda, const void* B, int ldb, const float* bias,
