@@ -433,7 +433,7 @@ int pscf_pair_assemble(int64_t P, const int* d_pinfo, const unsigned char* d_val
  *   op 2: out = (A B^T) * silu'(aux) (FP32 and BF16 out2)         [backward data]
  *   op 3: out += A^T B (FP32 atomics; up to ksplit slices of K)   [weight gradient]
  *   op 4: out2 = (A B^T) * silu'(aux) (BF16), out[n] += its column sums (FP32
- *         atomics; rows of A and B start 16-byte aligned)         [backward data and bias] */
+ *         atomics; rows of A and B start 16-byte aligned)         [backward data and bias, in no fixed order] */
 int pscf_mlp_gemm(int op, int M, int N, int K, const void* d_A, int lda, const void* d_B, int ldb,
                   const float* d_bias, const float* d_aux, float* d_out, void* d_out2, int ldc, int ksplit,
                   void* stream);
@@ -441,12 +441,10 @@ int pscf_mlp_gemm(int op, int M, int N, int K, const void* d_A, int lda, const v
  * inv_n (FP32 and BF16); the loss sum is added to *d_loss. */
 int pscf_mlp_mse_grad(int B, const float* d_pred, const float* d_Y, const float* d_mask, float inv_n, float* d_g32,
                       void* d_g16, double* d_loss, void* stream);
-/* pscf_mlp_mse_grad, and the column sums of g (the output layer's bias
- * gradient) added to d_db[32] (optional). */
-int pscf_mlp_mse_grad_bias(int B, const float* d_pred, const float* d_Y, const float* d_mask, float inv_n,
-                           float* d_g32, void* d_g16, double* d_loss, float* d_db, void* stream);
-/* Bias gradient: d_db[n] = sum_m dZ[m][n]. */
+/* Bias gradient: d_db[n] = sum_m dZ[m][n], summed in a fixed order. */
 int pscf_mlp_colsum(int M, int N, const float* d_dz, int ld, float* d_db, void* stream);
+/* The same bits, faster for many rows, with a workspace of 256 N floats. */
+int pscf_mlp_colsum_ws(int M, int N, const float* d_dz, int ld, float* d_db, float* d_ws, void* stream);
 /* Adam (bias-corrected, step >= 1) on FP32 master weights; refreshes the BF16
  * copy d_w16 when given. */
 int pscf_mlp_adam(int64_t n, float* d_w, void* d_w16, const float* d_g, float* d_m, float* d_v, float lr, float b1,

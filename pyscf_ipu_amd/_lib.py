@@ -122,9 +122,8 @@ _SIGS = {
                               c_void_p, c_void_p, c_int, c_int, c_void_p]),
     "pscf_mlp_mse_grad": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p,
                                   c_void_p]),
-    "pscf_mlp_mse_grad_bias": (c_int, [c_int, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p,
-                                       c_void_p, c_void_p]),
     "pscf_mlp_colsum": (c_int, [c_int, c_int, c_void_p, c_int, c_void_p, c_void_p]),
+    "pscf_mlp_colsum_ws": (c_int, [c_int, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p]),
     "pscf_mlp_adam": (c_int, [c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_float, c_float,
                               c_float, c_int, c_void_p]),
     "pscf_mlp_to_bf16": (c_int, [c_int64, c_void_p, c_void_p, c_void_p]),

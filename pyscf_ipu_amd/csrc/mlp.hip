@@ -316,58 +316,65 @@ __global__ void __launch_bounds__(256) gemm_bf16_kernel(int M, int N, int K, con
 // g = 2 (pred - Y) mask / nvalid on the padded output (ld = 32); BF16 and
 // FP32 copies of g; loss accumulated into *loss (FP64).  At most 512
 // workgroups: the loss is one address, and with an atomic per 256 elements
-// that was the time (27 -> 9 us for 16384 rows).  A thread keeps its column, so
-// db (optional) gets the column sums of g, the output layer's bias gradient.
+// that was the time (27 -> 9 us for 16384 rows).
 __global__ void __launch_bounds__(256) mse_grad_kernel(int64_t n, const float* __restrict__ pred,
                                                        const float* __restrict__ Y, const float* __restrict__ mask,
                                                        float inv_n, float* __restrict__ g32, bf16_t* __restrict__ g16,
-                                                       double* __restrict__ loss, float* __restrict__ db) {
+                                                       double* __restrict__ loss) {
   __shared__ double red[4];
-  __shared__ float cred[8][32];
   double l = 0.0;
-  float cs = 0.f;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const float d = (pred[i] - Y[i]) * mask[i];
     l += (double)d * d * inv_n;
     const float g = 2.0f * d * inv_n;
     g32[i] = g;
     g16[i] = f2bf(g);
-    cs += g;
   }
   l = wave_sum_last(l);
   if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = l;
-  cred[threadIdx.x >> 5][threadIdx.x & 31] = cs;
   __syncthreads();
   if (threadIdx.x == 0) atomicAdd(loss, red[0] + red[1] + red[2] + red[3]);
-  if (db && threadIdx.x < 32) {
-    float t = 0.f;
-    for (int k = 0; k < 8; ++k) t += cred[k][threadIdx.x];
-    atomicAdd(db + threadIdx.x, t);
-  }
 }
 
-// db[n] = sum_m dZ[m][n], db zeroed first: workgroups of 256 rows x 32 columns
-// (rows in 128-byte pieces) add their sums.
-constexpr int CS_ROWS = 256;
-__global__ void colsum_zero_kernel(int N, float* __restrict__ db) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n < N) db[n] = 0.f;
-}
-__global__ void __launch_bounds__(256) colsum_kernel(int M, int N, const float* __restrict__ dz, int ld,
-                                                     float* __restrict__ db) {
-  __shared__ float red[8][32];
-  const int c = threadIdx.x & 31, r = threadIdx.x >> 5, n = blockIdx.x * 32 + c;
-  const int m1 = min(M, (int)(blockIdx.y + 1) * CS_ROWS);
+// db[n] = sum_m dZ[m][n] in a fixed order, so that a bias gradient repeats bit
+// for bit (Adam divides small gradients by themselves: a last bit here moves the
+// next step's loss by up to 1e-8): CS_ROWS chains over every CS_ROWS-th row, then
+// a tree.  The chains of 32 columns x 8 rows a workgroup, whole cache lines, all
+// CUs; the tree is colsum_kernel over their results.  Memory-bound: 16384 x 256
+// in 9 us with the tree (the matrix at HBM rate: 4), 27 with colsum_kernel
+// alone, whose few workgroups take 16-byte pieces, 32 with a workgroup per column.
+constexpr int CS_ROWS = 256, CS_COLS = 4;
+
+template <int AHEAD>
+__device__ __forceinline__ float colsum_chain(int M, const float* __restrict__ dz, int ld, int t, int n) {
   float s = 0.f;
-  if (n < N)
-    for (int m = blockIdx.y * CS_ROWS + r; m < m1; m += 8) s += dz[(int64_t)m * ld + n];
-  red[r][c] = s;
-  __syncthreads();
-  if (threadIdx.x < 32 && n < N) {
-    float t = 0.f;
-    for (int k = 0; k < 8; ++k) t += red[k][c];
-    atomicAdd(db + n, t);
+  for (int64_t m = t; m < M; m += CS_ROWS * AHEAD) {
+    float v[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) v[u] = m + u * CS_ROWS < M ? dz[(m + u * CS_ROWS) * ld + n] : 0.f;
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) s += v[u];
   }
+  return s;
+}
+
+__global__ void __launch_bounds__(256) colsum_chain_kernel(int M, int N, const float* __restrict__ dz, int ld,
+                                                           float* __restrict__ part) {
+  const int n = blockIdx.x * 32 + threadIdx.x % 32, t = blockIdx.y * 8 + threadIdx.x / 32;
+  if (n < N) part[t * N + n] = colsum_chain<32>(M, dz, ld, t, n);
+}
+
+__global__ void __launch_bounds__(CS_COLS * CS_ROWS) colsum_kernel(int M, int N, const float* __restrict__ dz, int ld,
+                                                                   float* __restrict__ db) {
+  __shared__ float red[CS_ROWS][CS_COLS];
+  const int c = threadIdx.x % CS_COLS, t = threadIdx.x / CS_COLS, n = blockIdx.x * CS_COLS + c;
+  red[t][c] = n < N ? colsum_chain<8>(M, dz, ld, t, n) : 0.f;
+  for (int off = 32; off > 0; off >>= 1) {
+    __syncthreads();
+    if (t % 64 < off) red[t][c] += red[t + off][c];
+  }
+  __syncthreads();
+  if (t == 0 && n < N) db[n] = red[0][c] + red[64][c] + red[128][c] + red[192][c];
 }
 
 // Adam on FP32 master weights; BF16 working copy refreshed.
@@ -563,30 +570,36 @@ extern "C" int pscf_mlp_gemm(int op, int M, int N, int K, const void* d_A, int l
   return PSCF_EINVAL;
 }
 
-extern "C" int pscf_mlp_mse_grad_bias(int B, const float* d_pred, const float* d_Y, const float* d_mask, float inv_n,
-                                      float* d_g32, void* d_g16, double* d_loss, float* d_db, void* stream) {
+extern "C" int pscf_mlp_mse_grad(int B, const float* d_pred, const float* d_Y, const float* d_mask, float inv_n,
+                                 float* d_g32, void* d_g16, double* d_loss, void* stream) {
   PSCF_REQUIRE(B >= 0 && d_pred && d_Y && d_mask && d_g32 && d_g16 && d_loss, "pscf_mlp_mse_grad: bad arguments");
   if (B == 0) return PSCF_OK;
   const int64_t n = (int64_t)B * 32, blocks = (n + 255) / 256;
   mse_grad_kernel<<<(unsigned)(blocks < 512 ? blocks : 512), 256, 0, (hipStream_t)stream>>>(
-      n, d_pred, d_Y, d_mask, inv_n, d_g32, (bf16_t*)d_g16, d_loss, d_db);
+      n, d_pred, d_Y, d_mask, inv_n, d_g32, (bf16_t*)d_g16, d_loss);
   PSCF_HIP(hipGetLastError());
   return PSCF_OK;
 }
 
-extern "C" int pscf_mlp_mse_grad(int B, const float* d_pred, const float* d_Y, const float* d_mask, float inv_n,
-                                 float* d_g32, void* d_g16, double* d_loss, void* stream) {
-  return pscf_mlp_mse_grad_bias(B, d_pred, d_Y, d_mask, inv_n, d_g32, d_g16, d_loss, nullptr, stream);
+static int colsum(int M, int N, const float* dz, int ld, float* db, float* ws, hipStream_t st) {
+  if (ws) {
+    colsum_chain_kernel<<<dim3((N + 31) / 32, CS_ROWS / 8), 256, 0, st>>>(M, N, dz, ld, ws);
+    PSCF_HIP(hipGetLastError());
+  }
+  colsum_kernel<<<(N + CS_COLS - 1) / CS_COLS, CS_COLS * CS_ROWS, 0, st>>>(ws ? CS_ROWS : M, N, ws ? ws : dz,
+                                                                          ws ? N : ld, db);
+  PSCF_HIP(hipGetLastError());
+  return PSCF_OK;
 }
 
 extern "C" int pscf_mlp_colsum(int M, int N, const float* d_dz, int ld, float* d_db, void* stream) {
   PSCF_REQUIRE(M >= 0 && N > 0 && d_dz && d_db, "pscf_mlp_colsum: bad arguments");
-  colsum_zero_kernel<<<(N + 255) / 256, 256, 0, (hipStream_t)stream>>>(N, d_db);
-  if (M > 0)
-    colsum_kernel<<<dim3((N + 31) / 32, (M + CS_ROWS - 1) / CS_ROWS), 256, 0, (hipStream_t)stream>>>(M, N, d_dz, ld,
-                                                                                                      d_db);
-  PSCF_HIP(hipGetLastError());
-  return PSCF_OK;
+  return colsum(M, N, d_dz, ld, d_db, nullptr, (hipStream_t)stream);
+}
+
+extern "C" int pscf_mlp_colsum_ws(int M, int N, const float* d_dz, int ld, float* d_db, float* d_ws, void* stream) {
+  PSCF_REQUIRE(M >= 0 && N > 0 && N <= 1 << 20 && d_dz && d_db && d_ws, "pscf_mlp_colsum_ws: bad arguments");
+  return colsum(M, N, d_dz, ld, d_db, d_ws, (hipStream_t)stream);
 }
 
 extern "C" int pscf_mlp_adam(int64_t n, float* d_w, void* d_w16, const float* d_g, float* d_m, float* d_v, float lr,

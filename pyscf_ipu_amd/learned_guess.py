@@ -148,6 +148,8 @@ class PairMLP:
             self.out = device.empty((B, NOUT_PAD), f32)
             self.g32 = device.empty((B, NOUT_PAD), f32)
             self.g16 = device.empty((B, NOUT_PAD), BF16)
+            self.dZ = device.empty((B, NHID), f32)
+            self.colsum_ws = device.empty((256, NHID), f32)
             self.dZ16 = [device.empty((B, NHID), BF16) for _ in range(2)]
             self.loss = device.zeros(1, torch.float64)
 
@@ -178,18 +180,19 @@ class PairMLP:
         self.loss.zero_()
         ksplit = max(1, min(64, B // 512))
         G = lambda *a: _lib.call("pscf_mlp_gemm", *a)
-        _lib.call("pscf_mlp_mse_grad_bias", B, P(self.out), ctypes_ptr(Y, row0 * NOUT_PAD),
-                  ctypes_ptr(mask, row0 * NOUT_PAD), 1.0 / max(nvalid, 1.0), P(self.g32), P(self.g16), P(self.loss),
-                  self._p("b3", self.g), st)
+        _lib.call("pscf_mlp_mse_grad", B, P(self.out), ctypes_ptr(Y, row0 * NOUT_PAD), ctypes_ptr(mask, row0 * NOUT_PAD),
+                  1.0 / max(nvalid, 1.0), P(self.g32), P(self.g16), P(self.loss), st)
         # output layer
         G(3, NHID, NOUT_PAD, B, P(self.H[2]), NHID, P(self.g16), NOUT_PAD, None, None, self._p("W3", self.g), None,
           NOUT_PAD, ksplit, st)
+        _lib.call("pscf_mlp_colsum_ws", B, NOUT_PAD, P(self.g32), NOUT_PAD, self._p("b3", self.g), P(self.colsum_ws), st)
         up16, up_ld, Wname = self.g16, NOUT_PAD, "W3"
         for i in (2, 1, 0):
             dz16 = self.dZ16[i % 2]
-            # dZ_i = (dZ_{i+1} W_{i+1}^T) * silu'(Z_i), its column sums into the bias gradient
-            G(4, B, NHID, up_ld, P(up16), up_ld, self._p(Wname, self.w16), up_ld, None, P(self.Z[i]),
-              self._p(f"b{i}", self.g), P(dz16), NHID, 1, st)
+            # dZ_i = (dZ_{i+1} W_{i+1}^T) * silu'(Z_i)
+            G(2, B, NHID, up_ld, P(up16), up_ld, self._p(Wname, self.w16), up_ld, None, P(self.Z[i]), P(self.dZ),
+              P(dz16), NHID, 1, st)
+            _lib.call("pscf_mlp_colsum_ws", B, NHID, P(self.dZ), NHID, self._p(f"b{i}", self.g), P(self.colsum_ws), st)
             if i > 0:
                 G(3, NHID, NHID, B, P(self.H[i - 1]), NHID, P(dz16), NHID, None, None, self._p(f"W{i}", self.g), None,
                   NHID, ksplit, st)
