@@ -270,7 +270,7 @@ def _batched(mol_strs, workload: str, steps: int, warmup: int, its: int, golden=
     if "eri_s8" in sm:
         fl = roofline.batch_eri_flops(sizes_b)
         rl["eri_s8"] = _roof("valu", fl / (sm["eri_s8"] * 1e-3) / 1e12, PEAK_TFLOPS["fp32"], "TFLOP/s", sm["eri_s8"],
-                             "Rys op-count model (pyscf_ipu_amd/roofline.py); peak = FP32 vector rate")
+                             "Hermite op-count model (pyscf_ipu_amd/roofline.py); peak = FP32 vector rate")
     out["minao"]["kernel_rooflines"] = rl
     out["minao"]["setup_ms"] = {k: round(v, 2) for k, v in sm.items()}
     common = {"mean_scf_iters_fp64_minao": float(its64.mean()),
