@@ -217,11 +217,6 @@ class BatchRKS:
         # work list of the grid expansion (per atom): chunk counts here, the
         # (owner, first) list built on the device at set-up (pscf_batch_chunks)
         self.grid_counts = apts
-        # shell quartets per molecule of each ERI class
-        self.eri_counts = []
-        for X, Y in CLASSES:
-            nx, ny = class_pairs(X, ns, npp), class_pairs(Y, ns, npp)
-            self.eri_counts.append(nx * (nx + 1) // 2 if X == Y else nx * ny)
         self.order = np.argsort(-nao, kind="stable").astype(np.int32)
         self.max_nao = int(nao.max())
         # XC and J/K launches per class of nao rounded up to 16 (LDS sized per
@@ -232,6 +227,17 @@ class BatchRKS:
             pos = np.where(npad == v)[0]
             self.nao_classes.append((int(pos[0]), len(pos), int(nao[self.order[pos[0]]])))
 
+
+    @property
+    def eri_counts(self) -> list:
+        """Shell quartets per molecule of each ERI class (CLASSES), what the work
+        lists of pscf_batch_eri_s8 cover."""
+        ns, npp = self.desc[:, 6], self.desc[:, 7]
+        out = []
+        for X, Y in CLASSES:
+            nx, ny = class_pairs(X, ns, npp), class_pairs(Y, ns, npp)
+            out.append(nx * (nx + 1) // 2 if X == Y else nx * ny)
+        return out
 
     # ------------------------------------------------------------ device set-up ---
     @staticmethod
