@@ -134,9 +134,11 @@ class LargeRKS(RKS):
                   P(self.X), G, 1, st)
         _lib.call("pscf_xc_large_stage", 2, self.gemm_type, N, G, P(self.X), P(self.phi), P(self.weights64),
                   EPSILON_B3LYP, P(self.coef), P(self.e_part), P(self.Y), st)
-        # Vh[mu][nu] = sum_p phi0[mu][p] Y[nu][p], K = G split over workgroups
+        # Vh[mu][nu] = sum_p phi0[mu][p] Y[nu][p], K = G split over workgroups.  FP32
+        # accumulation keeps ranges of 2048 points: their length sets its rounding,
+        # and with it the iteration at which such an SCF meets its stop
         self.Vh.zero_()
-        ksplit = max(1, min(256, G // 512))
+        ksplit = max(1, min(256, G // (512 if self.acc64 else 2048)))
         _lib.call("pscf_gemm", self.gemm_type, self.acc64, 0, 1, 1, N, N, G, P(self.phi), G, P(self.Y), G,
                   P(self.Vh), N, ksplit, st)
         _lib.call("pscf_xc_large_finish", N, P(self.Vh), P(self.e_part), self.nparts, P(self.Vxc), P(self.exc), st)
