@@ -440,7 +440,7 @@ def main(argv=None):
     else:
         achieved = work["flops"] / mean_s / 1e12
         peak, unit = PEAK_TFLOPS[a.dtype], "TFLOP/s"
-    kname = {"scf_step": "scf_step_kernel", "jk_s8": "jk_s8_kernel", "xc": "xc_fused_kernel"}.get(dominant)
+    kname = {"scf_step": "scf_step_kernel", "jk_s8": "jk_s8_kernel", "xc": "xc_wave_kernel"}.get(dominant)
     tdt = "double" if a.dtype == "fp64" else "float"
     traffic = _profile_traffic(f"{kname}<{tdt}>") if kname else None
     roof = {"kernel": dominant, "bound": work["bound"], "achieved": achieved, "peak": peak, "unit": unit,

@@ -249,9 +249,10 @@ int pscf_batch_eri_s8(int dtype, const void* d_mols, int nmol, const int* const*
 int pscf_batch_eri_s8_div(int dtype, const void* d_mols, int nmol, const int* const* h_work, const int* h_nwork,
                           const int* d_atm, const int* d_bas, const double* d_env, const int* d_shell_ao,
                           const int* d_shl_sorted, void* d_out, void* stream);
-/* The same ERIs of every molecule (div as in pscf_batch_eri_s8_div) without
- * work lists: each angular class enumerates the molecules' own shell-pair
- * tiles.  d_order (optional) lists the molecules largest first. */
+/* The same ERIs of every molecule (div as in pscf_batch_eri_s8_div), bit for bit,
+ * without work lists, the form that BatchRKS calls: each angular class
+ * enumerates the molecules' own quartets.  d_order (optional) lists the molecules
+ * largest first. */
 int pscf_batch_eri_s8_all(int dtype, const void* d_mols, const int* d_order, int nmol, const int* d_atm,
                           const int* d_bas, const double* d_env, const int* d_shell_ao, const int* d_shl_sorted,
                           void* d_out, int div, void* stream);

@@ -58,9 +58,9 @@ def class_split(split: int, count: int) -> int:
     """Workgroups per molecule of an XC or J/K launch over `count` molecules."""
     return min(64, max(split, -(-MIN_WORKGROUPS // count)))
 JK_THREADS = (256, 512)   # J/K workgroup sizes tried by the autotuner
-# grid points per XC tile, as the entry points take it (the kernels' tiles have
-# one shape).  The autotuner varies only launch shapes that leave the result's
-# bits unchanged (XC split, J/K workgroup size and split).
+# grid points per XC tile, as the entry points take it (it chooses nothing: a
+# type's kernel has tiles of one shape).  The autotuner varies only launch shapes
+# that leave the result's bits unchanged (XC split, J/K workgroup size and split).
 XC_TILES = {"fp32": (32,), "fp64": (32,)}
 XC_CHUNK_PTS = 512  # points per chunk of pscf_batch_xc (PSCF_XC_CHUNK_PTS)
 _TUNE_CACHE = {}        # tuning results per batch shape

@@ -71,14 +71,13 @@ __device__ __forceinline__ float gemm_store(float v, int row, int col, int64_t o
 // The same product for operands with 16-byte aligned rows (every layer of the
 // network): 16-byte global loads one K step ahead of the MFMAs, both operands
 // staged as [row][k] (a k-major operand is transposed on the way, four k rows
-// at a time), fragments read as one ds_read_b64.  Row stride 36 elements: the
-// fragment reads and the transposing writes fall on all banks.  Each output
-// accumulates k in steps of 16 in order, as in gemm_bf16_kernel: same bits.
+// at a time), fragments read as one ds_read_b64.  Each output accumulates k in
+// steps of 16 in order, as in gemm_bf16_kernel: same bits.
 // 16384 rows: a hidden layer 28 -> 17 us (its 34 MB take 7 at HBM rate; 128 x
-// 128 tiles, one workgroup per CU: 25), backward data with its column sums 68
-// -> 18 us, a weight gradient 64 -> 16 us; a training step 653 -> 182 us.
-// Row stride of the staged operands: the fragment reads (16 rows, 8 bytes) and
-// the transposing writes fall on all banks.
+// 128 tiles, one workgroup per CU: 25), backward data 38 -> 17 us, a weight
+// gradient 64 -> 19 us; a training step 658 -> 217 us.
+// Row stride of the staged operands, 36 elements for 32 of k and 144 for 128: the
+// fragment reads (16 rows, 8 bytes) and the transposing writes fall on all banks.
 constexpr int tile_stride(int TK) { return TK == 32 ? 36 : TK + 16; }
 
 // Stages rows [r0, r0 + R) x k [k0, k0 + TK) of a [row][k] operand (T: stored

@@ -792,8 +792,8 @@ __global__ void __launch_bounds__(XC_THREADS) xc_batch_kernel(
   }
 }
 
-// xc_batch_kernel with wave-private tiles: the same chunks and outputs; a
-// chunk's slot holds the lower triangle of its V + V^T, packed.
+// xc_batch_kernel with wave-private tiles, for FP32 batches: the same chunks and
+// outputs; a chunk's slot holds the lower triangle of its V + V^T, packed.
 template <typename T, int NP, bool DIRECT>
 __global__ void __launch_bounds__((XW<T, NP, !DIRECT>::THREADS), (xw_min_blocks<T, NP>())) xc_wave_batch_kernel(
     const BatchMol* __restrict__ mols, const int* __restrict__ order, int max_nao, const double* __restrict__ ctl,

@@ -12,8 +12,8 @@ The integer work list of `prepare_integrals_2_inputs` is reproduced exactly,
 including the reference's shell-quartet filter i>=j, k>=l, i*j>=k*l (:772),
 its grouping by block size with `np.argsort` (:914-933) and the per-class
 scratch sizes of `get_shapes` (:813-911); the Python quadruple loop is
-vectorised.  The integrals themselves run in the library's Rys kernel
-(`pscf_eri_quartets` / `pscf_eri_s8`).
+vectorised.  The integrals themselves run in the library's kernels
+(`pscf_eri_quartets`: Rys quadrature; `pscf_eri_s8`: shell-pair lists).
 """
 from __future__ import annotations
 
